@@ -2,18 +2,20 @@
 // (normalised weighted average over in-bounds neighbours), exact transpose, and
 // the SIMP adjoint fused with the transpose.
 //
-// Forward and transpose are LDS-halo stencils.  A workgroup owns a tile of
-// TY x TZ element columns (3-D TY x 64 with TY 4 or 8, a wavefront per row along the
-// fastest axis; 2-D 1 x 256) and marches along x through a chunk of planes (4 to 32, as
-// many as keep about two workgroups per compute unit busy).  Each step stages one
-// new element plane of the tile plus its y/z halo into a ring of 8 plane slots
-// in LDS (zero outside the grid) and produces one output plane from the ring,
-// so every input value is read from memory once per tile (plus the halo rows)
-// and every output is written once, with no atomics.  Sums follow the offset
-// table's order, so results are deterministic; the forward pass is bitwise the
-// reference's (out-of-grid taps add an exact 0.0).  The forward's denominator
-// depends only on the output's distances to the six faces clipped to the radius,
-// so each workgroup tabulates it once per boundary class (at most 3^6 classes).
+// 3-D: a workgroup owns a tile of TY x 64 element columns (TY 8 or 4, a wavefront per row along
+// z) and marches along x through a chunk of planes (4 to 32, as many as keep about two
+// workgroups per compute unit busy).  Each step stages one element plane of the tile with its
+// y/z halo into one of two LDS planes and adds it to the 2R + 1 outputs of its column that it
+// reaches, which wait in registers: an LDS value is read once per thread and not once per tap.
+// At 256 x 128 x 128, radius 1, that took the forward from 51 to 25 us (67 MB, 2.7 TB/s) and the
+// transpose from 51 to 27 us (100 MB, 3.7 TB/s) against one LDS read per tap and weight; what is
+// left is load and barrier latency at 4 wavefronts per SIMD (128 VGPRs at radius 2).
+// 2-D: one workgroup stages one 4 x 64 tile with its halo and sums it; a small grid is bound by
+// launch and load latency (120 x 40: 9 us with the plane march, 4.4 us with one tile).
+// Every output is written once, with no atomics, and sums follow the offset table's order, so
+// results are deterministic; the forward pass is bitwise the reference's (out-of-grid taps add
+// an exact 0.0).  The forward's denominator depends only on the output's distances to the six
+// faces clipped to the radius, so each 3-D workgroup tabulates it once per boundary class.
 //
 //   forward    y_i = (sum_k w_k x_{i+o_k}) / (sum_k [i+o_k in grid] w_k)
 //              (apply_filter_{2D,3D}_kernel, core/_templated_cuda.cu:1526-1583)
@@ -31,10 +33,11 @@
 // host picks that form only for element matrices with the brick's reflection
 // structure (k0_structure); any other K0 takes the full product.
 //
-// 2-D grids run as 3-D grids of one element in y (element i * nely + j sits at
-// x = i, z = j).  Each workgroup reads the offset radii from the table; taps
-// wider than the ring (kMaxR per axis) are gathered from memory directly (the
-// adjoint then recomputes the neighbour's sensitivity per tap).
+// The march needs a radius of at most kMaxR per axis and a table in ascending (dx, dy, dz) order
+// with weights even in each of them (every table the meshes build up to rmin 3); the 2-D tile a
+// radius of at most kR2.  Each workgroup checks that on the device, where the table is; any
+// other table is gathered from memory tap by tap (the adjoint then recomputes the neighbour's
+// sensitivity per tap).
 #include "common.hpp"
 #include "op_tiled.hpp"
 #include "stiffness.hpp"
@@ -42,8 +45,8 @@
 namespace et {
 
 constexpr int kMaxOff = 1024;
-constexpr int kMaxR = 2;     // halo radius per axis held in the stencil kernels' ring (rmin <= 3)
-constexpr int kMaxTaps = 512;  // taps held in LDS by the stencil kernels (rmin up to about 4.9)
+constexpr int kMaxR = 2;     // halo radius per axis of the 3-D march (rmin <= 3)
+constexpr int kMaxTaps = 512;  // taps held in LDS (rmin up to about 4.9)
 constexpr int kMaxCX = 32;   // x planes per workgroup, at most
 
 template <int DIM>
@@ -256,297 +259,496 @@ __device__ __forceinline__ double stencil_value(const Grid& g, const SGrid& sg, 
   return simp_factor<(EN & 4) != 0>(xe, adj.penal) * en / adj.norm[e];
 }
 
-// Tap sum over the full (2R+1)^DIM cube around the output, in the offset table's
-// (dx, dy, dz) ascending order, with the weight of each cube position (0 where the
-// table has no tap, and such positions are skipped): the loop is unrolled, every
-// LDS address is an immediate offset from one base per x plane.
-template <int R, int DIM, int PZ, int PL, int RING>
-__device__ __forceinline__ double cube_sum(const double* ring, const double* s_wc, int xo, int me) {
-  constexpr int W = 2 * R + 1, WY = DIM == 3 ? W : 1, RY = DIM == 3 ? R : 0;
-  double sv = 0.0;
-#pragma unroll
-  for (int ix = 0; ix < W; ++ix) {
-    const double* p = ring + ((xo + ix - R) & (RING - 1)) * PL + me;
-#pragma unroll
-    for (int iy = 0; iy < WY; ++iy)
-#pragma unroll
-      for (int iz = 0; iz < W; ++iz) {
-        const double wk = s_wc[(ix * WY + iy) * W + iz];
-        const double v = p[(iy - RY) * PZ + iz - R];
-        sv = wk != 0.0 ? fma(wk, v, sv) : sv;
-      }
-  }
-  return sv;
-}
+// The offset table in LDS, with what the kernels derive from it.
+struct TapTable {
+  double w[kMaxTaps];
+  int d[kMaxTaps];      // dx, dy, dz + 8, 5 bits each (radii up to 7)
+  double cube[125];     // weight at each position of the (2 rc + 1)^3 cube, 0 where there is no tap
+  double bw[125];       // weight sum of every boundary class (forward)
+  int r[3];             // radius per axis
+  int odd;              // the march does not apply: order, duplicates or asymmetric weights
+};
 
-// MODE 1: forward, 2: transpose (values v / N), 3: SIMP adjoint (values s / N).
-// Tile: TY x TZ outputs per plane (3-D TY x 64, 2-D 1 x 256), one per thread.  Ring of
-// 8 element planes (x mod 8): 2 kMaxR + 1 in use plus the one being filled.  EN (MODE 3, 3-D): 1 = the
-// element energy in the transformed basis (element matrices with the brick's reflection
-// structure, chosen on the host), 2 = the full product; EN + 4: a penalty other than 3.
-template <int MODE, int DIM, int EN, int TY>
-__global__ __launch_bounds__(DIM == 3 ? 64 * TY : 256)
-__attribute__((amdgpu_waves_per_eu(MODE == 3 ? 2 : 4))) void stencil_kernel(const Grid g, const SGrid sg, int cx,
-                                                                          int n_off,
-                                                      const int32_t* __restrict__ off,
-                                                      const double* __restrict__ w,
-                                                      const double* __restrict__ x,
-                                                      const AdjArgs adj,
-                                                      double* __restrict__ y) {
-  static_assert(DIM == 3 || TY == 1, "2-D tiles are one row");
-  constexpr int TZ = DIM == 3 ? 64 : 256, NT = TY * TZ;
-  constexpr int RYM = DIM == 3 ? kMaxR : 0;  // y halo capacity (2-D grids have one y row)
-  constexpr int PY = TY + 2 * RYM, PZ = TZ + 2 * kMaxR, PL = PY * PZ;
-  constexpr int RING = 8;
-  constexpr int NK = MODE == 3 ? (DIM == 3 ? 576 : 64) : 1;
-  __shared__ double ring[RING * PL];
-  __shared__ int s_tap[kMaxTaps];  // dx + 8 in bits 16+, in-plane LDS offset dy * PZ + dz + 2^15 below
-  __shared__ double s_w[kMaxTaps];
-  __shared__ double sK[NK];
-  __shared__ double sG[MODE == 3 ? 63 : 1];
-  __shared__ int s_r[3];
-  // MODE 1: weight sum of every boundary class.  An output's in-grid taps depend only on its
-  // distances to the six faces clipped to the radius, (lx, hx, ly, hy, lz, hz) in [0, r]^6.
-  constexpr int NB = MODE == 1 ? (DIM == 3 ? 729 : 81) : 1;
-  __shared__ double s_bw[NB];
-  __shared__ int s_d[kMaxTaps];  // dx, dy, dz + 8, 5 bits each
-  constexpr int NC = DIM == 3 ? 125 : 25;  // (2 kMaxR + 1)^DIM cube positions
-  __shared__ double s_wc[NC];
-  __shared__ int s_cube;
+// One block-wide pass over the table.  Returns with the radii, and in 3-D with the cube of
+// weights and `odd` set, behind a barrier.
+template <int DIM, int NT>
+__device__ __forceinline__ void load_taps(TapTable& T, int n_off, const int32_t* __restrict__ off,
+                                          const double* __restrict__ w) {
   const int tid = threadIdx.x;
-  if (tid < 3) s_r[tid] = 0;
-  for (int t = tid; t < NC; t += NT) s_wc[t] = 0.0;
-  if (MODE == 3)
-    for (int t = tid; t < NK; t += NT) sK[t] = adj.K0[t];
+  if (tid < 3) T.r[tid] = 0;
+  if (tid == 3) T.odd = 0;
+  if (DIM == 3)
+    for (int t = tid; t < 125; t += NT) T.cube[t] = 0.0;
   __syncthreads();
   for (int t = tid; t < n_off; t += NT) {
     const int dx = off[t * DIM];
     const int dy = DIM == 3 ? off[t * 3 + 1] : 0;
     const int dz = DIM == 3 ? off[t * 3 + 2] : off[t * 2 + 1];
-    s_tap[t] = ((dx + 8) << 16) | (dy * PZ + dz + (1 << 15));
-    s_w[t] = w[t];
-    s_d[t] = ((dx + 8) << 10) | ((dy + 8) << 5) | (dz + 8);
-    atomicMax(&s_r[0], abs(dx));
-    atomicMax(&s_r[1], abs(dy));
-    atomicMax(&s_r[2], abs(dz));
-  }
-  if (MODE == 3 && DIM == 3 && (EN & 3) == 1 && tid < 63) {
-    // kept couplings of G = H K0 H / 64
-    const int M = 1 + tid / 9, c = (tid / 3) % 3, d = tid % 3;
-    const int Mp = M ^ (1 << c) ^ (1 << d);
-    double sum = 0.0;
-    for (int bb = 0; bb < 8; ++bb)
-      for (int bp = 0; bp < 8; ++bp) {
-        const double k = sK[(3 * fcorner(bb) + c) * 24 + 3 * fcorner(bp) + d];
-        sum += ((__builtin_popcount(M & bb) ^ __builtin_popcount(Mp & bp)) & 1) ? -k : k;
-      }
-    sG[tid] = fk_kept(M, c, d) ? sum / 64.0 : 0.0;
+    T.w[t] = w[t];
+    T.d[t] = ((dx + 8) << 10) | ((dy + 8) << 5) | (dz + 8);
+    if (dx != 0) atomicMax(&T.r[0], abs(dx));
+    if (dy != 0) atomicMax(&T.r[1], abs(dy));
+    if (dz != 0) atomicMax(&T.r[2], abs(dz));
   }
   __syncthreads();
-  const int rx = s_r[0], ry = DIM == 3 ? s_r[1] : 0, rz = s_r[2];
-  const bool wide = rx > kMaxR || ry > RYM || rz > kMaxR;
-  // boundary classes: index ((((lx * (rx+1) + hx) * (ry+1) + ly) * (ry+1) + hy) * (rz+1) + lz) * (rz+1) + hz;
-  // each sum adds the in-grid taps in tap order, as the reference's loop does
-  const int bx = rx + 1, by = ry + 1, bz = rz + 1;
-  // cube form of the tap sum: taps strictly ascending in (dx, dy, dz), radius <= kMaxR
-  const int rc = max(rx, max(ry, rz));
-  if (!wide) {
-    const int wc = 2 * rc + 1, wcy = DIM == 3 ? wc : 1, rcy = DIM == 3 ? rc : 0;
-    for (int t = tid; t < n_off; t += NT) {
-      const int d = s_d[t];
-      const int dx = (d >> 10) - 8, dy = ((d >> 5) & 31) - 8, dz = (d & 31) - 8;
-      s_wc[((dx + rc) * wcy + dy + rcy) * wc + dz + rc] = s_w[t];
-    }
-    if (tid == 0) {
-      int ok = 1;
-      for (int t = 1; t < n_off; ++t) ok &= s_d[t] > s_d[t - 1];
-      s_cube = ok;
-    }
-    __syncthreads();
+  if (DIM != 3) return;
+  const int rm = max(T.r[0], max(T.r[1], T.r[2]));
+  if (rm > kMaxR) return;
+  const int rc = max(rm, 1), wc = 2 * rc + 1;
+  for (int t = tid; t < n_off; t += NT) {
+    const int d = T.d[t];
+    T.cube[(((d >> 10) - 8 + rc) * wc + ((d >> 5) & 31) - 8 + rc) * wc + (d & 31) - 8 + rc] = T.w[t];
+    if (t > 0 && T.d[t - 1] >= d) T.odd = 1;
   }
-  const bool cube = !wide && s_cube != 0;
-  if (MODE == 1 && !wide) {
-    const int nbc = bx * bx * by * by * bz * bz;
-    for (int c = tid; c < nbc; c += NT) {
-      int r = c;
-      const int hz = r % bz; r /= bz;
-      const int lz = r % bz; r /= bz;
-      const int hy = r % by; r /= by;
-      const int ly = r % by; r /= by;
-      const int hx = r % bx, lx = r / bx;
-      double ws = 0.0;
-      for (int t = 0; t < n_off; ++t) {
-        const int d = s_d[t];
-        const int dx = (d >> 10) - 8, dy = ((d >> 5) & 31) - 8, dz = (d & 31) - 8;
-        ws += (dx >= -lx && dx <= hx && dy >= -ly && dy <= hy && dz >= -lz && dz <= hz) ? s_w[t] : 0.0;
-      }
-      s_bw[c] = ws;
-    }
-    __syncthreads();
+  __syncthreads();
+  for (int t = tid; t < wc * wc * wc; t += NT) {
+    const int iz = t % wc, iy = (t / wc) % wc, ix = t / (wc * wc);
+    const int m = (max(ix, 2 * rc - ix) * wc + max(iy, 2 * rc - iy)) * wc + max(iz, 2 * rc - iz);
+    if (T.cube[t] != T.cube[m]) T.odd = 1;
   }
+  __syncthreads();
+}
 
-  const int y0 = blockIdx.x * TY, z0 = blockIdx.y * TZ;
-  const int x0 = blockIdx.z * cx, x1 = min(x0 + cx, sg.X);
-  const int ty = tid / TZ, tz = tid % TZ;
+// Boundary classes of one axis: an output's in-grid taps depend only on its distances to the two
+// ends clipped to the radius.  S >= 2R + 1 positions fall into 2R + 1 classes, fewer into S.
+__device__ __forceinline__ int axis_class(int o, int S, int R) {
+  if (S <= 2 * R + 1) return o;
+  return o < R ? o : (o > S - 1 - R ? 2 * R - (S - 1 - o) : R);
+}
+// (distance to the low end, distance to the high end), clipped, of class c
+__device__ __forceinline__ void class_reach(int c, int S, int R, int& lo, int& hi) {
+  const int o = S <= 2 * R + 1 ? c : (c <= R ? c : S - 1 - (2 * R - c));
+  lo = min(o, R);
+  hi = min(S - 1 - o, R);
+}
+
+// the value in a scalar register (every lane holds the same)
+__device__ __forceinline__ double scalar_of(double v) {
+  const int2 b = __builtin_bit_cast(int2, v);
+  return __builtin_bit_cast(double, int2{__builtin_amdgcn_readfirstlane(b.x), __builtin_amdgcn_readfirstlane(b.y)});
+}
+
+// Weights by (|dx|, |dy|, |dz|) in scalar registers.
+template <int R>
+struct ClassWeights {
+  static constexpr int W = R + 1;
+  double w[W * W * W];
+  __device__ __forceinline__ void load(const TapTable& T) {
+    constexpr int C = 2 * R + 1;
+#pragma unroll
+    for (int k = 0; k < W * W * W; ++k)
+      w[k] = scalar_of(T.cube[((R + k / (W * W)) * C + R + (k / W) % W) * C + R + k % W]);
+  }
+};
+
+// Adds plane xs to the outputs xs - R .. xs + R held in a[0 .. 2R] (dx = R .. -R), the in-plane taps in
+// ascending (dy, dz): together with the march along x every output sums its taps in the offset
+// table's ascending order.  Each value is read from LDS once for its 2R + 1 outputs.  Cube positions
+// without a tap add an exact zero while the values are finite; an output that is not finite is
+// recomputed from the table's own taps (a zero weight times an infinity must not count).
+template <int R, int PZ, bool ROWS = false>
+__device__ __forceinline__ void add_plane(const double* me, const ClassWeights<R>& cw, double (&a)[2 * R + 1]) {
+  constexpr int C = 2 * R + 1, W = R + 1;
+#pragma unroll
+  for (int iy = 0; iy < C; ++iy) {
+    if (ROWS) asm volatile("" ::: "memory");  // one row's values in registers at a time
+    const int ay = iy < R ? R - iy : iy - R;
+#pragma unroll
+    for (int iz = 0; iz < C; ++iz) {
+      const int az = iz < R ? R - iz : iz - R;
+      const double v = me[(iy - R) * PZ + iz - R];
+#pragma unroll
+      for (int j = 0; j < C; ++j) {
+        const int ax = j < R ? R - j : j - R;
+        a[j] = fma(cw.w[(ax * W + ay) * W + az], v, a[j]);
+      }
+    }
+  }
+}
+
+// Taps beyond the march (radius above kMaxR, or a table in another order or without the mirror
+// symmetry): gathers from memory, the adjoint recomputing each tap's value.
+template <int MODE, int DIM, int EN>
+__device__ __forceinline__ void wide_taps(const Grid& g, const SGrid& sg, int x0, int x1, int oy, int oz, int n_off,
+                                          const int32_t* __restrict__ off, const TapTable& T,
+                                          const double* __restrict__ x, const AdjArgs& adj, const double* sK,
+                                          const double* sG, double* __restrict__ y) {
+#pragma unroll 1
+  for (int xo = x0; xo < x1; ++xo) {
+    double sv = 0.0, sw = 0.0;
+#pragma unroll 1
+    for (int t = 0; t < n_off; ++t) {
+      const int dx = off[t * DIM];
+      const int dy = DIM == 3 ? off[t * 3 + 1] : 0;
+      const int dz = DIM == 3 ? off[t * 3 + 2] : off[t * 2 + 1];
+      const int a = xo + dx, b = oy + dy, c = oz + dz;
+      if (a < 0 || a >= sg.X || b < 0 || b >= sg.Y || c < 0 || c >= sg.Z) continue;
+      if (MODE == 3) asm volatile("" ::: "memory");
+      sv = fma(T.w[t], stencil_value<MODE, DIM, EN>(g, sg, a, b, c, x, adj, sK, sG), sv);
+      sw += T.w[t];
+    }
+    const int64_t e = ((int64_t)xo * sg.Y + oy) * sg.Z + oz;
+    y[e] = MODE == 1 ? (sw > 0.0 ? sv / sw : 0.0) : sv;
+  }
+}
+
+// ------------------------------------------------- 3-D forward, transpose ---
+
+// Marches planes x0 - R .. x1 - 1 + R through two LDS planes.  A plane's loads are issued PD steps
+// before it is stored, unconditionally (slots outside the grid read a clamped element and are
+// zeroed at the store), so no wait but the store's own touches them.  Returns whether all of the
+// thread's outputs are finite.
+template <int MODE, int R, int TY>
+__device__ __forceinline__ bool march(const SGrid& sg, int x0, int x1, int y0, int z0, const TapTable& T,
+                                      double* planes, const double* __restrict__ x,
+                                      const double* __restrict__ norm, double* __restrict__ y) {
+  constexpr int NT = 64 * TY, PY = TY + 2 * R, PZ = 64 + 2 * R, PL = PY * PZ;
+  constexpr int KP = (PL + NT - 1) / NT, PD = 4;
+  const int tid = threadIdx.x, ty = tid >> 6, tz = tid & 63;
   const int oy = y0 + ty, oz = z0 + tz;
   const bool mine = oy < sg.Y && oz < sg.Z;
-  if (wide) {
-    // taps beyond the ring: gathers from memory (the adjoint recomputes each tap's value)
-    if (!mine) return;
-#pragma unroll 1
-    for (int xo = x0; xo < x1; ++xo) {
-      double sv = 0.0, sw = 0.0;
-#pragma unroll 1
-      for (int t = 0; t < n_off; ++t) {
-        const int dx = off[t * DIM];
-        const int dy = DIM == 3 ? off[t * 3 + 1] : 0;
-        const int dz = DIM == 3 ? off[t * 3 + 2] : off[t * 2 + 1];
-        const int a = xo + dx, b = oy + dy, c = oz + dz;
-        if (a < 0 || a >= sg.X || b < 0 || b >= sg.Y || c < 0 || c >= sg.Z) continue;
-        if (MODE == 3) asm volatile("" ::: "memory");
-        sv = fma(s_w[t], stencil_value<MODE, DIM, EN>(g, sg, a, b, c, x, adj, sK, sG), sv);
-        sw += s_w[t];
-      }
-      const int64_t e = ((int64_t)xo * sg.Y + oy) * sg.Z + oz;
-      y[e] = MODE == 1 ? (sw > 0.0 ? sv / sw : 0.0) : sv;
-    }
-    return;
-  }
-  const int py = TY + 2 * ry, pz = TZ + 2 * rz, pn = py * pz;
-  // A plane is staged in two halves: fetch() forms this thread's values of plane xs in
-  // registers (zero outside the grid), put() stores them to ring slot xs mod 8.  The loop
-  // fetches plane xo + rx + 1 before it computes plane xo, so the loads are in flight during
-  // the taps; the ring's spare slot (8 > 2 rx + 1) means the store needs no extra barrier.
-  constexpr int KP = (PL + NT - 1) / NT;
-  // MODES 1 and 2: plane xs is fetched into registers PD steps before it is stored to its
-  // ring slot, so PD planes' loads are in flight while the taps run.  MODE 3 computes each
-  // staged value (an element energy) and stores it at once, one at a time: holding a
-  // plane's share across the taps would take most of the register file.  A ring slot is
-  // written one step before it is read and is not in use then (8 slots, at most
-  // 2 rx + 1 = 5 read per step).
-  constexpr bool kDirect = MODE == 3;
-  constexpr int PD = kDirect ? 1 : 4;
-  double pre[PD][KP];
-  // per staged slot q: its element's offset within a plane (-1: outside the grid in y or z)
-  // and its LDS offset (-1: past the tile); both are the same for every plane
-  int qe[KP], ql[KP];
+  ClassWeights<R> cw;
+  cw.load(T);
+  int qe[KP];  // element of the slot within a plane, -1 outside the grid
 #pragma unroll
   for (int q = 0; q < KP; ++q) {
     const int t = tid + NT * q;
-    const int ly = t / pz, lz = t - ly * pz;
-    const int gy = y0 - ry + ly, gz = z0 - rz + lz;
-    const bool in = t < pn;
-    ql[q] = in ? (ly + RYM - ry) * PZ + lz + kMaxR - rz : -1;
-    qe[q] = in && gy >= 0 && gy < sg.Y && gz >= 0 && gz < sg.Z ? gy * sg.Z + gz : -1;
+    const int gy = y0 - R + t / PZ, gz = z0 - R + t % PZ;
+    qe[q] = t < PL && gy >= 0 && gy < sg.Y && gz >= 0 && gz < sg.Z ? gy * sg.Z + gz : -1;
   }
-  // the loads are unconditional (slots outside the grid read element 0 and are zeroed
-  // afterwards), so the loop has no branches around them and a plane's loads stay in
-  // flight across the steps until its store
-  // MODE 2 also keeps N of each slot (prn), the quotient v / N is formed at the store
-  double prn[MODE == 2 ? PD : 1][KP];
+  const int YZ = sg.Y * sg.Z;
+  double pre[PD][KP], prn[MODE == 2 ? PD : 1][KP];
   auto fetch = [&](double (&r)[KP], double (&rn)[KP], int xs) {
-    // planes outside the grid read the nearest one (every lane loads, no branch)
-    const int64_t base = (int64_t)min(max(xs, 0), sg.X - 1) * sg.Y * sg.Z;
+    const int base = min(max(xs, 0), sg.X - 1) * YZ;
 #pragma unroll
     for (int q = 0; q < KP; ++q) {
-      const int64_t e = base + max(qe[q], 0);
+      const int e = base + max(qe[q], 0);
       r[q] = x[e];
-      if (MODE == 2) rn[q] = adj.norm[e];
+      if (MODE == 2) rn[q] = norm[e];
     }
   };
   auto put = [&](const double (&r)[KP], const double (&rn)[KP], int xs) {
-    double* pl = ring + (xs & (RING - 1)) * PL;
+    double* pl = planes + (xs & 1) * PL;
     const bool xin = xs >= 0 && xs < sg.X;
 #pragma unroll
     for (int q = 0; q < KP; ++q) {
       const double v = MODE == 2 ? r[q] / rn[q] : r[q];
-      if (ql[q] >= 0) pl[ql[q]] = xin && qe[q] >= 0 ? v : 0.0;
+      if ((q + 1) * NT <= PL || tid + NT * q < PL) pl[tid + NT * q] = xin && qe[q] >= 0 ? v : 0.0;
     }
   };
-  auto fill = [&](int xs) {
-    double* pl = ring + (xs & (RING - 1)) * PL;
-#pragma unroll 1
-    for (int q = 0; q < KP; ++q) {
-      const int t = tid + NT * q;
-      if (t < pn) {
-        const int ly = t / pz, lz = t - (t / pz) * pz;
-        const int gy = y0 - ry + ly, gz = z0 - rz + lz;
-        double v = 0.0;
-        asm volatile("" ::: "memory");  // K0 / G re-read from LDS per element
-        if (xs >= 0 && xs < sg.X && gy >= 0 && gy < sg.Y && gz >= 0 && gz < sg.Z)
-          v = stencil_value<MODE, DIM, EN>(g, sg, xs, gy, gz, x, adj, sK, sG);
-        pl[(ly + RYM - ry) * PZ + lz + kMaxR - rz] = v;
+  double a[2 * R + 1];
+#pragma unroll
+  for (int j = 0; j <= 2 * R; ++j) a[j] = 0.0;
+  const int ncy = min(sg.Y, 2 * R + 1), ncz = min(sg.Z, 2 * R + 1);
+  const int cyz = MODE == 1 && mine ? axis_class(oy, sg.Y, R) * ncz + axis_class(oz, sg.Z, R) : 0;
+  bool fine = true;
+  auto step = [&](int xs) {
+    add_plane<R, PZ>(planes + (xs & 1) * PL + (ty + R) * PZ + tz + R, cw, a);
+    const int xo = xs - R;
+    if (xo >= x0 && mine) {
+      double out = a[0];
+      if (MODE == 1) {
+        const double sw = T.bw[axis_class(xo, sg.X, R) * (ncy * ncz) + cyz];
+        out = sw > 0.0 ? out / sw : 0.0;
       }
-    }
-  };
-  // this output's boundary class in y and z (x is added per plane)
-  const int byz = ((min(oy, ry) * by + min(sg.Y - 1 - oy, ry)) * bz + min(oz, rz)) * bz + min(sg.Z - 1 - oz, rz);
-  const int me = (ty + RYM) * PZ + tz + kMaxR - (1 << 15);
-  auto taps = [&](int xo) {
-    if (!mine) return;
-    double sv = 0.0;
-    // the cube weights are re-read from LDS per plane (uniform broadcasts), not held in
-    // registers across the march
-    asm volatile("" ::: "memory");
-    if (cube && rc == 1) {
-      sv = cube_sum<1, DIM, PZ, PL, RING>(ring, s_wc, xo, me + (1 << 15));
-    } else if (cube && rc == 2) {
-      sv = cube_sum<2, DIM, PZ, PL, RING>(ring, s_wc, xo, me + (1 << 15));
-    } else {
-      for (int t = 0; t < n_off; ++t) {
-        const int tp = s_tap[t];
-        const int slot = (xo + (tp >> 16) - 8) & (RING - 1);
-        sv = fma(s_w[t], ring[slot * PL + (tp & 0xffff) + me], sv);
-      }
-    }
-    double out = sv;
-    if (MODE == 1) {
-      const double sw = s_bw[(min(xo, rx) * bx + min(sg.X - 1 - xo, rx)) * (by * by * bz * bz) + byz];
-      out = sw > 0.0 ? sv / sw : 0.0;
-    }
-    y[((int64_t)xo * sg.Y + oy) * sg.Z + oz] = out;
-  };
-  if (kDirect) {
-    for (int xs = x0 - rx; xs <= x0 + rx; ++xs) fill(xs);
-    for (int xo = x0; xo < x1; ++xo) {
-      __syncthreads();
-      if (xo + 1 < x1) fill(xo + rx + 1);
-      taps(xo);
-    }
-  } else {
-    // planes x0 - rx .. x0 + rx - 1 go to the ring now; x0 + rx + k is in flight in pre[k]
-    for (int xs = x0 - rx; xs < x0 + rx; ++xs) {
-      fetch(pre[0], prn[0], xs);
-      put(pre[0], prn[0], xs);
+      y[xo * YZ + oy * sg.Z + oz] = out;
+      fine = fine && isfinite(out);
     }
 #pragma unroll
-    for (int k = 0; k < PD; ++k)
-      if (x0 + k < x1) fetch(pre[k], prn[MODE == 2 ? k : 0], x0 + rx + k);
-    // step xo stores plane xo + rx from pre[k] and refills pre[k] with plane xo + rx + PD.
-    // Whole groups of PD steps run without conditions (planes past the grid are fetched
-    // clamped and never stored), so every path through the loop issues the same loads and
-    // each store waits only for its own plane's loads.
-    int xb = x0;
-    for (; xb + PD <= x1; xb += PD) {
+    for (int j = 0; j < 2 * R; ++j) a[j] = a[j + 1];
+    a[2 * R] = 0.0;
+  };
+  const int xe = x1 + R;  // one past the last plane
 #pragma unroll
-      for (int k = 0; k < PD; ++k) {
-        const int xo = xb + k;
-        put(pre[k], prn[MODE == 2 ? k : 0], xo + rx);
-        __syncthreads();
-        fetch(pre[k], prn[MODE == 2 ? k : 0], xo + rx + PD);
-        taps(xo);
-      }
-    }
+  for (int k = 0; k < PD; ++k) fetch(pre[k], prn[MODE == 2 ? k : 0], x0 - R + k);
+  // groups of PD steps whose loads and stores have no conditions: every path issues the same ones
+  for (int xb = x0 - R; xb < xe; xb += PD) {
 #pragma unroll
     for (int k = 0; k < PD; ++k) {
-      const int xo = xb + k;
-      if (xo < x1) {
-        put(pre[k], prn[MODE == 2 ? k : 0], xo + rx);
-        __syncthreads();
-        taps(xo);
-      }
+      put(pre[k], prn[MODE == 2 ? k : 0], xb + k);
+      __syncthreads();
+      fetch(pre[k], prn[MODE == 2 ? k : 0], xb + k + PD);
+      if (xb + k < xe) step(xb + k);
     }
   }
+  return fine;
+}
+
+// MODE 1: forward, 2: transpose (values v / N).  Tile: TY x 64 outputs per plane, one per thread.
+template <int MODE, int TY>
+__global__ __launch_bounds__(64 * TY) __attribute__((amdgpu_waves_per_eu(4))) void march_kernel(
+    const Grid g, const SGrid sg, int cx, int n_off, const int32_t* __restrict__ off, const double* __restrict__ w,
+    const double* __restrict__ x, const double* __restrict__ norm, double* __restrict__ y) {
+  constexpr int NT = 64 * TY;
+  __shared__ TapTable T;
+  __shared__ double planes[2 * (TY + 2 * kMaxR) * (64 + 2 * kMaxR)];
+  const int tid = threadIdx.x;
+  load_taps<3, NT>(T, n_off, off, w);
+  const int rm = max(T.r[0], max(T.r[1], T.r[2])), rc = max(rm, 1);
+  const int y0 = blockIdx.x * TY, z0 = blockIdx.y * 64;
+  const int x0 = blockIdx.z * cx, x1 = min(x0 + cx, sg.X);
+  bool fine = false;
+  if (rm <= kMaxR && !T.odd) {
+    if (MODE == 1) {
+      const int nx = min(sg.X, 2 * rc + 1), ny = min(sg.Y, 2 * rc + 1), nz = min(sg.Z, 2 * rc + 1);
+      for (int c = tid; c < nx * ny * nz; c += NT) {
+        int lx, hx, ly, hy, lz, hz;
+        class_reach(c / (ny * nz), sg.X, rc, lx, hx);
+        class_reach((c / nz) % ny, sg.Y, rc, ly, hy);
+        class_reach(c % nz, sg.Z, rc, lz, hz);
+        double ws = 0.0;
+        for (int t = 0; t < n_off; ++t) {
+          const int d = T.d[t];
+          const int dx = (d >> 10) - 8, dy = ((d >> 5) & 31) - 8, dz = (d & 31) - 8;
+          ws += (dx >= -lx && dx <= hx && dy >= -ly && dy <= hy && dz >= -lz && dz <= hz) ? T.w[t] : 0.0;
+        }
+        T.bw[c] = ws;  // made visible by the march's first barrier
+      }
+    }
+    fine = rc == 1 ? march<MODE, 1, TY>(sg, x0, x1, y0, z0, T, planes, x, norm, y)
+                   : march<MODE, 2, TY>(sg, x0, x1, y0, z0, T, planes, x, norm, y);
+  }
+  const int oy = y0 + (tid >> 6), oz = z0 + (tid & 63);
+  if (!fine && oy < sg.Y && oz < sg.Z) {
+    AdjArgs adj{};
+    adj.norm = norm;
+    wide_taps<MODE, 3, 0>(g, sg, x0, x1, oy, oz, n_off, off, T, x, adj, nullptr, nullptr, y);
+  }
+}
+
+// ------------------------------------------------------- 3-D SIMP adjoint ---
+
+// Energy coefficients of the transformed basis, G[M][c][c] at (M - 1) * 3 + c, then for each pair
+// c < d (third axis t) the four couplings uh_c[M] uh_d[M ^ e_c ^ e_d], M in {e_c, e_d, e_c + e_t,
+// e_d + e_t}, with both of K0's entries for them added up.
+constexpr int kEnDiag = 21, kEnCoef = 33;
+__host__ __device__ constexpr int en_pair_c(int p) { return p == 2 ? 1 : 0; }
+__host__ __device__ constexpr int en_pair_d(int p) { return p == 0 ? 1 : 2; }
+__host__ __device__ constexpr int en_pair_M(int p, int m) {
+  const int c = 1 << en_pair_c(p), d = 1 << en_pair_d(p), t = 7 ^ c ^ d;
+  return (m & 1 ? d : c) | (m & 2 ? t : 0);
+}
+
+// 4-point transform over (y, z) of one x face of an element: corner (by, bz) at 2 bz + by
+struct Face {
+  double f[3][4];
+};
+__device__ __forceinline__ void load_face(Face& f, const double* __restrict__ U, int m, int sy) {
+#pragma unroll
+  for (int b = 0; b < 4; ++b)
+#pragma unroll
+    for (int c = 0; c < 3; ++c) f.f[c][b] = U[(m + (b & 1) * sy + (b >> 1)) * 3 + c];
+}
+__device__ __forceinline__ void face_transform(Face& f) {
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    const double p = f.f[c][0] + f.f[c][1], q = f.f[c][0] - f.f[c][1];
+    const double r = f.f[c][2] + f.f[c][3], s = f.f[c][2] - f.f[c][3];
+    f.f[c][0] = p + r;
+    f.f[c][1] = q + s;
+    f.f[c][2] = p - r;
+    f.f[c][3] = q - s;
+  }
+}
+// -u^T K0 u from the transformed faces at x (lo) and x + 1 (hi)
+__device__ __forceinline__ double face_energy(const Face& lo, const Face& hi, const double* sC) {
+  double u[3][8];
+#pragma unroll
+  for (int c = 0; c < 3; ++c)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      u[c][2 * k] = lo.f[c][k] + hi.f[c][k];
+      u[c][2 * k + 1] = lo.f[c][k] - hi.f[c][k];
+    }
+  double e = 0.0;
+#pragma unroll
+  for (int M = 1; M < 8; ++M)
+#pragma unroll
+    for (int c = 0; c < 3; ++c) e = fma(sC[(M - 1) * 3 + c], u[c][M] * u[c][M], e);
+#pragma unroll
+  for (int p = 0; p < 3; ++p)
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      constexpr int kPair[3][2] = {{0, 1}, {0, 2}, {1, 2}};
+      const int c = kPair[p][0], d = kPair[p][1], M = en_pair_M(p, m);
+      e = fma(sC[kEnDiag + 4 * p + m], u[c][M] * u[d][M ^ (1 << c) ^ (1 << d)], e);
+    }
+  return -e;
+}
+
+// One staged value per thread and plane, s_e / N_e (about 120 FP64 operations: VALU bound, 34 to 21 us
+// at 128 x 64 x 64 against 24 gathered displacements and 45 couplings per value).  In the transformed basis (EN & 3 == 1) a thread
+// keeps its element column's x + 1 face for the next plane, so each node column is read once per
+// plane; any other K0 takes the full product.
+template <int EN, int R, int TY>
+__device__ __forceinline__ bool march_adjoint(const Grid& g, const SGrid& sg, int x0, int x1, int y0, int z0,
+                                              const TapTable& T, double* planes, const AdjArgs& adj,
+                                              const double* sK, const double* sC, double* __restrict__ y) {
+  constexpr int PY = TY + 2 * R, PZ = 64 + 2 * R, PL = PY * PZ;
+  constexpr bool WHT = (EN & 3) == 1;
+  const int tid = threadIdx.x, ty = tid >> 6, tz = tid & 63;
+  const int oy = y0 + ty, oz = z0 + tz;
+  const bool mine = ty < TY && oy < sg.Y && oz < sg.Z;
+  const int gy = y0 - R + tid / PZ, gz = z0 - R + tid % PZ;
+  const bool slot = tid < PL, in = slot && gy >= 0 && gy < sg.Y && gz >= 0 && gz < sg.Z;
+  const int cy = min(max(gy, 0), sg.Y - 1), cz = min(max(gz, 0), sg.Z - 1);
+  const int YZ = sg.Y * sg.Z, nz = g.nz(), sy = g.nx() * nz;
+  const int q = cy * sg.Z + cz, m = cy * sy + cz;  // this slot's element in plane 0 and its first node
+  ClassWeights<R> cw;
+  cw.load(T);
+  Face lo, hi;
+  double xv = 0.0, nv = 1.0;
+  // operands of plane xs: the face at xs + 1, the density and N (clamped to the grid)
+  auto fetch = [&](int xs) {
+    const int xc = min(max(xs, 0), sg.X - 1);
+    if (WHT) load_face(hi, adj.U, m + (xc + 1) * nz, sy);
+    xv = adj.xt[xc * YZ + q];
+    nv = adj.norm[xc * YZ + q];
+  };
+  double a[2 * R + 1];
+#pragma unroll
+  for (int j = 0; j <= 2 * R; ++j) a[j] = 0.0;
+  if (WHT) {
+    load_face(lo, adj.U, m + min(max(x0 - R, 0), sg.X - 1) * nz, sy);
+    face_transform(lo);
+  }
+  fetch(x0 - R);
+  bool fine = true;
+  for (int xs = x0 - R; xs < x1 + R; ++xs) {
+    const bool xin = xs >= 0 && xs < sg.X;
+    double v = 0.0;
+    if (WHT) {
+      if (xin) {
+        face_transform(hi);
+        v = face_energy(lo, hi, sC);
+        lo = hi;
+      }
+    } else if (xin && in) {
+      v = elem_energy3<false>(g, xs, gy, gz, adj.U, sK, nullptr);
+    }
+    const double xe = fmin(fmax(xv, adj.vmin), 1.0);
+    v = simp_factor<(EN & 4) != 0>(xe, adj.penal) * v / nv;
+    if (slot) planes[(xs & 1) * PL + tid] = xin && in ? v : 0.0;
+    fetch(xs + 1);
+    __syncthreads();
+    if (mine) {
+      add_plane<R, PZ, (R > 1)>(planes + (xs & 1) * PL + (ty + R) * PZ + tz + R, cw, a);
+      if (xs - R >= x0) {
+        y[(xs - R) * YZ + oy * sg.Z + oz] = a[0];
+        fine = fine && isfinite(a[0]);
+      }
+#pragma unroll
+      for (int j = 0; j < 2 * R; ++j) a[j] = a[j + 1];
+      a[2 * R] = 0.0;
+    }
+  }
+  return fine;
+}
+
+// threads of the adjoint's workgroup: one staged slot each at the largest radius, whole wavefronts
+__host__ __device__ constexpr int adjoint_threads(int ty) {
+  return ((ty + 2 * kMaxR) * (64 + 2 * kMaxR) + 63) / 64 * 64;
+}
+
+// EN 1: the element energy in the transformed basis (element matrices with the brick's reflection
+// structure, chosen on the host), 2: the full product; EN + 4: a penalty other than 3.
+template <int EN, int TY>
+__global__ __launch_bounds__(adjoint_threads(TY)) void adjoint_kernel(
+    const Grid g, const SGrid sg, int cx, int n_off, const int32_t* __restrict__ off, const double* __restrict__ w,
+    const AdjArgs adj, double* __restrict__ y) {
+  constexpr int NT = adjoint_threads(TY);
+  __shared__ TapTable T;
+  __shared__ double planes[2 * (TY + 2 * kMaxR) * (64 + 2 * kMaxR)];
+  __shared__ double sK[576];
+  __shared__ double sC[kEnCoef];
+  __shared__ double sG[63];
+  const int tid = threadIdx.x;
+  for (int t = tid; t < 576; t += NT) sK[t] = adj.K0[t];
+  load_taps<3, NT>(T, n_off, off, w);  // its barriers also cover sK
+  if ((EN & 3) == 1) {
+    if (tid < 63) {
+      // kept couplings of G = H K0 H / 64
+      const int M = 1 + tid / 9, c = (tid / 3) % 3, d = tid % 3;
+      const int Mp = M ^ (1 << c) ^ (1 << d);
+      double sum = 0.0;
+      for (int bb = 0; bb < 8; ++bb)
+        for (int bp = 0; bp < 8; ++bp) {
+          const double k = sK[(3 * fcorner(bb) + c) * 24 + 3 * fcorner(bp) + d];
+          sum += ((__builtin_popcount(M & bb) ^ __builtin_popcount(Mp & bp)) & 1) ? -k : k;
+        }
+      sG[tid] = fk_kept(M, c, d) ? sum / 64.0 : 0.0;
+    }
+    __syncthreads();
+    if (tid < kEnDiag) sC[tid] = sG[tid / 3 * 9 + tid % 3 * 4];
+    if (tid >= kEnDiag && tid < kEnCoef) {
+      const int p = (tid - kEnDiag) / 4, M = en_pair_M(p, (tid - kEnDiag) % 4);
+      const int c = en_pair_c(p), d = en_pair_d(p), Mp = M ^ (1 << c) ^ (1 << d);
+      sC[tid] = sG[(M - 1) * 9 + c * 3 + d] + sG[(Mp - 1) * 9 + d * 3 + c];
+    }
+    __syncthreads();
+  }
+  const int rm = max(T.r[0], max(T.r[1], T.r[2]));
+  const int y0 = blockIdx.x * TY, z0 = blockIdx.y * 64;
+  const int x0 = blockIdx.z * cx, x1 = min(x0 + cx, sg.X);
+  bool fine = false;
+  if (rm <= kMaxR && !T.odd)
+    fine = rm <= 1 ? march_adjoint<EN, 1, TY>(g, sg, x0, x1, y0, z0, T, planes, adj, sK, sC, y)
+                   : march_adjoint<EN, 2, TY>(g, sg, x0, x1, y0, z0, T, planes, adj, sK, sC, y);
+  const int oy = y0 + (tid >> 6), oz = z0 + (tid & 63);
+  if (!fine && tid < 64 * TY && oy < sg.Y && oz < sg.Z)
+    wide_taps<3, 3, EN>(g, sg, x0, x1, oy, oz, n_off, off, T, nullptr, adj, sK, sG, y);
+}
+
+// -------------------------------------------------------------------- 2-D ---
+
+constexpr int kR2 = 4;                  // halo radius of the 2-D tile (rmin <= 5)
+constexpr int kTX2 = 4, kTZ2 = 64;      // outputs per workgroup, one per thread
+
+// MODE 1: forward, 2: transpose, 3: SIMP adjoint, on one staged tile with its halo.  At most
+// 2^19 outputs in use and all of them in cache: launch and load latency bound, so one
+// workgroup does one tile and meets two barriers.
+template <int MODE, int EN>
+__global__ __launch_bounds__(256) void filter2_kernel(const Grid g, const SGrid sg, int n_off,
+                                                      const int32_t* __restrict__ off,
+                                                      const double* __restrict__ w, const double* __restrict__ x,
+                                                      const AdjArgs adj, double* __restrict__ y) {
+  constexpr int PZ = kTZ2 + 2 * kR2;
+  __shared__ TapTable T;
+  __shared__ double tile[(kTX2 + 2 * kR2) * PZ];
+  __shared__ double sK[MODE == 3 ? 64 : 1];
+  const int tid = threadIdx.x;
+  if (MODE == 3 && tid < 64) sK[tid] = adj.K0[tid];
+  load_taps<2, 256>(T, n_off, off, w);
+  const int rx = T.r[0], rz = T.r[2];
+  const int x0 = blockIdx.y * kTX2, z0 = blockIdx.x * kTZ2;
+  const int ox = x0 + (tid >> 6), oz = z0 + (tid & 63);
+  const bool mine = ox < sg.X && oz < sg.Z;
+  if (rx > kR2 || rz > kR2) {
+    if (mine) wide_taps<MODE, 2, EN>(g, sg, ox, ox + 1, 0, oz, n_off, off, T, x, adj, sK, nullptr, y);
+    return;
+  }
+  const int pz = kTZ2 + 2 * rz, pn = (kTX2 + 2 * rx) * pz;
+  for (int t = tid; t < pn; t += 256) {
+    const int lx = t / pz, lz = t - lx * pz;
+    const int gx = x0 - rx + lx, gz = z0 - rz + lz;
+    double v = 0.0;
+    if (gx >= 0 && gx < sg.X && gz >= 0 && gz < sg.Z)
+      v = stencil_value<MODE, 2, EN>(g, sg, gx, 0, gz, x, adj, sK, nullptr);
+    tile[lx * PZ + lz] = v;
+  }
+  __syncthreads();
+  if (!mine) return;
+  const double* me = tile + ((tid >> 6) + rx) * PZ + (tid & 63) + rz;
+  double sv = 0.0, sw = 0.0;
+#pragma unroll 4
+  for (int t = 0; t < n_off; ++t) {
+    const int d = T.d[t];
+    const int dx = (d >> 10) - 8, dz = (d & 31) - 8;
+    const double wk = T.w[t];
+    sv = fma(wk, me[dx * PZ + dz], sv);
+    if (MODE == 1) sw += ox + dx >= 0 && ox + dx < sg.X && oz + dz >= 0 && oz + dz < sg.Z ? wk : 0.0;
+  }
+  y[(int64_t)ox * sg.Z + oz] = MODE == 1 ? (sw > 0.0 ? sv / sw : 0.0) : sv;
 }
 
 // ------------------------------------------------------------------- host ---
@@ -568,22 +770,48 @@ static int g_stencil_ty = 8;
 void set_stencil_rows(int ty) { g_stencil_ty = ty; }
 int get_stencil_rows() { return g_stencil_ty; }
 
-template <int MODE, int EN>
-static int launch_stencil(const Grid& g, int n_off, const int32_t* off, const double* w, const double* x,
-                          const AdjArgs& adj, double* y, hipStream_t s) {
-  const SGrid sg = sgrid(g);
-  const int ty = g.dim == 3 ? g_stencil_ty : 1, tz = g.dim == 3 ? 64 : 256;
-  const int64_t tiles = (int64_t)((sg.Y + ty - 1) / ty) * ((sg.Z + tz - 1) / tz);
-  // the longest x chunk that still gives about 512 workgroups (two per compute unit)
+// x planes per workgroup: the longest chunk that still gives about 512 workgroups (two per compute unit)
+static int chunk_planes(const SGrid& sg, int ty) {
+  const int64_t tiles = (int64_t)((sg.Y + ty - 1) / ty) * ((sg.Z + 63) / 64);
   int cx = kMaxCX;
   while (cx > 4 && tiles * ((sg.X + cx - 1) / cx) < 512) cx /= 2;
-  const dim3 grid((sg.Y + ty - 1) / ty, (sg.Z + tz - 1) / tz, (sg.X + cx - 1) / cx);
+  return cx;
+}
+
+static dim3 march_grid(const SGrid& sg, int ty, int cx) {
+  return dim3((sg.Y + ty - 1) / ty, (sg.Z + 63) / 64, (sg.X + cx - 1) / cx);
+}
+
+template <int MODE>
+static int launch_filter(const Grid& g, int n_off, const int32_t* off, const double* w, const double* norm,
+                         const double* x, double* y, hipStream_t s) {
+  const SGrid sg = sgrid(g);
+  AdjArgs adj{};
+  adj.norm = norm;
+  const int ty = g_stencil_ty, cx = chunk_planes(sg, ty);
   if (g.dim == 2)
-    stencil_kernel<MODE, 2, EN, 1><<<grid, 256, 0, s>>>(g, sg, cx, n_off, off, w, x, adj, y);
+    filter2_kernel<MODE, 0><<<dim3((sg.Z + kTZ2 - 1) / kTZ2, (sg.X + kTX2 - 1) / kTX2), 256, 0, s>>>(
+        g, sg, n_off, off, w, x, adj, y);
   else if (ty == 4)
-    stencil_kernel<MODE, 3, EN, 4><<<grid, 256, 0, s>>>(g, sg, cx, n_off, off, w, x, adj, y);
+    march_kernel<MODE, 4><<<march_grid(sg, ty, cx), 256, 0, s>>>(g, sg, cx, n_off, off, w, x, norm, y);
   else
-    stencil_kernel<MODE, 3, EN, 8><<<grid, 512, 0, s>>>(g, sg, cx, n_off, off, w, x, adj, y);
+    march_kernel<MODE, 8><<<march_grid(sg, ty, cx), 512, 0, s>>>(g, sg, cx, n_off, off, w, x, norm, y);
+  ET_CHECK_LAUNCH();
+  return ET_OK;
+}
+
+template <int EN>
+static int launch_adjoint(const Grid& g, int n_off, const int32_t* off, const double* w, const AdjArgs& adj,
+                          double* y, hipStream_t s) {
+  const SGrid sg = sgrid(g);
+  const int ty = g_stencil_ty, cx = chunk_planes(sg, ty);
+  if (g.dim == 2)
+    filter2_kernel<3, EN><<<dim3((sg.Z + kTZ2 - 1) / kTZ2, (sg.X + kTX2 - 1) / kTX2), 256, 0, s>>>(
+        g, sg, n_off, off, w, nullptr, adj, y);
+  else if (ty == 4)
+    adjoint_kernel<EN, 4><<<march_grid(sg, ty, cx), adjoint_threads(4), 0, s>>>(g, sg, cx, n_off, off, w, adj, y);
+  else
+    adjoint_kernel<EN, 8><<<march_grid(sg, ty, cx), adjoint_threads(8), 0, s>>>(g, sg, cx, n_off, off, w, adj, y);
   ET_CHECK_LAUNCH();
   return ET_OK;
 }
@@ -598,16 +826,14 @@ int filter_fwd(const Grid& g, int n_off, const int32_t* off, const double* w, co
                double* y, hipStream_t s) {
   ET_REQUIRE(n_off > 0 && n_off <= kMaxOff, "filter offset count out of range (1..1024)");
   if (n_off > kMaxTaps) return launch_gather<1>(g, n_off, off, w, nullptr, x, y, s);
-  return launch_stencil<1, 0>(g, n_off, off, w, x, AdjArgs{}, y, s);
+  return launch_filter<1>(g, n_off, off, w, nullptr, x, y, s);
 }
 
 int filter_adj(const Grid& g, int n_off, const int32_t* off, const double* w, const double* norm,
                const double* v, double* y, hipStream_t s) {
   ET_REQUIRE(n_off > 0 && n_off <= kMaxOff, "filter offset count out of range (1..1024)");
   if (n_off > kMaxTaps) return launch_gather<2>(g, n_off, off, w, norm, v, y, s);
-  AdjArgs a{};
-  a.norm = norm;
-  return launch_stencil<2, 0>(g, n_off, off, w, v, a, y, s);
+  return launch_filter<2>(g, n_off, off, w, norm, v, y, s);
 }
 
 int simp_adjoint(const Grid& g, const double* K0, const double* U, const double* xt, double penal, double vmin,
@@ -617,10 +843,10 @@ int simp_adjoint(const Grid& g, const double* K0, const double* U, const double*
   const AdjArgs a{K0, U, xt, penal, vmin, norm};
   const bool wht = g.dim == 3 && (k0_flags & K0S_WHT);
   if (penal == 3.0)
-    return wht ? launch_stencil<3, 1>(g, n_off, off, w, nullptr, a, y, s)
-               : launch_stencil<3, 2>(g, n_off, off, w, nullptr, a, y, s);
-  return wht ? launch_stencil<3, 5>(g, n_off, off, w, nullptr, a, y, s)
-             : launch_stencil<3, 6>(g, n_off, off, w, nullptr, a, y, s);
+    return wht ? launch_adjoint<1>(g, n_off, off, w, a, y, s)
+               : launch_adjoint<2>(g, n_off, off, w, a, y, s);
+  return wht ? launch_adjoint<5>(g, n_off, off, w, a, y, s)
+             : launch_adjoint<6>(g, n_off, off, w, a, y, s);
 }
 
 }  // namespace et

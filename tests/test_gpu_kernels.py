@@ -198,6 +198,61 @@ def test_filter_tap_orders_and_tiles(nel, rmin, spacing):
         assert torch.equal(outs[(4, order)][1], outs[(8, order)][1])
 
 
+@pytest.mark.parametrize("nel,rmin", [((1, 1, 1), 2.5), ((3, 8, 64), 1.5), ((5, 9, 65), 2.0), ((67, 7, 63), 2.5),
+                                      ((36, 17, 4), 2.9), ((4, 64), 1.5), ((9, 65), 4.4)])
+@pytest.mark.parametrize("values", ["finite", "special"])
+def test_filter_tile_edges_and_special_values(nel, rmin, values):
+    """Forward, transpose and SIMP adjoint at the edges of the tiles and of the x chunks.  An
+    infinity or NaN reaches exactly the outputs that have it among their taps (the cube of the
+    march also holds positions without a tap), and a table with uneven weights is summed as given."""
+    L = _lib()
+    dim, n = len(nel), int(np.prod(nel))
+    rng = np.random.default_rng(21)
+    offs, w = ofilt.offsets_weights(rmin, (1,) * dim)
+    norm = ofilt.normalizer(nel, offs, w)
+    x = rng.uniform(0.1, 1, n)
+    if values == "special":
+        x[rng.integers(0, n, 3)] = [np.inf, np.nan, -np.inf]
+    wu = w * rng.uniform(0.5, 1.5, len(w))
+    for ww in (w, wu):
+        o_t, w_t, y = dev(offs.astype(np.int32)), dev(ww), torch.empty(n, dtype=torch.float64, device="cuda")
+        with np.errstate(invalid="ignore"):
+            refs = _plain_filter(x, nel, offs, ww, None), _plain_filter(x / norm, nel, offs, ww, norm)
+        for name, ref in zip(("et_filter_fwd_f64", "et_filter_adj_f64"), refs):
+            extra = (L.ptr(dev(norm)),) if name == "et_filter_adj_f64" else ()
+            L.call(name, dim, L.nel_arg(nel), len(ww), L.ptr(o_t), L.ptr(w_t), *extra, L.ptr(dev(x)), L.ptr(y),
+                   L.stream())
+            got, ok = y.cpu().numpy(), np.isfinite(ref)
+            assert np.array_equal(np.isnan(got), np.isnan(ref)) and np.array_equal(np.isfinite(got), ok)
+            # at most 93 taps of one sign: a relative error of a few ulps times the sum of magnitudes
+            assert np.all(np.abs(got[ok] - ref[ok]) <= 1e-14 * np.abs(ref[ok]))
+    p = _problem(nel, seed=23)
+    xt = rng.uniform(0.0, 1.0, n)
+    mat = otop.SingleMaterial(void=1e-9, penalty=3.0)
+    ref = ofilt.transpose(mat.grad(xt) * oops.process_dk(p["K0"], p["el"], p["u"]), nel, offs, w, norm)
+    flags = ctypes.c_int(0)
+    K0 = np.ascontiguousarray(p["K0"])
+    L.call("et_k0_structure", dim, K0.ctypes.data_as(ctypes.POINTER(ctypes.c_double)), ctypes.byref(flags))
+    for fl in (flags.value, 0):
+        out = torch.empty(n, dtype=torch.float64, device="cuda")
+        L.call("et_simp_adjoint_f64", dim, L.nel_arg(nel), L.f64(dev(K0)), L.f64(dev(p["u"])), L.f64(dev(xt)), 3.0,
+               1e-9, len(w), L.i32(dev(offs.astype(np.int32))), L.f64(dev(w)), L.f64(dev(norm)), fl, L.f64(out),
+               L.stream())
+        assert rel(out.cpu().numpy(), ref) < 1e-12
+
+
+def _plain_filter(x, nel, offs, w, norm):
+    """Tap by tap over the in-grid neighbours only (norm None: divided by their weight sum)."""
+    c = np.stack(np.unravel_index(np.arange(x.size), nel), 1)
+    y, sw = np.zeros(x.size), np.zeros(x.size)
+    for o, wk in zip(offs, w):
+        q = c + o
+        ok = np.all((q >= 0) & (q < np.array(nel)), axis=1)
+        y[ok] += wk * x[np.ravel_multi_index(tuple(q[ok].T), nel)]
+        sw[ok] += wk
+    return y / sw if norm is None else y
+
+
 @pytest.mark.parametrize("nel", [(8, 4), (12, 6), (8, 4, 4), (6, 4, 8), (7, 5, 3)])
 def test_transfers(nel):
     L = _lib()
