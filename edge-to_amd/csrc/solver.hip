@@ -49,7 +49,7 @@ __device__ __forceinline__ void op_epilogue(int64_t n, const T (&ax)[DIM],
   }
 }
 
-// Level-0 operator, matrix free.  omega is read from device memory.
+// Level-0 operator, matrix free: 3-D grids with a general K0.  omega is read from device memory.
 template <typename T, int DIM, int MODE>
 __global__ __launch_bounds__(256) void op0_kernel(const Grid g, const T* __restrict__ K0,
                                                   const T* __restrict__ E,
@@ -455,6 +455,12 @@ static int op_launch(const MGLevel<T>& L, const MGShared& sh, int mode, const T*
     sh.prof->end(s);
     return st;
   }
+  if (L.level == 0 && g.dim == 2) {
+    const int st = op2d<T>(mode, g, sh.K0<T>(), sh.E<T>(), sh.cons, x, b, L.Dinv, omega, wscale, xadd, y, nullptr,
+                           nullptr, s);
+    sh.prof->end(s);
+    return st;
+  }
   const unsigned grid = grid_for(g.n_nodes());
 #define ET_OP0(DIM, MODE)                                                                   \
   op0_kernel<T, DIM, MODE><<<grid, kBlock, 0, s>>>(g, sh.K0<T>(), sh.E<T>(), sh.cons, x, b, \
@@ -470,10 +476,7 @@ static int op_launch(const MGLevel<T>& L, const MGShared& sh, int mode, const T*
 #define ET_DISPATCH(M)                \
   do {                                \
     if (L.level == 0) {               \
-      if (g.dim == 3)                 \
-        ET_OP0(3, M);                 \
-      else                            \
-        ET_OP0(2, M);                 \
+      ET_OP0(3, M);                   \
     } else {                          \
       if (g.dim == 3)                 \
         ET_OPS(3, M);                 \
@@ -512,7 +515,8 @@ int MGHierarchy<T>::vcycle(int l, MGShared& sh, hipStream_t s, bool x0_ready) {
   } else {
     int it = 1;
     // both precisions (the FP64 sweeps run on 8-slice tiles, where the fused pass is faster)
-    if (l == 0 && n_smooth >= 2 && sh.tiled && !(sizeof(T) == 4 && sh.mfma) && fine_jac0_supported(L.g, sizeof(T))) {
+    if (l == 0 && n_smooth >= 2 &&
+        (L.g.dim == 2 || (sh.tiled && !(sizeof(T) == 4 && sh.mfma) && fine_jac0_supported(L.g, sizeof(T))))) {
       // x0 = w D^-1 b and the first sweep from it in one pass
       ET_TRY(op_launch<T>(L, sh, OP_JAC0, nullptr, L.b, om, ws, nullptr, L.t, s));
       std::swap(L.x, L.t);
@@ -553,9 +557,12 @@ int MGHierarchy<T>::vcycle(int l, MGShared& sh, hipStream_t s, bool x0_ready) {
       } else if (l == 0 && pass + 1 == passes && sh.want_dot) {
         // the preconditioned residual z is final here: r.z partials in the same pass
         sh.prof->begin(ET_PROF_L0_JACADD, s);
-        const int st = op0_wht_jac_add_dot<T>(L.g, (int64_t)L.g.ey * L.g.ez, L.g.ez, sh.wht, sh.E<T>(),
-                                              sh.cons, L.e, L.r, L.Dinv, om, ws, L.x, L.t, L.b,
-                                              sh.dot_part, kRedBlocks, s);
+        const int st =
+            L.g.dim == 2
+                ? op2d<T>(TM_JAC_ADD_DOT, L.g, sh.K0<T>(), sh.E<T>(), sh.cons, L.e, L.r, L.Dinv, om, ws, L.x, L.t,
+                          L.b, sh.dot_part, s)
+                : op0_wht_jac_add_dot<T>(L.g, (int64_t)L.g.ey * L.g.ez, L.g.ez, sh.wht, sh.E<T>(), sh.cons, L.e,
+                                         L.r, L.Dinv, om, ws, L.x, L.t, L.b, sh.dot_part, kRedBlocks, s);
         sh.prof->end(s);
         ET_TRY(st);
         sh.dot_done = true;
@@ -612,23 +619,17 @@ int level0_op(int mode, const Grid& g, const T* K0, const T* E, const uint8_t* c
   if (g.dim == 3 && fine != nullptr && fine_supported(g, sizeof(T)))
     return op0_fine<T>(mode, g, (int64_t)g.ey * g.ez, g.ez, K0, *fine, E, cons, x, b, Dinv, omega, wscale, xadd, y,
                        s);
+  if (g.dim == 2)
+    return op2d<T>(mode, g, K0, E, cons, x, b, Dinv, omega, wscale, xadd, y, nullptr, nullptr, s);
   const unsigned grid = grid_for(g.n_nodes());
-#define ET_L0(DIM, MODE) \
-  op0_kernel<T, DIM, MODE><<<grid, kBlock, 0, s>>>(g, K0, E, cons, x, b, Dinv, omega, wscale, xadd, y)
-#define ET_L0D(MODE)     \
-  do {                   \
-    if (g.dim == 3)      \
-      ET_L0(3, MODE);    \
-    else                 \
-      ET_L0(2, MODE);    \
-  } while (0)
+#define ET_L0(MODE) \
+  op0_kernel<T, 3, MODE><<<grid, kBlock, 0, s>>>(g, K0, E, cons, x, b, Dinv, omega, wscale, xadd, y)
   switch (mode) {
-    case OP_Y: ET_L0D(OP_Y); break;
-    case OP_RES: ET_L0D(OP_RES); break;
-    case OP_JAC: ET_L0D(OP_JAC); break;
-    default: ET_L0D(OP_JAC_ADD); break;
+    case OP_Y: ET_L0(OP_Y); break;
+    case OP_RES: ET_L0(OP_RES); break;
+    case OP_JAC: ET_L0(OP_JAC); break;
+    default: ET_L0(OP_JAC_ADD); break;
   }
-#undef ET_L0D
 #undef ET_L0
   ET_CHECK_LAUNCH();
   return ET_OK;
@@ -874,17 +875,16 @@ int MGSolver::apply_A64(const double* x, double* y, int mode, const double* b) {
     prof.end(s);
     return st;
   }
-  if (g0.dim == 3) {
-    if (mode == OP_Y)
-      op0_kernel<double, 3, OP_Y><<<grid, kBlock, 0, s>>>(g0, sh.K0d, sh.Ed, sh.cons, x, b, nullptr, sh.scal, 1.0, nullptr, y);
-    else
-      op0_kernel<double, 3, OP_RES><<<grid, kBlock, 0, s>>>(g0, sh.K0d, sh.Ed, sh.cons, x, b, nullptr, sh.scal, 1.0, nullptr, y);
-  } else {
-    if (mode == OP_Y)
-      op0_kernel<double, 2, OP_Y><<<grid, kBlock, 0, s>>>(g0, sh.K0d, sh.Ed, sh.cons, x, b, nullptr, sh.scal, 1.0, nullptr, y);
-    else
-      op0_kernel<double, 2, OP_RES><<<grid, kBlock, 0, s>>>(g0, sh.K0d, sh.Ed, sh.cons, x, b, nullptr, sh.scal, 1.0, nullptr, y);
+  if (g0.dim == 2) {
+    const int st = op2d<double>(mode, g0, sh.K0d, sh.Ed, sh.cons, x, b, nullptr, nullptr, 1.0, nullptr, y, nullptr,
+                                nullptr, s);
+    prof.end(s);
+    return st;
   }
+  if (mode == OP_Y)
+    op0_kernel<double, 3, OP_Y><<<grid, kBlock, 0, s>>>(g0, sh.K0d, sh.Ed, sh.cons, x, b, nullptr, sh.scal, 1.0, nullptr, y);
+  else
+    op0_kernel<double, 3, OP_RES><<<grid, kBlock, 0, s>>>(g0, sh.K0d, sh.Ed, sh.cons, x, b, nullptr, sh.scal, 1.0, nullptr, y);
   prof.end(s);
   ET_CHECK_LAUNCH();
   return ET_OK;
@@ -963,16 +963,17 @@ int MGSolver::pcg(MGHierarchy<T>& h, const double* b, double* x, double tol, int
   pcg_update_p_kernel<T><<<kRedBlocks, 256, 0, s>>>(n_dof, sh.scal, 0, partial, kRedBlocks, z, p_, x, 1);
   prof.end(s);
   ET_CHECK_LAUNCH();
-  // the fused q = A p, p.q path exists for the transformed-basis operator
-  const bool fused_pq = sh.tiled && g0.dim == 3 && get_wht() && wht_supported(g0, sizeof(double)) &&
-                        wht_partials(g0, sizeof(double), TM_YDOT) <= kRedBlocks;
-  const int n_pq_fused = fused_pq ? wht_partials(g0, sizeof(double), TM_YDOT) : 0;
+  // the fused q = A p, p.q path exists for the 2-D and the transformed-basis operator
+  const bool fused2 = g0.dim == 2 && op2d_partials(g0) <= kRedBlocks;
+  const bool fused_pq = fused2 || (sh.tiled && g0.dim == 3 && get_wht() && wht_supported(g0, sizeof(double)) &&
+                                   wht_partials(g0, sizeof(double), TM_YDOT) <= kRedBlocks);
+  const int n_pq_fused = fused2 ? op2d_partials(g0) : fused_pq ? wht_partials(g0, sizeof(double), TM_YDOT) : 0;
   // the last fine-grid sweep of the V-cycle (same operator) yields r.z, with r
   // in the V-cycle's precision (FP32 V-cycles: the copy of r they read)
-  const bool fused_rz = fused_pq && get_fused_rz() &&
-                        wht_supported(g0, sizeof(T)) && wht_partials(g0, sizeof(T), TM_JAC_ADD_DOT) <= kRedBlocks &&
-                        !sh.mfma && h.n_smooth > 0;
-  const int n_rz_fused = fused_rz ? wht_partials(g0, sizeof(T), TM_JAC_ADD_DOT) : kRedBlocks;
+  const bool fused_rz = fused_pq && get_fused_rz() && !sh.mfma && h.n_smooth > 0 &&
+                        (fused2 || (wht_supported(g0, sizeof(T)) &&
+                                    wht_partials(g0, sizeof(T), TM_JAC_ADD_DOT) <= kRedBlocks));
+  const int n_rz_fused = !fused_rz ? kRedBlocks : fused2 ? n_pq_fused : wht_partials(g0, sizeof(T), TM_JAC_ADD_DOT);
   int last = 0;
   auto read_ring = [&](int k, double* R, int* st) -> bool {
     ET_CHECK_HIP(hipEventSynchronize(ring_ev[k & 1]));
@@ -991,8 +992,12 @@ int MGSolver::pcg(MGHierarchy<T>& h, const double* b, double* x, double tol, int
     if (fused_pq) {
       // q = A p with p.q summed per workgroup inside the operator
       prof.begin(ET_PROF_MATVEC64, s);
-      ET_TRY(op0_wht_ydot<double>(g0, (int64_t)g0.ey * g0.ez, g0.ez, sh.wht, sh.Ed, sh.cons, p_, q, partial,
-                                  kRedBlocks, s));
+      if (fused2)
+        ET_TRY(op2d<double>(TM_YDOT, g0, sh.K0d, sh.Ed, sh.cons, p_, nullptr, nullptr, nullptr, 1.0, nullptr, q,
+                            nullptr, partial, s));
+      else
+        ET_TRY(op0_wht_ydot<double>(g0, (int64_t)g0.ey * g0.ez, g0.ez, sh.wht, sh.Ed, sh.cons, p_, q, partial,
+                                    kRedBlocks, s));
       prof.end(s);
       n_pq = n_pq_fused;
       prof.begin(ET_PROF_PCG_VEC, s);

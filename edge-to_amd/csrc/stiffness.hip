@@ -124,7 +124,7 @@ int matvec(const Grid& g, const T* K0, const T* E, const uint8_t* cons, const T*
   if (g.dim == 3)
     matvec_kernel<T, 3><<<grid, kBlock, 0, s>>>(g, K0, E, cons, u, y);
   else
-    matvec_kernel<T, 2><<<grid, kBlock, 0, s>>>(g, K0, E, cons, u, y);
+    return op2d<T>(TM_Y, g, K0, E, cons, u, nullptr, nullptr, nullptr, 1.0, nullptr, y, nullptr, nullptr, s);
   ET_CHECK_LAUNCH();
   return ET_OK;
 }

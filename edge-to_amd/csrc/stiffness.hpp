@@ -94,6 +94,12 @@ template <typename T>
 int op0_fine(int mode, const Grid& g, int64_t e_sx, int64_t e_sy, const T* K0, const WhtTable& tab, const T* E,
              const uint8_t* cons, const T* x, const T* b, const T* Dinv, const double* omega,
              double wscale, const T* xadd, T* y, hipStream_t s);
+// 2-D grids, every mode and any K0 (op_2d.hip); bdot and part only used by the modes with a dot
+// product, which write op2d_partials(g) per-workgroup sums to part.
+template <typename T>
+int op2d(int mode, const Grid& g, const T* K0, const T* E, const uint8_t* cons, const T* x, const T* b, const T* Dinv,
+         const double* omega, double wscale, const T* xadd, T* y, const T* bdot, double* part, hipStream_t s);
+int op2d_partials(const Grid& g);
 // whether op0_fine supports the fused zero-guess Jacobi mode (5) on this grid
 bool fine_jac0_supported(const Grid& g, size_t elem_bytes);
 bool fine_supported(const Grid& g, size_t elem_bytes);

@@ -92,6 +92,32 @@ def test_matvec_f64(nel, with_cons):
     assert rel(y.cpu().numpy(), ref) < 1e-12
 
 
+@pytest.mark.parametrize("nel", [(1, 1), (1, 40), (31, 7), (32, 8), (33, 1), (63, 17), (100, 3)])
+@pytest.mark.parametrize("dt", [torch.float64, torch.float32])
+def test_op2d_tile_edges(nel, dt):
+    """y = A x, b - A x and the Jacobi sweep of the 2-D operator at the edges of its 32 x 8 node
+    tiles, with constraints and with none.  Sums of 32 products and 4 terms: 40 ulps of the
+    largest value bound the difference (FP32: 5e-6)."""
+    L = _lib()
+    p = _problem(nel, seed=31)
+    s = "f64" if dt == torch.float64 else "f32"
+    tol = 1e-13 if dt == torch.float64 else 1e-5
+    b = np.random.default_rng(32).standard_normal(p["n_dof"])
+    x, bt, y = dev(p["u"], dt), dev(b, dt), torch.empty(p["n_dof"], dtype=dt, device="cuda")
+    for cons in (p["cons"], None):
+        ct = None if cons is None else dev(cons.astype(np.uint8))
+        A = oops.assemble(p["K0"], p["el"], p["E"], np.zeros(p["n_dof"], bool) if cons is None else cons, p["n_dof"])
+        Dinv = 1.0 / A.diagonal()
+        args = (2, L.nel_arg(nel), L.ptr(dev(p["K0"], dt)), L.ptr(dev(p["E"], dt)), L.ptr(ct), L.ptr(x))
+        r_ref = b - A @ p["u"]
+        L.call("et_matvec_" + s, *args, L.ptr(y), L.stream())
+        assert rel(y.cpu().numpy(), A @ p["u"]) < tol
+        L.call("et_residual_" + s, *args, L.ptr(bt), L.ptr(y), L.stream())
+        assert rel(y.cpu().numpy(), r_ref) < tol
+        L.call("et_jacobi_" + s, *args, L.ptr(bt), L.ptr(dev(Dinv, dt)), 0.6, L.ptr(y), L.stream())
+        assert rel(y.cpu().numpy(), p["u"] + 0.6 * Dinv * r_ref) < tol
+
+
 @pytest.mark.parametrize("nel", [(12, 8), (6, 4, 4)])
 def test_matvec_f32(nel):
     L = _lib()
