@@ -5,11 +5,13 @@
 //
 // CG (cupyx cg semantics): atol = tol |b|; rho = r.r, beta = rho / rho_old,
 // p = r + beta p, q = A p, alpha = rho / p.q, x += alpha p, r -= alpha q,
-// stop when |r| <= atol.  Every iteration is four launches (p update, operator,
-// x/r update with the p.q reduction finalised in-kernel, convergence check);
-// the state lives on the device and every kernel returns at once after the
-// stop, so the host enqueues chunks of iterations and reads the state once per
-// chunk.
+// stop when |r| <= atol.  A small system is bound by the chain of launches, so an iteration is as
+// few as possible: on an assembled operator two, the row pass (the test of the previous step,
+// p = r + beta p formed while it is gathered, q = A p, p.q) and the x / r update; on any other
+// operator four (p update with the test, operator, p.q, x / r update).  28 611 unknowns, 1.2 M
+// entries: 25 us per iteration in five launches, 12 us in two.  The state lives on the device
+// and every kernel returns at once after the stop, so the host enqueues chunks of iterations and
+// reads the state once per chunk.
 //
 // GMRES(m) (cupyx gmres semantics): each cycle forms r = b - A x, stops if
 // |r| <= atol, runs m Arnoldi steps with one classical Gram-Schmidt pass per
@@ -29,12 +31,46 @@
 
 namespace et {
 
+// State of the iterations.  Iteration k reads slot (k - 1) & 1 and writes slot k & 1 (the first reads
+// slot 1), so no kernel reads a slot that one of its own blocks writes.
+struct CgSlot {
+  double rho;
+  int stop, iters;
+};
 struct CgState {
-  double rho, rho_old, atol2, rr, pq;
-  int stop, iters, first;
+  CgSlot slot[2];
+  double atol2, bb;
+  // what the host reads: written by cg_report_kernel
+  double rr;
+  int stop, iters;
 };
 
-constexpr int kCgChunk = 8;
+// iterations enqueued between two reads of the state, at least and at most
+constexpr int kCgChunk = 8, kCgChunkMax = 64;
+
+// r (interleaved with the search direction, so that one gather fetches both)
+struct alignas(8) CgPair {
+  double r, p;
+};
+
+// partial sums of b.b and r.r; with rp also rp = {r, 0}
+__global__ __launch_bounds__(256) void cg_start_kernel(int64_t n, const double* __restrict__ b,
+                                                       const double* __restrict__ r, CgPair* __restrict__ rp,
+                                                       double* __restrict__ part_bb, double* __restrict__ part_rr) {
+  double sb = 0.0, sr = 0.0;
+  for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (int64_t)gridDim.x * blockDim.x) {
+    const double bv = b[t], rv = r[t];
+    sb += bv * bv;
+    sr += rv * rv;
+    if (rp != nullptr) rp[t] = CgPair{rv, 0.0};
+  }
+  sb = block_sum256(sb);
+  sr = block_sum256(sr);
+  if (threadIdx.x == 0) {
+    part_bb[blockIdx.x] = sb;
+    part_rr[blockIdx.x] = sr;
+  }
+}
 
 __global__ void cg_init_kernel(const double* __restrict__ part_bb, const double* __restrict__ part_rr, int nb,
                                double tol, CgState* st) {
@@ -47,32 +83,52 @@ __global__ void cg_init_kernel(const double* __restrict__ part_bb, const double*
   rr = block_sum256(rr);
   if (threadIdx.x == 0) {
     const double atol = tol * sqrt(bb);
+    st->bb = bb;
     st->atol2 = atol * atol;
-    st->rr = rr;
-    st->rho = rr;
-    st->rho_old = 0.0;
-    st->iters = 0;
-    st->first = 1;
     // |r| <= atol before any step stops at once (|b| = 0 is handled by the host)
-    st->stop = (bb == 0.0 || rr <= st->atol2) ? 1 : 0;
+    st->slot[1] = CgSlot{rr, bb == 0.0 || rr <= st->atol2 ? 1 : 0, 0};
+    st->rr = rr;
+    st->stop = st->slot[1].stop;
+    st->iters = 0;
   }
 }
 
-// p = r (first iteration) or p = r + (rho / rho_old) p
-__global__ __launch_bounds__(256) void cg_p_kernel(int64_t n, const CgState* __restrict__ st,
-                                                   const double* __restrict__ r, double* __restrict__ p) {
-  if (st->stop) return;
-  const bool first = st->first != 0;
-  const double beta = first ? 0.0 : st->rho / st->rho_old;
-  for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < n;
-       t += (int64_t)gridDim.x * blockDim.x)
-    p[t] = first ? r[t] : r[t] + beta * p[t];
+// The convergence test of step k - 1 and the start of step k, evaluated by every block from the same
+// partials in the same order; block 0 records it.  Returns whether step k runs; beta = rho / rho_old
+// (0 on the first step).
+__device__ __forceinline__ bool cg_begin(CgState* st, int k, const double* __restrict__ part_rr, int nb,
+                                         double& beta) {
+  const CgSlot prev = st->slot[(k + 1) & 1];
+  CgSlot cur = prev;
+  beta = 0.0;
+  if (k > 0 && !prev.stop) {
+    double rr = 0.0;
+    for (int t = threadIdx.x; t < nb; t += blockDim.x) rr += part_rr[t];
+    rr = block_sum256_all(rr);
+    cur.rho = rr;
+    cur.iters = k;
+    cur.stop = rr <= st->atol2 || !(rr == rr) ? 1 : 0;
+    beta = rr / prev.rho;
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) st->slot[k & 1] = cur;
+  return !cur.stop;
 }
 
-__global__ __launch_bounds__(256) void cg_pq_kernel(int64_t n, const CgState* __restrict__ st,
+// p = r (first step) or p = r + beta p
+__global__ __launch_bounds__(256) void cg_p_kernel(int64_t n, CgState* __restrict__ st, int k,
+                                                   const double* __restrict__ part_rr, int nb,
+                                                   const double* __restrict__ r, double* __restrict__ p) {
+  double beta;
+  if (!cg_begin(st, k, part_rr, nb, beta)) return;
+  for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < n;
+       t += (int64_t)gridDim.x * blockDim.x)
+    p[t] = k == 0 ? r[t] : r[t] + beta * p[t];
+}
+
+__global__ __launch_bounds__(256) void cg_pq_kernel(int64_t n, const CgState* __restrict__ st, int k,
                                                     const double* __restrict__ p, const double* __restrict__ q,
                                                     double* __restrict__ partial) {
-  if (st->stop) return;
+  if (st->slot[k & 1].stop) return;
   double s = 0.0;
   for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < n;
        t += (int64_t)gridDim.x * blockDim.x)
@@ -81,57 +137,130 @@ __global__ __launch_bounds__(256) void cg_pq_kernel(int64_t n, const CgState* __
   if (threadIdx.x == 0) partial[blockIdx.x] = s;
 }
 
+// Step k of an assembled operator up to p.q: p = r + beta p formed for every gathered entry and
+// stored for the own row, q = A p, per-block sums of p.q.  8 lanes per row as in the plain product
+// (lane j sums entries j, j + 8, ..., then a fixed tree), blocks striding over the rows.
+__global__ __launch_bounds__(256) void cg_csr_kernel(int64_t n, CgState* __restrict__ st, int k,
+                                                     const double* __restrict__ part_rr, int nb,
+                                                     const int* __restrict__ row_ptr, const int* __restrict__ cols,
+                                                     const double* __restrict__ vals,
+                                                     const CgPair* __restrict__ rp, double* __restrict__ p,
+                                                     double* __restrict__ q, double* __restrict__ part_pq) {
+  constexpr int NP = 6;
+  const int lane = threadIdx.x & 7;
+  // the first row's entries are on their way while the partials are summed
+  int64_t row = (int64_t)blockIdx.x * 32 + (threadIdx.x >> 3);
+  int a = 0, e = 0;
+  double pv[NP];
+  CgPair pg[NP], own{0.0, 0.0};
+  auto fetch = [&]() {
+    const int64_t rc = row < n ? row : n - 1;
+    a = row_ptr[rc];
+    e = row < n ? row_ptr[rc + 1] : a;
+    own = rp[rc];
+#pragma unroll
+    for (int u = 0; u < NP; ++u) {
+      const int t = a + lane + 8 * u;
+      const bool in = t < e;
+      pv[u] = in ? vals[t] : 0.0;
+      pg[u] = in ? rp[cols[t]] : CgPair{0.0, 0.0};
+    }
+  };
+  fetch();
+  double beta;
+  if (!cg_begin(st, k, part_rr, nb, beta)) return;
+  double dot = 0.0;
+  for (int64_t row0 = (int64_t)blockIdx.x * 32;;) {
+    double s = 0.0;
+#pragma unroll
+    for (int u = 0; u < NP; ++u)
+      if (a + lane + 8 * u < e) s += pv[u] * (k == 0 ? pg[u].r : pg[u].r + beta * pg[u].p);
+    for (int t = a + lane + 8 * NP; t < e; t += 8) {
+      const CgPair v = rp[cols[t]];
+      s += vals[t] * (k == 0 ? v.r : v.r + beta * v.p);
+    }
+    s += __shfl_xor(s, 4, 8);
+    s += __shfl_xor(s, 2, 8);
+    s += __shfl_xor(s, 1, 8);
+    if (row < n && lane == 0) {
+      const double pn = k == 0 ? own.r : own.r + beta * own.p;
+      p[row] = pn;
+      q[row] = s;
+      dot += pn * s;
+    }
+    row0 += (int64_t)gridDim.x * 32;
+    if (row0 >= n) break;
+    row = row0 + (threadIdx.x >> 3);
+    fetch();
+  }
+  dot = block_sum256(dot);
+  if (threadIdx.x == 0) part_pq[blockIdx.x] = dot;
+}
+
 // alpha = rho / p.q (every block sums the same partials in the same order);
-// x += alpha p, r -= alpha q, partial sums of r.r
-__global__ __launch_bounds__(256) void cg_xr_kernel(int64_t n, const CgState* __restrict__ st,
+// x += alpha p, r -= alpha q, partial sums of r.r.  PAIR: r lives in rp, which also takes p.
+template <bool PAIR>
+__global__ __launch_bounds__(256) void cg_xr_kernel(int64_t n, const CgState* __restrict__ st, int k,
                                                     const double* __restrict__ part_pq, int nb,
                                                     const double* __restrict__ p, const double* __restrict__ q,
                                                     double* __restrict__ x, double* __restrict__ r,
-                                                    double* __restrict__ part_rr) {
-  if (st->stop) return;
-  __shared__ double s_alpha;
+                                                    CgPair* __restrict__ rp, double* __restrict__ part_rr) {
+  // the first values are on their way while the partials are summed
+  int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t step = (int64_t)gridDim.x * blockDim.x, t0 = t < n ? t : n - 1;
+  double pv = p[t0], qv = q[t0], xv = x[t0], rv = PAIR ? rp[t0].r : r[t0];
+  if (st->slot[k & 1].stop) return;
   double pq = 0.0;
-  for (int t = threadIdx.x; t < nb; t += blockDim.x) pq += part_pq[t];
-  pq = block_sum256(pq);
-  if (threadIdx.x == 0) s_alpha = st->rho / pq;
-  __syncthreads();
-  const double alpha = s_alpha;
+  for (int u = threadIdx.x; u < nb; u += blockDim.x) pq += part_pq[u];
+  const double alpha = st->slot[k & 1].rho / block_sum256_all(pq);
   double s = 0.0;
-  for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < n;
-       t += (int64_t)gridDim.x * blockDim.x) {
-    x[t] += alpha * p[t];
-    const double rv = r[t] - alpha * q[t];
-    r[t] = rv;
+  while (t < n) {
+    x[t] = xv + alpha * pv;
+    rv -= alpha * qv;
+    if (PAIR)
+      rp[t] = CgPair{rv, pv};
+    else
+      r[t] = rv;
     s += rv * rv;
+    t += step;
+    if (t >= n) break;
+    pv = p[t];
+    qv = q[t];
+    xv = x[t];
+    rv = PAIR ? rp[t].r : r[t];
   }
   s = block_sum256(s);
   if (threadIdx.x == 0) part_rr[blockIdx.x] = s;
 }
 
-__global__ void cg_check_kernel(const double* __restrict__ part_rr, int nb, int maxiter, CgState* st) {
-  if (st->stop) return;
+// the test of the last enqueued step, k - 1, for the host (step k repeats it)
+__global__ void cg_report_kernel(const double* __restrict__ part_rr, int nb, int k, CgState* st) {
+  const CgSlot prev = st->slot[(k + 1) & 1];
   double rr = 0.0;
   for (int t = threadIdx.x; t < nb; t += blockDim.x) rr += part_rr[t];
   rr = block_sum256(rr);
-  if (threadIdx.x == 0) {
-    st->iters += 1;
-    st->first = 0;
-    st->rr = rr;
-    st->rho_old = st->rho;
-    st->rho = rr;
-    if (rr <= st->atol2 || st->iters >= maxiter || !(rr == rr)) st->stop = 1;
-  }
+  if (threadIdx.x != 0) return;
+  st->rr = prev.stop ? prev.rho : rr;
+  st->iters = prev.stop ? prev.iters : k;
+  st->stop = prev.stop || rr <= st->atol2 || !(rr == rr) ? 1 : 0;
 }
 
 namespace {
 inline int64_t up256(int64_t bytes) { return (bytes + 255) / 256 * 256; }
 }  // namespace
 
+// without the interleaved copy of p: assembled operators then take separate passes
+static int64_t cg_work_min(int64_t n) {
+  const int64_t vec = up256(n * (int64_t)sizeof(double));
+  const int64_t red = up256(kRedBlocks * (int64_t)sizeof(double));
+  return 3 * vec + 2 * red + up256(sizeof(CgState)) + up256(4 * sizeof(double));
+}
+
 int64_t krylov_work_size(int64_t n, int restart) {
   const int64_t vec = up256(n * (int64_t)sizeof(double));
   const int64_t red = up256(kRedBlocks * (int64_t)sizeof(double));
-  if (restart <= 0)  // CG: r, p, q, two reduction buffers, state + scalars
-    return 3 * vec + 2 * red + up256(sizeof(CgState)) + up256(4 * sizeof(double));
+  if (restart <= 0)  // CG: r, p, q, two reduction buffers, state + scalars; p interleaved with r
+    return cg_work_min(n) + vec;
   // GMRES: V (restart columns), u, r, reductions, H and scalars
   return up256((int64_t)restart * n * (int64_t)sizeof(double)) + 2 * vec +
          up256((int64_t)(restart + 2) * kRedBlocks * (int64_t)sizeof(double)) +
@@ -184,58 +313,69 @@ int cg_solve_op(const KrylovOp& op, const double* b, double* x, double tol, int 
                 int64_t work_bytes, int* iters, double* residual, hipStream_t s) {
   const int64_t n = op.n;
   ET_REQUIRE(maxiter >= 1, "cg: maxiter must be >= 1");
-  ET_REQUIRE(work_bytes >= krylov_work_size(n, 0), "cg: work buffer too small");
+  ET_REQUIRE(work_bytes >= cg_work_min(n), "cg: work buffer too small");
+  const bool pair = op.row_ptr != nullptr && work_bytes >= krylov_work_size(n, 0);
   Carve c{static_cast<char*>(work)};
-  double* r = c.take<double>(n);
   double* p = c.take<double>(n);
   double* q = c.take<double>(n);
   double* part_a = c.take<double>(kRedBlocks);
   double* part_b = c.take<double>(kRedBlocks);
   CgState* st = c.take<CgState>(1);
-  double* scal = c.take<double>(4);  // [0] |b|^2, [1] |b - A x|^2 after the loop
-  {
-    // |b| = 0: x = b = 0 at once, as cupyx returns
-    ET_TRY(dot(n, b, b, part_a, scal, s));
-    double bb0 = 0.0;
-    ET_CHECK_HIP(hipMemcpyAsync(&bb0, scal, sizeof(double), hipMemcpyDeviceToHost, s));
-    ET_CHECK_HIP(hipStreamSynchronize(s));
-    if (bb0 == 0.0) {
-      ET_CHECK_HIP(hipMemsetAsync(x, 0, n * sizeof(double), s));
-      if (iters) *iters = 0;
-      if (residual) *residual = 0.0;
-      return ET_OK;
-    }
-  }
+  double* scal = c.take<double>(4);  // [1] |b - A x|^2 after the loop
+  double* r = c.take<double>(pair ? 2 * n : n);
+  CgPair* rp = pair ? reinterpret_cast<CgPair*>(r) : nullptr;
+  // one value per thread up to kRedBlocks blocks of the vector passes; each block of the next pass
+  // sums one partial per block of this one
+  const int nb = (int)std::min<int64_t>(kRedBlocks, (n + 255) / 256);
+  const int nbr = (int)std::min<int64_t>(kRedBlocks, (n + 31) / 32);  // blocks of the row pass
+  const int nb_pq = pair ? nbr : nb;
   // r = b - A x, |b|^2, |r|^2
-  ET_TRY(op.apply(1, x, b, r, s));
-  ET_TRY(dot_partials(n, b, b, part_a, s));
-  ET_TRY(dot_partials(n, r, r, part_b, s));
-  cg_init_kernel<<<1, 256, 0, s>>>(part_a, part_b, kRedBlocks, tol, st);
+  ET_TRY(op.apply(1, x, b, pair ? p : r, s));
+  cg_start_kernel<<<nb, 256, 0, s>>>(n, b, pair ? p : r, rp, part_a, part_b);
+  cg_init_kernel<<<1, 256, 0, s>>>(part_a, part_b, nb, tol, st);
   ET_CHECK_LAUNCH();
   CgState h{};
-  for (int done = 0; done < maxiter;) {
-    const int chunk = std::min(kCgChunk, maxiter - done);
-    for (int k = 0; k < chunk; ++k) {
-      cg_p_kernel<<<kRedBlocks, 256, 0, s>>>(n, st, r, p);
-      ET_TRY(op.apply(0, p, nullptr, q, s));
-      cg_pq_kernel<<<kRedBlocks, 256, 0, s>>>(n, st, p, q, part_a);
-      cg_xr_kernel<<<kRedBlocks, 256, 0, s>>>(n, st, part_a, kRedBlocks, p, q, x, r, part_b);
-      cg_check_kernel<<<1, 256, 0, s>>>(part_b, kRedBlocks, maxiter, st);
+  double rr0 = 0.0;
+  int chunk = kCgChunk;
+  for (int done = 0;;) {
+    const int end = done + std::min(chunk, maxiter - done);
+    for (int k = done; k < end; ++k) {
+      if (pair) {
+        cg_csr_kernel<<<nbr, 256, 0, s>>>(n, st, k, part_b, nb, op.row_ptr, op.cols, op.vals, rp, p, q, part_a);
+        cg_xr_kernel<true><<<nb, 256, 0, s>>>(n, st, k, part_a, nb_pq, p, q, x, nullptr, rp, part_b);
+      } else {
+        cg_p_kernel<<<nb, 256, 0, s>>>(n, st, k, part_b, nb, r, p);
+        ET_TRY(op.apply(0, p, nullptr, q, s));
+        cg_pq_kernel<<<nb, 256, 0, s>>>(n, st, k, p, q, part_a);
+        cg_xr_kernel<false><<<nb, 256, 0, s>>>(n, st, k, part_a, nb_pq, p, q, x, r, nullptr, part_b);
+      }
     }
+    done = end;
+    cg_report_kernel<<<1, 256, 0, s>>>(part_b, nb, done, st);
     ET_CHECK_LAUNCH();
-    done += chunk;
     ET_CHECK_HIP(hipMemcpyAsync(&h, st, sizeof(CgState), hipMemcpyDeviceToHost, s));
     ET_CHECK_HIP(hipStreamSynchronize(s));
-    if (h.stop) break;
+    if (h.stop || done >= maxiter) break;
+    // Each read drains the queue (about 20 us, two steps), and steps enqueued past the stop are empty
+    // launches: half of the steps that the mean rate so far leaves, within the limits.
+    if (rr0 == 0.0) rr0 = h.rr;
+    const double rate = std::log(rr0 / h.rr), left = std::log(h.rr / h.atol2);
+    const double est = rate > 0.0 ? left / rate * done / 2 : kCgChunkMax;
+    chunk = (int)std::fmin(std::fmax(est, (double)kCgChunk), (double)kCgChunkMax);
   }
-  ET_CHECK_HIP(hipMemcpyAsync(&h, st, sizeof(CgState), hipMemcpyDeviceToHost, s));
+  if (h.bb == 0.0) {
+    // |b| = 0: x = b = 0 at once, as cupyx returns
+    ET_CHECK_HIP(hipMemsetAsync(x, 0, n * sizeof(double), s));
+    if (iters) *iters = 0;
+    if (residual) *residual = 0.0;
+    return ET_OK;
+  }
   // the reported residual is the true one, |b - A x| / |b| (solvers/_gpu.py:43)
-  ET_TRY(dot(n, b, b, part_a, scal, s));
-  ET_TRY(residual_norm(op, b, x, r, part_b, scal + 1, s));
-  double tail[2];
-  ET_CHECK_HIP(hipMemcpyAsync(tail, scal, sizeof(tail), hipMemcpyDeviceToHost, s));
+  ET_TRY(residual_norm(op, b, x, q, part_b, scal + 1, s));
+  double rr = 0.0;
+  ET_CHECK_HIP(hipMemcpyAsync(&rr, scal + 1, sizeof(double), hipMemcpyDeviceToHost, s));
   ET_CHECK_HIP(hipStreamSynchronize(s));
-  const double bb = tail[0], rr = tail[1];
+  const double bb = h.bb;
   if (iters) *iters = h.iters;
   if (residual) *residual = bb > 0.0 ? std::sqrt(rr / bb) : 0.0;
   if (!(rr == rr)) {

@@ -182,6 +182,9 @@ int64_t krylov_work_size(int64_t n, int restart);
 struct KrylovOp {
   int64_t n = 0;
   std::function<int(int mode, const double* x, const double* b, double* y, hipStream_t s)> apply;
+  // set when the operator is a CSR matrix (CG then fuses its passes into the product)
+  const int *row_ptr = nullptr, *cols = nullptr;
+  const double* vals = nullptr;
 };
 // general (unstructured) meshes (unstructured.hip)
 int umesh_star(int64_t n_nodes, int64_t n_el, const int* elem_ptr, const int* elem_nodes, int* star_ptr, int* star,

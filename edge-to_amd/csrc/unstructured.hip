@@ -593,6 +593,9 @@ int uassemble(const et_umesh* m, const double* E, const uint8_t* cons, const int
 KrylovOp csr_op(int64_t n_rows, const int* row_ptr, const int* cols, const double* vals) {
   KrylovOp op;
   op.n = n_rows;
+  op.row_ptr = row_ptr;
+  op.cols = cols;
+  op.vals = vals;
   op.apply = [=](int mode, const double* x, const double* b, double* y, hipStream_t s) {
     return csr_spmv(n_rows, row_ptr, cols, vals, x, y, s, mode, b);
   };

@@ -316,3 +316,43 @@ def test_simp_on_tet_mesh_matches_oracle_loop():
         comps.append(c)
     got = np.asarray(hist["comp_history"], dtype=float)
     assert rel(got, np.array(comps)) < 1e-7, (got, comps)
+
+
+@pytest.mark.parametrize("n,per_row", [(1, 1), (31, 9), (33, 33), (700, 120), (40000, 5)])
+def test_csr_cg_steps(n, per_row):
+    """et_csr_cg_f64 on random sparse SPD systems (rows longer than the entries fetched ahead, more
+    rows than one sweep of the blocks): iterates after few steps and converged solves, with the
+    full workspace and with one vector less (separate passes instead of the fused row pass)."""
+    import scipy.sparse as sps
+    from oracle import krylov
+    import ctypes
+    from edgeto_amd import _lib as L
+    rng = np.random.default_rng(n)
+    R = sps.random(n, n, density=min(1.0, per_row / n), random_state=rng, format="csr")
+    R = R + R.T
+    A = (R + sps.diags(np.abs(R).sum(1).A1 + 1.0)).tocsr()
+    A.sort_indices()
+    b = rng.standard_normal(n)
+    rp, cols, vals = (torch.tensor(v, device="cuda") for v in
+                      (A.indptr.astype(np.int32), A.indices.astype(np.int32), A.data))
+    bt = torch.tensor(b, device="cuda")
+    full = int(L.lib().et_krylov_work_size(n, 0))
+    less = full - (n * 8 + 255) // 256 * 256
+    for size in (full, less):
+        work = torch.empty(full // 8 + 1, dtype=torch.float64, device="cuda")
+        for maxiter, tol in ((3, 0.0), (500, 1e-11)):
+            x = torch.zeros(n, dtype=torch.float64, device="cuda")
+            it, res = ctypes.c_int(0), ctypes.c_double(0.0)
+            st = L.lib().et_csr_cg_f64(n, L.i32(rp), L.i32(cols), L.f64(vals), L.f64(bt), L.f64(x), tol, maxiter,
+                                       L.f64(work), size, ctypes.byref(it), ctypes.byref(res), L.stream())
+            ref, steps = krylov.cg(lambda v: A @ v, b, tol=tol, maxiter=maxiter)
+            assert st in (L.ET_OK, L.ET_ENOCONV)
+            if tol > 0.0:
+                assert res.value <= 2e-11 and abs(it.value - steps) <= 1
+            elif n > 3:
+                assert it.value == maxiter
+            # a few steps on well-conditioned systems: rounding grows little
+            assert np.linalg.norm(x.cpu().numpy() - ref) <= 1e-9 * np.linalg.norm(ref)
+    st = L.lib().et_csr_cg_f64(n, L.i32(rp), L.i32(cols), L.f64(vals), L.f64(bt), L.f64(x), 1e-9, 5,
+                               L.f64(work), less - 256, ctypes.byref(it), ctypes.byref(res), L.stream())
+    assert st == L.ET_EINVAL
