@@ -399,6 +399,33 @@ def test_oc_update(n, seed, scale):
     assert rel(out.cpu().numpy(), ref0) < 1e-14
 
 
+@pytest.mark.parametrize("n", [1, 63, 1024, 1025, 5121, 8193, 10240, 10241, 270000])
+def test_oc_update_forms(n):
+    """The one-workgroup and the multi-pass bisection at the edges of their sizes, with one measure
+    and with a measure per element: the oracle's step count and design (1e-14), infinite and NaN
+    sensitivities included (an infinite quotient is clipped to the upper limit, NaN counts as 0)."""
+    L = _lib()
+    rng = np.random.default_rng(n)
+    x = rng.uniform(0.01, 1.0, n)
+    dc = -rng.uniform(0.0, 2.0, n) * rng.uniform(0, 1, n) ** 3
+    if n > 4:
+        dc[1], dc[2] = -np.inf, np.nan
+    mat = otop.SingleMaterial(void=1e-9, penalty=3.0, volume_fraction=0.45)
+    work = torch.empty(int(L.lib().et_oc_work_size(n)) // 8 + 1, dtype=torch.float64, device="cuda")
+    out, st = torch.empty(n, dtype=torch.float64, device="cuda"), ctypes.c_int(0)
+    for A in (1.0, rng.uniform(0.5, 1.5, n)):
+        vol = float(np.sum(A * np.ones(n)))
+        ref, steps = otop.oc_update(x, dc, A, vol, 0.45, 0.2, mat)
+        if np.ndim(A):
+            L.call("et_oc_update_elem_f64", n, L.f64(dev(x)), L.f64(dev(dc)), L.f64(dev(A)), vol, 0.45, 0.2,
+                   L.f64(out), L.f64(work), ctypes.byref(st), L.stream())
+        else:
+            L.call("et_oc_update_f64", n, L.f64(dev(x)), L.f64(dev(dc)), A, vol, 0.45, 0.2, L.f64(out),
+                   L.f64(work), ctypes.byref(st), L.stream())
+        assert st.value == steps
+        assert rel(out.cpu().numpy(), ref) < 1e-14
+
+
 @pytest.mark.parametrize("nel", [(8, 4), (12, 6), (6, 4, 4), (8, 4, 6), (4, 2, 2)])
 def test_galerkin_from_elements(nel):
     """Element-based first coarse operator equals R A_hat R^T (with constraints)."""
