@@ -38,12 +38,13 @@ namespace {
 // structure (k0_structure); K0 arrives in device memory here, so it is read
 // back first (this synchronises the stream), and its transformed-basis table is
 // built from the same copy.  *fine = tab when the fine-grid kernels apply, else
-// null (2-D grids always use the general kernel).
+// null (2-D grids always use the general kernel).  single: one operator call, which
+// on a small grid takes the tile operator with K0 as it is and needs no check.
 template <typename T>
 static int fine_allowed(const Grid& g, const T* K0, hipStream_t stream, et::WhtTable* tab,
-                        const et::WhtTable** fine) {
+                        const et::WhtTable** fine, bool single = true) {
   *fine = nullptr;
-  if (g.dim != 3) return ET_OK;
+  if (g.dim != 3 || (single && et::tile3_active(g, sizeof(T)))) return ET_OK;
   T h[576];
   ET_CHECK_HIP(hipMemcpyAsync(h, K0, sizeof(h), hipMemcpyDeviceToHost, stream));
   ET_CHECK_HIP(hipStreamSynchronize(stream));
@@ -96,6 +97,11 @@ int et_tune_set(int param, int value) {
     if (param == ET_TUNE_ROW_STENCIL_NODES) {
       ET_REQUIRE(value >= 0, "et_tune_set: node count must be >= 0");
       et::set_row_stencil_nodes(value);
+      return ET_OK;
+    }
+    if (param == ET_TUNE_TILE3_NODES) {
+      ET_REQUIRE(value >= 0, "et_tune_set: node count must be >= 0");
+      et::set_tile3_nodes(value);
       return ET_OK;
     }
     ET_REQUIRE(value >= 0 && value <= 1024, "et_tune_set: value out of range");
@@ -159,6 +165,7 @@ int et_tune_get(int param) {
     return et::get_wht_threads(param == ET_TUNE_WHT_THREADS_F64);
   if (param == ET_TUNE_WHT_WGS) return et::get_wht_wgs();
   if (param == ET_TUNE_FILTER_ROWS) return et::get_stencil_rows();
+  if (param == ET_TUNE_TILE3_NODES) return (int)et::get_tile3_nodes();
   return -1;
 }
 
@@ -455,7 +462,7 @@ int et_cg_f64(int dim, const int* nel, const double* K0, const double* E, const 
     ET_REQUIRE(std::isfinite(tol) && tol >= 0, "et_cg_f64: tol must be finite and >= 0");
     et::WhtTable tab;
     const et::WhtTable* fine = nullptr;
-    ET_TRY(fine_allowed(g, K0, stream, &tab, &fine));
+    ET_TRY(fine_allowed(g, K0, stream, &tab, &fine, false));
     return et::cg_solve(g, K0, E, cons, fine, b, x, tol, maxiter, work, work_bytes, iters, residual, stream);
   })
 }
@@ -471,7 +478,7 @@ int et_gmres_f64(int dim, const int* nel, const double* K0, const double* E, con
     ET_REQUIRE(std::isfinite(tol) && tol >= 0, "et_gmres_f64: tol must be finite and >= 0");
     et::WhtTable tab;
     const et::WhtTable* fine = nullptr;
-    ET_TRY(fine_allowed(g, K0, stream, &tab, &fine));
+    ET_TRY(fine_allowed(g, K0, stream, &tab, &fine, false));
     return et::gmres_solve(g, K0, E, cons, fine, b, x, tol, restart, maxiter, work, work_bytes, iters, residual,
                            stream);
   })

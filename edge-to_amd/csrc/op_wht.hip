@@ -66,17 +66,6 @@ struct WCfg {
   static_assert(slots >= 1 && estage >= 1 && nodes >= 1, "tile smaller than the workgroup");
 };
 
-// structural non-zeros of G[M][c][d] (M = 1..7)
-__host__ __device__ constexpr bool wht_nz(int M, int c, int d) {
-  if (M == 0) return false;
-  if (c == d) return true;
-  if (M == 7) return false;
-  const int pair = (1 << c) | (1 << d);
-  const int bits = __builtin_popcount(M);
-  // single-bit M: zero on the pair of the other two axes; two-bit M: zero on its own pair
-  return bits == 1 ? (pair & M) != 0 : pair != M;
-}
-
 __host__ inline int wht_tc(const Grid& g, int ns) { return g.ez <= 64 ? ns : ns / 2; }
 
 __host__ inline size_t wht_lds_values(const Grid& g, int ns) {

@@ -449,6 +449,12 @@ static int op_launch(const MGLevel<T>& L, const MGShared& sh, int mode, const T*
     sh.prof->end(s);
     return st;
   }
+  if (L.level == 0 && sh.tiled && tile3_faster(g, sizeof(T))) {
+    const int st = op_tile3<T>(mode, g, sh.K0<T>(), &sh.wht, sh.E<T>(), sh.cons, x, b, L.Dinv,
+                               omega, wscale, xadd, y, nullptr, nullptr, s);
+    sh.prof->end(s);
+    return st;
+  }
   if (L.level == 0 && sh.tiled) {
     const int st = op0_fine<T>(mode, g, (int64_t)g.ey * g.ez, g.ez, sh.K0<T>(), sh.wht, sh.E<T>(), sh.cons,
                                 x, b, L.Dinv, omega, wscale, xadd, y, s);
@@ -516,7 +522,8 @@ int MGHierarchy<T>::vcycle(int l, MGShared& sh, hipStream_t s, bool x0_ready) {
     int it = 1;
     // both precisions (the FP64 sweeps run on 8-slice tiles, where the fused pass is faster)
     if (l == 0 && n_smooth >= 2 &&
-        (L.g.dim == 2 || (sh.tiled && !(sizeof(T) == 4 && sh.mfma) && fine_jac0_supported(L.g, sizeof(T))))) {
+        (L.g.dim == 2 || (!(sizeof(T) == 4 && sh.mfma) &&
+                          sh.tiled && (tile3_faster(L.g, sizeof(T)) || fine_jac0_supported(L.g, sizeof(T)))))) {
       // x0 = w D^-1 b and the first sweep from it in one pass
       ET_TRY(op_launch<T>(L, sh, OP_JAC0, nullptr, L.b, om, ws, nullptr, L.t, s));
       std::swap(L.x, L.t);
@@ -561,6 +568,9 @@ int MGHierarchy<T>::vcycle(int l, MGShared& sh, hipStream_t s, bool x0_ready) {
             L.g.dim == 2
                 ? op2d<T>(TM_JAC_ADD_DOT, L.g, sh.K0<T>(), sh.E<T>(), sh.cons, L.e, L.r, L.Dinv, om, ws, L.x, L.t,
                           L.b, sh.dot_part, s)
+            : sh.tiled && tile3_faster(L.g, sizeof(T))
+                ? op_tile3<T>(TM_JAC_ADD_DOT, L.g, sh.K0<T>(), &sh.wht, sh.E<T>(), sh.cons, L.e,
+                              L.r, L.Dinv, om, ws, L.x, L.t, L.b, sh.dot_part, s)
                 : op0_wht_jac_add_dot<T>(L.g, (int64_t)L.g.ey * L.g.ez, L.g.ez, sh.wht, sh.E<T>(), sh.cons, L.e,
                                          L.r, L.Dinv, om, ws, L.x, L.t, L.b, sh.dot_part, kRedBlocks, s);
         sh.prof->end(s);
@@ -616,6 +626,8 @@ template <typename T>
 int level0_op(int mode, const Grid& g, const T* K0, const T* E, const uint8_t* cons, const T* x,
               const T* b, const T* Dinv, const double* omega, double wscale, const T* xadd, T* y,
               hipStream_t s, const WhtTable* fine) {
+  if (fine == nullptr ? tile3_active(g, sizeof(T)) : tile3_faster(g, sizeof(T)))
+    return op_tile3<T>(mode, g, K0, fine, E, cons, x, b, Dinv, omega, wscale, xadd, y, nullptr, nullptr, s);
   if (g.dim == 3 && fine != nullptr && fine_supported(g, sizeof(T)))
     return op0_fine<T>(mode, g, (int64_t)g.ey * g.ez, g.ez, K0, *fine, E, cons, x, b, Dinv, omega, wscale, xadd, y,
                        s);
@@ -869,6 +881,12 @@ int MGSolver::apply_A64(const double* x, double* y, int mode, const double* b) {
   hipStream_t s = stream;
   const unsigned grid = grid_for(g0.n_nodes());
   prof.begin(ET_PROF_MATVEC64, s);
+  if (sh.tiled && tile3_faster(g0, sizeof(double))) {
+    const int st = op_tile3<double>(mode, g0, sh.K0d, &sh.wht, sh.Ed, sh.cons, x, b, nullptr,
+                                    nullptr, 1.0, nullptr, y, nullptr, nullptr, s);
+    prof.end(s);
+    return st;
+  }
   if (sh.tiled) {
     const int st = op0_fine<double>(mode, g0, (int64_t)g0.ey * g0.ez, g0.ez, sh.K0d, sh.wht, sh.Ed, sh.cons,
                                      x, b, nullptr, sh.scal, 1.0, nullptr, y, s);
@@ -965,15 +983,25 @@ int MGSolver::pcg(MGHierarchy<T>& h, const double* b, double* x, double tol, int
   ET_CHECK_LAUNCH();
   // the fused q = A p, p.q path exists for the 2-D and the transformed-basis operator
   const bool fused2 = g0.dim == 2 && op2d_partials(g0) <= kRedBlocks;
-  const bool fused_pq = fused2 || (sh.tiled && g0.dim == 3 && get_wht() && wht_supported(g0, sizeof(double)) &&
-                                   wht_partials(g0, sizeof(double), TM_YDOT) <= kRedBlocks);
-  const int n_pq_fused = fused2 ? op2d_partials(g0) : fused_pq ? wht_partials(g0, sizeof(double), TM_YDOT) : 0;
+  const bool tile3 = sh.tiled && tile3_faster(g0, sizeof(double));
+  const bool fused3 = tile3 && tile3_partials(g0, sizeof(double)) <= kRedBlocks;
+  const bool fused_pq = fused2 || fused3 ||
+                        (sh.tiled && g0.dim == 3 && get_wht() && wht_supported(g0, sizeof(double)) &&
+                         !tile3 && wht_partials(g0, sizeof(double), TM_YDOT) <= kRedBlocks);
+  const int n_pq_fused = fused2 ? op2d_partials(g0)
+                         : fused3 ? tile3_partials(g0, sizeof(double))
+                         : fused_pq ? wht_partials(g0, sizeof(double), TM_YDOT) : 0;
   // the last fine-grid sweep of the V-cycle (same operator) yields r.z, with r
   // in the V-cycle's precision (FP32 V-cycles: the copy of r they read)
   const bool fused_rz = fused_pq && get_fused_rz() && !sh.mfma && h.n_smooth > 0 &&
-                        (fused2 || (wht_supported(g0, sizeof(T)) &&
-                                    wht_partials(g0, sizeof(T), TM_JAC_ADD_DOT) <= kRedBlocks));
-  const int n_rz_fused = !fused_rz ? kRedBlocks : fused2 ? n_pq_fused : wht_partials(g0, sizeof(T), TM_JAC_ADD_DOT);
+                        (fused2 ||
+                         (sh.tiled && tile3_faster(g0, sizeof(T))
+                              ? tile3_partials(g0, sizeof(T)) <= kRedBlocks
+                              : wht_supported(g0, sizeof(T)) && wht_partials(g0, sizeof(T), TM_JAC_ADD_DOT) <= kRedBlocks));
+  const int n_rz_fused = !fused_rz ? kRedBlocks
+                         : fused2 ? n_pq_fused
+                         : tile3_faster(g0, sizeof(T)) ? tile3_partials(g0, sizeof(T))
+                                                       : wht_partials(g0, sizeof(T), TM_JAC_ADD_DOT);
   int last = 0;
   auto read_ring = [&](int k, double* R, int* st) -> bool {
     ET_CHECK_HIP(hipEventSynchronize(ring_ev[k & 1]));
@@ -995,6 +1023,9 @@ int MGSolver::pcg(MGHierarchy<T>& h, const double* b, double* x, double tol, int
       if (fused2)
         ET_TRY(op2d<double>(TM_YDOT, g0, sh.K0d, sh.Ed, sh.cons, p_, nullptr, nullptr, nullptr, 1.0, nullptr, q,
                             nullptr, partial, s));
+      else if (fused3)
+        ET_TRY(op_tile3<double>(TM_YDOT, g0, sh.K0d, &sh.wht, sh.Ed, sh.cons, p_, nullptr, nullptr,
+                                nullptr, 1.0, nullptr, q, nullptr, partial, s));
       else
         ET_TRY(op0_wht_ydot<double>(g0, (int64_t)g0.ey * g0.ez, g0.ez, sh.wht, sh.Ed, sh.cons, p_, q, partial,
                                     kRedBlocks, s));

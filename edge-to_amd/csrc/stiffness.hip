@@ -118,6 +118,8 @@ template <typename T>
 int matvec(const Grid& g, const T* K0, const T* E, const uint8_t* cons, const T* u, T* y,
            hipStream_t s, const WhtTable* fine) {
   const unsigned grid = grid_for(g.n_nodes());
+  if (fine == nullptr ? tile3_active(g, sizeof(T)) : tile3_faster(g, sizeof(T)))
+    return op_tile3<T>(TM_Y, g, K0, fine, E, cons, u, nullptr, nullptr, nullptr, 1.0, nullptr, y, nullptr, nullptr, s);
   if (g.dim == 3 && fine != nullptr && fine_supported(g, sizeof(T)))
     return op0_fine<T>(0, g, (int64_t)g.ey * g.ez, g.ez, K0, *fine, E, cons, u, nullptr, nullptr, nullptr,
                         1.0, nullptr, y, s);

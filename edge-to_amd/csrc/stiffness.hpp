@@ -33,6 +33,16 @@ struct WhtTable {
   double g[48];
 };
 void wht_table(const double* K0_host, WhtTable* t);
+// structural non-zeros of G[M][c][d] (M = 1..7)
+__host__ __device__ constexpr bool wht_nz(int M, int c, int d) {
+  if (M == 0) return false;
+  if (c == d) return true;
+  if (M == 7) return false;
+  const int pair = (1 << c) | (1 << d);
+  const int bits = __builtin_popcount(M);
+  // single-bit M: zero on the pair of the other two axes; two-bit M: zero on its own pair
+  return bits == 1 ? (pair & M) != 0 : pair != M;
+}
 
 template <typename T>
 int matvec(const Grid& g, const T* K0, const T* E, const uint8_t* cons, const T* u, T* y,
@@ -94,6 +104,17 @@ template <typename T>
 int op0_fine(int mode, const Grid& g, int64_t e_sx, int64_t e_sy, const T* K0, const WhtTable& tab, const T* E,
              const uint8_t* cons, const T* x, const T* b, const T* Dinv, const double* omega,
              double wscale, const T* xadd, T* y, hipStream_t s);
+// Small 3-D grids (at most 64 elements in z), every mode; tab: the transformed basis, null: any K0
+// (op_tile3.hip).  dotv and part: the modes with a dot product, which write tile3_partials sums.
+template <typename T>
+int op_tile3(int mode, const Grid& g, const T* K0, const WhtTable* tab, const T* E, const uint8_t* cons, const T* x,
+             const T* b, const T* Dinv, const double* omega, double wscale, const T* xadd, T* y, const T* dotv,
+             double* part, hipStream_t s);
+bool tile3_active(const Grid& g, size_t elem_bytes);  // it takes single calls, whose K0 is not known
+bool tile3_faster(const Grid& g, size_t elem_bytes);  // and beats the marching operator with its table
+void set_tile3_nodes(int64_t n);
+int64_t get_tile3_nodes();
+int tile3_partials(const Grid& g, size_t elem_bytes);
 // 2-D grids, every mode and any K0 (op_2d.hip); bdot and part only used by the modes with a dot
 // product, which write op2d_partials(g) per-workgroup sums to part.
 template <typename T>

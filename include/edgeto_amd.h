@@ -81,7 +81,10 @@ const char* et_version(void);
  *   V-cycle's precision (FP32 V-cycles: their FP32 copy of r); no separate pass over r
  *   and z.  0 = separate reduction with r in FP64.  Read by each solve.
  * ET_TUNE_FILTER_ROWS: y rows of the 3-D filter stencils' tiles (64 elements along z each):
- *   8 (default, 512 threads) or 4 (256 threads). */
+ *   8 (default, 512 threads) or 4 (256 threads).
+ * ET_TUNE_TILE3_NODES: 3-D fine grids with at most this many nodes (and at most 64 elements
+ *   in z) apply their operator on one-shot tiles instead of marching, while ET_TUNE_WHT is on;
+ *   0 = never. */
 enum {
   ET_TUNE_TILED_JC = 0,
   ET_TUNE_MFMA_JC = 1,
@@ -100,7 +103,8 @@ enum {
   ET_TUNE_FUSED_RZ = 14,
   ET_TUNE_WHT_SLICES_F32 = 15,
   ET_TUNE_WHT_SLICES_F64 = 16,
-  ET_TUNE_FILTER_ROWS = 17
+  ET_TUNE_FILTER_ROWS = 17,
+  ET_TUNE_TILE3_NODES = 18
 };
 int et_tune_set(int param, int value);
 int et_tune_get(int param);

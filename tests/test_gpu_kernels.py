@@ -695,3 +695,53 @@ def test_simp_adjoint_fused(nel, rmin, spacing, k0):
         assert err < 1e-12, (fl, err)
     if k0 == "rotated":
         assert not flags.value & 4  # no transformed-basis structure: the full product ran
+
+
+@pytest.fixture
+def no_tile3():
+    """Single operator calls on small grids through the marching and node-gather kernels."""
+    L = _lib()
+    old = L.lib().et_tune_get(18)
+    L.call("et_tune_set", 18, 0)
+    yield
+    L.call("et_tune_set", 18, old)
+
+
+@pytest.mark.parametrize("nel,prec,variant", [((6, 4, 4), "f64", "wht"), ((9, 5, 17), "f32", "wht"),
+                                              ((13, 6, 70), "f64", "wht"), ((20, 9, 40), "f32", "wht")])
+def test_marching_operator_on_small_grids(no_tile3, nel, prec, variant):
+    test_residual_and_jacobi(nel, prec, variant)
+
+
+@pytest.mark.parametrize("k0", ["iso", "rotated", "unsymmetric"])
+@pytest.mark.parametrize("nel", [(1, 1, 1), (2, 9, 63), (7, 6, 31), (12, 11, 20), (40, 3, 48)])
+@pytest.mark.parametrize("dt", [torch.float64, torch.float32])
+def test_op_tile3(nel, dt, k0):
+    """y = A x, b - A x and the Jacobi sweep of the tile operator for any element matrix (one to many
+    tiles, several columns per wavefront, the tallest grid), with constraints and with none, against
+    the assembled operator.  A row has at most 192 products: 1e-13 (FP32 1e-5) of the largest value."""
+    L = _lib()
+    p = _problem(nel, seed=41)
+    K0 = p["K0"]
+    rng = np.random.default_rng(42)
+    if k0 == "rotated":
+        Q, _ = np.linalg.qr(rng.standard_normal((3, 3)))
+        T = np.kron(np.eye(8), Q)
+        K0 = T.T @ K0 @ T
+    elif k0 == "unsymmetric":
+        K0 = K0 + 0.1 * rng.standard_normal((24, 24))
+    s = "f64" if dt == torch.float64 else "f32"
+    tol = 1e-13 if dt == torch.float64 else 1e-5
+    b = rng.standard_normal(p["n_dof"])
+    x, bt, y = dev(p["u"], dt), dev(b, dt), torch.empty(p["n_dof"], dtype=dt, device="cuda")
+    for cons in (p["cons"], None):
+        ct = None if cons is None else dev(cons.astype(np.uint8))
+        ax = oops.matvec(K0, p["el"], p["E"], p["u"], cons)
+        Dinv = rng.uniform(0.5, 1.5, p["n_dof"])
+        args = (3, L.nel_arg(nel), L.ptr(dev(np.ascontiguousarray(K0), dt)), L.ptr(dev(p["E"], dt)), L.ptr(ct), L.ptr(x))
+        L.call("et_matvec_" + s, *args, L.ptr(y), L.stream())
+        assert rel(y.cpu().numpy(), ax) < tol
+        L.call("et_residual_" + s, *args, L.ptr(bt), L.ptr(y), L.stream())
+        assert rel(y.cpu().numpy(), b - ax) < tol
+        L.call("et_jacobi_" + s, *args, L.ptr(bt), L.ptr(dev(Dinv, dt)), 0.6, L.ptr(y), L.stream())
+        assert rel(y.cpu().numpy(), p["u"] + 0.6 * Dinv * (b - ax)) < tol
