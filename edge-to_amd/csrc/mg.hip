@@ -6,13 +6,10 @@
 // block coupling node n to neighbour n + offset(o), one value per node, so a
 // wavefront reads each plane with unit stride.
 #include "common.hpp"
+#include "mg_weights.hpp"
 #include "stiffness.hpp"
 
 namespace et {
-
-__device__ __forceinline__ double pw(int d) {  // 2^-|d| for d in {-1, 0, 1}
-  return d == 0 ? 1.0 : 0.5;
-}
 
 template <int DIM>
 __device__ __forceinline__ void node_coords(const Grid& g, int64_t n, int& i, int& j, int& k) {
@@ -34,17 +31,6 @@ __device__ __forceinline__ double tw_of(const Grid& gc, int i, int j, int k) {
   double t = (i == 0 || i == gc.nx() - 1) ? 1.5 : 2.0;
   t *= (j == 0 || j == gc.ny() - 1) ? 1.5 : 2.0;
   if (DIM == 3) t *= (k == 0 || k == gc.nz() - 1) ? 1.5 : 2.0;
-  return t;
-}
-
-// 1/tw(c) as a product of per-axis factors (2/3 on the boundary, 1/2 inside),
-// in the working precision: no division in the transfer kernels
-template <typename T, int DIM>
-__device__ __forceinline__ T inv_tw_of(const Grid& gc, int i, int j, int k) {
-  const T bnd = T(2.0 / 3.0), mid = T(0.5);
-  T t = (i == 0 || i == gc.nx() - 1) ? bnd : mid;
-  t *= (j == 0 || j == gc.ny() - 1) ? bnd : mid;
-  if (DIM == 3) t *= (k == 0 || k == gc.nz() - 1) ? bnd : mid;
   return t;
 }
 

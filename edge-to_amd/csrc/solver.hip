@@ -20,6 +20,7 @@
 #include "galerkin_elem.hpp"
 #include "solver.hpp"
 #include "stiffness.hpp"
+#include "vcycle_2d.hpp"
 
 namespace et {
 
@@ -504,6 +505,14 @@ static int op_launch(const MGLevel<T>& L, const MGShared& sh, int mode, const T*
   return ET_OK;
 }
 
+// The fused legs cover two sweeps each way and one visit of the next level; their indices into a
+// level's stencil (20 values per node) are 32-bit.
+template <typename T>
+bool MGHierarchy<T>::vcycle2_level(int l) const {
+  return lv[l].g.dim == 2 && n_smooth == 2 && !(cycle_w && ((w_level_mask >> l) & 1)) &&
+         lv[l].g.n_nodes() < ((int64_t)1 << 31) / 20;
+}
+
 template <typename T>
 int MGHierarchy<T>::vcycle(int l, MGShared& sh, hipStream_t s, bool x0_ready) {
   MGLevel<T>& L = lv[l];
@@ -516,6 +525,22 @@ int MGHierarchy<T>::vcycle(int l, MGShared& sh, hipStream_t s, bool x0_ready) {
   const double ws = std::pow(1.06, l);
   const double* om = sh.scal + SC_OMEGA;
   const int64_t n = L.n;
+  if (vcycle2_level(l)) {
+    MGLevel<T>& C = lv[l + 1];
+    const T* op = l == 0 ? sh.K0<T>() : L.S;
+    sh.prof->begin(l == 0 ? ET_PROF_L0_JAC0 : ET_PROF_COARSE_OPS, s);
+    ET_TRY(vcycle2_down<T>(L.g, l == 0, op, sh.E<T>(), sh.cons, L.b, L.Dinv, om, ws, L.x, L.r, C.b, s));
+    sh.prof->end(s);
+    ET_TRY(vcycle(l + 1, sh, s));
+    const bool dot = l == 0 && sh.want_dot;
+    sh.prof->begin(l == 0 ? ET_PROF_L0_JACADD : ET_PROF_COARSE_OPS, s);
+    ET_TRY(vcycle2_up<T>(L.g, l == 0, op, sh.E<T>(), sh.cons, C.x, L.r, L.x, L.Dinv, om, ws, L.t, L.b,
+                         dot ? sh.dot_part : nullptr, s));
+    sh.prof->end(s);
+    if (dot) sh.dot_done = true;
+    std::swap(L.x, L.t);
+    return ET_OK;
+  }
   if (n_smooth == 0) {
     ET_CHECK_HIP(hipMemsetAsync(L.x, 0, n * sizeof(T), s));
   } else {
@@ -983,6 +1008,7 @@ int MGSolver::pcg(MGHierarchy<T>& h, const double* b, double* x, double tol, int
   ET_CHECK_LAUNCH();
   // the fused q = A p, p.q path exists for the 2-D and the transformed-basis operator
   const bool fused2 = g0.dim == 2 && op2d_partials(g0) <= kRedBlocks;
+  const bool legs2 = h.vcycle2_level(0);
   const bool tile3 = sh.tiled && tile3_faster(g0, sizeof(double));
   const bool fused3 = tile3 && tile3_partials(g0, sizeof(double)) <= kRedBlocks;
   const bool fused_pq = fused2 || fused3 ||
@@ -994,11 +1020,13 @@ int MGSolver::pcg(MGHierarchy<T>& h, const double* b, double* x, double tol, int
   // the last fine-grid sweep of the V-cycle (same operator) yields r.z, with r
   // in the V-cycle's precision (FP32 V-cycles: the copy of r they read)
   const bool fused_rz = fused_pq && get_fused_rz() && !sh.mfma && h.n_smooth > 0 &&
-                        (fused2 ||
+                        (legs2 ? vcycle2_tiles(g0) <= kRedBlocks
+                         : fused2 ||
                          (sh.tiled && tile3_faster(g0, sizeof(T))
                               ? tile3_partials(g0, sizeof(T)) <= kRedBlocks
                               : wht_supported(g0, sizeof(T)) && wht_partials(g0, sizeof(T), TM_JAC_ADD_DOT) <= kRedBlocks));
   const int n_rz_fused = !fused_rz ? kRedBlocks
+                         : legs2 ? vcycle2_tiles(g0)
                          : fused2 ? n_pq_fused
                          : tile3_faster(g0, sizeof(T)) ? tile3_partials(g0, sizeof(T))
                                                        : wht_partials(g0, sizeof(T), TM_JAC_ADD_DOT);

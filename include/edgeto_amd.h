@@ -484,7 +484,10 @@ int et_mg_last_timings(et_mg* handle, double* setup_ms, double* pcg_ms);
  * disables.  Each timed launch costs two event records on the stream, so time
  * only the classes needed inside a measured region.
  * et_mg_profile_read synchronises and fills ms[k] / launches[k] for the
- * ET_PROF_KINDS classes below (accumulated since the last enable). */
+ * ET_PROF_KINDS classes below (accumulated since the last enable).
+ * 2-D levels with two sweeps each way run as two kernels, transfers included: on
+ * the fine grid the way down counts as ET_PROF_L0_JAC0 and the way up as
+ * ET_PROF_L0_JACADD, on coarse levels both as ET_PROF_COARSE_OPS. */
 enum {
   ET_PROF_L0_JAC = 0,      /* fine-grid damped-Jacobi sweep  y = x + w D^-1 (b - A x)   */
   ET_PROF_L0_RES = 1,      /* fine-grid residual             y = b - A x               */
