@@ -853,7 +853,7 @@ int MGSolver::setup_levels(MGHierarchy<T>& h) {
   for (int l = 1; l <= L; ++l) {
     if (l == 1 && elem_galerkin) {
       ET_TRY(galerkin_from_elements(g0, sh.K0d, Mt, sh.Ed, sh.cons, eflag, S64[1], s));
-      if (use_l1) ET_TRY(l1.setup(sh.Ed, Mt, eflag, S64[1], s));
+      if (use_l1) ET_TRY(l1.setup(sh.Ed, eflag, S64[1], s));
     } else
       ET_TRY(galerkin(g, dof, S64[l - 1], S64[l], s, gal_work));
     g = g.coarse();

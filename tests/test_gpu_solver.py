@@ -175,6 +175,41 @@ def test_level_operators_match_galerkin(precision, level1_mf, nel):
         assert err < tol, (level, err)
 
 
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("nel", [(4, 4, 4), (30, 6, 8), (6, 36, 128), (8, 10, 130), (12, 8, 280), (128, 64, 64)])
+def test_level1_tiles(nel, precision):
+    """The matrix-free first coarse level against the stored Galerkin stencil of the same level: grids
+    of one tile and of several, columns of 64 elements and more (several tiles along z), with and
+    without the split by component (the largest grid), constrained DOFs on a face and inside.  Both
+    sum some 200 products in different orders."""
+    ET = _edgeto()
+    from edgeto_amd import _lib as L
+    rng = np.random.default_rng(51)
+    E = rng.uniform(0.01, 1.0, int(np.prod(nel)))
+    dt = torch.float32 if precision == "mixed" else torch.float64
+    x = torch.tensor(rng.standard_normal(3 * int(np.prod([n // 2 + 1 for n in nel]))), dtype=dt, device="cuda")
+    y = []
+    old = L.lib().et_tune_get(13)
+    for level1_mf in (1, 0):
+        L.call("et_tune_set", 13, level1_mf)
+        try:
+            mesh, kernel, filt, clamp, load = _cantilever_3d(ET, nel)
+            kernel.set_rho(torch.tensor(E, device="cuda"))
+            tp = ET.CuTopOpt(mesh, ET.SingleMaterial(void=1e-9, penalty=3.0, volume_fraction=0.3), kernel,
+                             None, filt, verbose=False)
+            tp.add_BC_nodal(clamp, np.array([[1, 1, 1]]))
+            tp.add_BC_nodal(np.arange(mesh.n_nodes)[7::1013], np.array([[0, 1, 0]]))
+            tp.add_F_nodal(load, np.array([[0.0, -1.0 / len(load), 0.0]]))
+            solver = ET.CuMultiGrid(mesh, kernel, tol=1e-30, maxiter=1, n_smooth=2, n_level=2, precision=precision)
+            solver.solve(tp.f, use_last=False)
+        finally:
+            L.call("et_tune_set", 13, old)
+        y.append(torch.empty_like(x))
+        L.call("et_mg_apply_level", solver._handle, 1, L.ptr(x), L.ptr(y[-1]))
+    err = ((y[0] - y[1]).abs().max() / y[1].abs().max()).item()
+    assert err < (1e-5 if precision == "mixed" else 1e-13), err
+
+
 @pytest.mark.parametrize("coarse_lib", [2, 1, 0])
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
 @pytest.mark.parametrize("nel", [(16, 8, 8), (24, 12, 12), (32, 16, 16)])
