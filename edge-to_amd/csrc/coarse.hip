@@ -245,6 +245,10 @@ __global__ __launch_bounds__(256) void yty_kernel(const double* Y, double* Ainv,
 //   panel:  A_ik <- A_ik W_kk^T for the nr tiles below;
 //   update: A_22 -= L_21 L_21^T on the nr x nr band block (one workgroup per
 //           lower tile: one launch where rocBLAS dsyrk took five).
+// A thread's 4 x 4 outputs of the panel and update products lie 16 rows and columns apart: lanes
+// then read consecutive LDS rows (the odd row length spreads them over the banks) and write
+// consecutive rows of A.  Four consecutive rows per lane meet in the banks: panel 12.5 -> 10.8 us,
+// update with the next diagonal factor 44 -> 41.7 us.
 // rocSOLVER trtri then overwrites L with Y = L^-1, and the coarse solve is
 // x = Y^T (Y b): two triangular products reading n^2 / 2 values each.
 
@@ -263,14 +267,14 @@ __global__ __launch_bounds__(256) void bchol_panel_kernel(double* A, int ld, int
     Ws[rr][cc] = Wk[rr + cc * NB];
   }
   __syncthreads();
-  const int r0 = (threadIdx.x % 16) * 4, c0 = (threadIdx.x / 16) * 4;
+  const int r0 = threadIdx.x % 16, c0 = threadIdx.x / 16;
   double acc[4][4] = {};
   for (int m = 0; m < NB; ++m) {
     double xa[4], wb[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      xa[u] = Xs[r0 + u][m];
-      wb[u] = Ws[c0 + u][m];
+      xa[u] = Xs[r0 + 16 * u][m];
+      wb[u] = Ws[c0 + 16 * u][m];
     }
 #pragma unroll
     for (int p = 0; p < 4; ++p)
@@ -280,7 +284,7 @@ __global__ __launch_bounds__(256) void bchol_panel_kernel(double* A, int ld, int
 #pragma unroll
   for (int q = 0; q < 4; ++q)
 #pragma unroll
-    for (int p = 0; p < 4; ++p) A[(int64_t)(o + c0 + q) * ld + row0 + r0 + p] = acc[p][q];
+    for (int p = 0; p < 4; ++p) A[(int64_t)(o + c0 + 16 * q) * ld + row0 + r0 + 16 * p] = acc[p][q];
 }
 
 // update: A_22 -= L_21 L_21^T on the lower tiles of the nr x nr band block below
@@ -304,14 +308,14 @@ __global__ __launch_bounds__(256) void bchol_syrk_kernel(double* A, int ld, int 
     Ys[rr][cc] = A[(int64_t)(o + cc) * ld + rj + rr];
   }
   __syncthreads();
-  const int r0 = (threadIdx.x % 16) * 4, c0 = (threadIdx.x / 16) * 4;
+  const int r0 = threadIdx.x % 16, c0 = threadIdx.x / 16;
   double acc[4][4] = {};
   for (int m = 0; m < NB; ++m) {
     double xa[4], yb[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      xa[u] = Xs[r0 + u][m];
-      yb[u] = Ys[c0 + u][m];
+      xa[u] = Xs[r0 + 16 * u][m];
+      yb[u] = Ys[c0 + 16 * u][m];
     }
 #pragma unroll
     for (int p = 0; p < 4; ++p)
@@ -322,7 +326,7 @@ __global__ __launch_bounds__(256) void bchol_syrk_kernel(double* A, int ld, int 
   for (int q = 0; q < 4; ++q)
 #pragma unroll
     for (int p = 0; p < 4; ++p)
-      if (i > j || r0 + p >= c0 + q) A[(int64_t)(rj + c0 + q) * ld + ri + r0 + p] -= acc[p][q];
+      if (i > j || r0 + 16 * p >= c0 + 16 * q) A[(int64_t)(rj + c0 + 16 * q) * ld + ri + r0 + 16 * p] -= acc[p][q];
   if (blockIdx.x == 0) {
     __syncthreads();  // the updated tile is read back by other threads of this workgroup
     chol_tile64(A, ld, o + NB, Wk, info);
