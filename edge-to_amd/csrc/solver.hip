@@ -19,8 +19,8 @@
 #include "common.hpp"
 #include "galerkin_elem.hpp"
 #include "solver.hpp"
+#include "pcg_check.hpp"
 #include "stiffness.hpp"
-#include "vcycle_2d.hpp"
 
 namespace et {
 
@@ -376,43 +376,14 @@ __global__ __launch_bounds__(256) void pcg_update_p_kernel(int64_t n, double* __
   }
 }
 
-// Convergence / breakdown test of one iteration, evaluated on the device so the
-// host never waits on the current iteration: r.r from the update's partials,
-// R = |r| / |b|; non-finite p.q or r.r, p.q <= 0 and R < tol stop the loop
-// (first reason wins, as in a plain sequential loop).  While running, omega =
-// min + d/2 exp((-clip(R, tol, 0.1) + tol) * 500) for the next V-cycle.
-// {R, status, stop} is published to pinned host memory.  One block of 256.
-__global__ __launch_bounds__(256) void pcg_check_kernel(double* sc, const double* __restrict__ rr_part, int n_rr,
-                                                        double tol, double wmin, double dw, double* ring) {
+// The convergence test as a kernel of its own, where the V-cycle does not make it.  One block of 256.
+__global__ __launch_bounds__(256) void pcg_check_kernel(const PcgCheck ck) {
+  const PcgState st = pcg_state(ck.sc);
   double rr = 0.0;
-  for (int t = threadIdx.x; t < n_rr; t += blockDim.x) rr += rr_part[t];
+  for (int t = threadIdx.x; t < ck.n_rr; t += blockDim.x) rr += ck.rr_part[t];
   rr = block_sum256(rr);
   if (threadIdx.x != 0) return;
-  if (sc[SC_STOP] == 0.0) {
-    sc[SC_RR] = rr;
-    const double pq = sc[SC_PQ];
-    const double R = sqrt(rr) / sqrt(sc[SC_BB]);
-    double status = (double)ET_OK, stop = 0.0;
-    if (!isfinite(pq) || !isfinite(rr)) {
-      status = (double)ET_ENONFINITE;
-      stop = 1.0;
-    } else if (!(pq > 0.0)) {
-      status = (double)ET_EBREAKDOWN;
-      stop = 1.0;
-    } else if (R < tol) {
-      stop = 1.0;
-    }
-    sc[SC_R] = R;
-    sc[SC_STATUS] = status;
-    sc[SC_STOP] = stop;
-    if (stop == 0.0) {
-      const double Rc = fmin(fmax(R, tol), 1e-1);
-      sc[SC_OMEGA] = wmin + dw / 2.0 * exp((-Rc + tol) * 500.0);
-    }
-  }
-  ring[0] = sc[SC_R];
-  ring[1] = sc[SC_STATUS];
-  ring[2] = sc[SC_STOP];
+  pcg_check(ck, st, rr);
   __threadfence_system();
 }
 
@@ -529,8 +500,10 @@ int MGHierarchy<T>::vcycle(int l, MGShared& sh, hipStream_t s, bool x0_ready) {
     MGLevel<T>& C = lv[l + 1];
     const T* op = l == 0 ? sh.K0<T>() : L.S;
     sh.prof->begin(l == 0 ? ET_PROF_L0_JAC0 : ET_PROF_COARSE_OPS, s);
-    ET_TRY(vcycle2_down<T>(L.g, l == 0, op, sh.E<T>(), sh.cons, L.b, L.Dinv, om, ws, L.x, L.r, C.b, s));
+    const PcgCheck* ck = l == 0 ? sh.check : nullptr;
+    ET_TRY(vcycle2_down<T>(L.g, l == 0, op, sh.E<T>(), sh.cons, L.b, L.Dinv, om, ws, L.x, L.r, C.b, ck, s));
     sh.prof->end(s);
+    if (ck != nullptr) ET_CHECK_HIP(hipEventRecord(sh.check_ev, s));
     ET_TRY(vcycle(l + 1, sh, s));
     const bool dot = l == 0 && sh.want_dot;
     sh.prof->begin(l == 0 ? ET_PROF_L0_JACADD : ET_PROF_COARSE_OPS, s);
@@ -1001,9 +974,12 @@ int MGSolver::pcg(MGHierarchy<T>& h, const double* b, double* x, double tol, int
   ET_TRY(precondition(h, false, &z));
   prof.begin(ET_PROF_PCG_VEC, s);
   // partial: first-stage sums of p.q and r.z; partial2: of r.r
+  // workgroups of the vector updates: a value of r, four of p a thread
+  const int n_rr = (int)std::min<int64_t>(kRedBlocks, (n_dof + 255) / 256);
+  const int n_pb = (int)std::min<int64_t>(kRedBlocks, (n_dof + 1023) / 1024);
   double* partial2 = partial + kRedBlocks;
   pcg_dot_kernel<T><<<kRedBlocks, 256, 0, s>>>(n_dof, r, z, partial);
-  pcg_update_p_kernel<T><<<kRedBlocks, 256, 0, s>>>(n_dof, sh.scal, 0, partial, kRedBlocks, z, p_, x, 1);
+  pcg_update_p_kernel<T><<<n_pb, 256, 0, s>>>(n_dof, sh.scal, 0, partial, kRedBlocks, z, p_, x, 1);
   prof.end(s);
   ET_CHECK_LAUNCH();
   // the fused q = A p, p.q path exists for the 2-D and the transformed-basis operator
@@ -1065,13 +1041,14 @@ int MGSolver::pcg(MGHierarchy<T>& h, const double* b, double* x, double tol, int
       prof.begin(ET_PROF_PCG_VEC, s);
       ET_TRY(dot_partials(n_dof, p_, q, partial, s));
     }
-    pcg_update_xr_kernel<T><<<kRedBlocks, 256, 0, s>>>(n_dof, sh.scal, cur, partial, n_pq, q, r, rb,
-                                                       partial2);
+    pcg_update_xr_kernel<T><<<n_rr, 256, 0, s>>>(n_dof, sh.scal, cur, partial, n_pq, q, r, rb, partial2);
     ET_CHECK_LAUNCH();
-    pcg_check_kernel<<<1, 256, 0, s>>>(sh.scal, partial2, kRedBlocks, tol, min_omega, d_omega,
-                                       ring_dev + 4 * (it & 1));
-    ET_CHECK_LAUNCH();
-    ET_CHECK_HIP(hipEventRecord(ring_ev[it & 1], s));
+    const PcgCheck ck{sh.scal, partial2, n_rr, tol, min_omega, d_omega, ring_dev + 4 * (it & 1)};
+    if (!legs2) {
+      pcg_check_kernel<<<1, 256, 0, s>>>(ck);
+      ET_CHECK_LAUNCH();
+      ET_CHECK_HIP(hipEventRecord(ring_ev[it & 1], s));
+    }
     prof.end(s);
     last = it;
     if (it > 1 && read_ring(it - 1, &R, &status)) {
@@ -1083,8 +1060,11 @@ int MGSolver::pcg(MGHierarchy<T>& h, const double* b, double* x, double tol, int
     sh.want_dot = fused_rz;
     sh.dot_part = partial;
     sh.dot_done = false;
+    sh.check = legs2 ? &ck : nullptr;
+    sh.check_ev = ring_ev[it & 1];
     const int pst = precondition(h, true, &z);
     sh.want_dot = false;
+    sh.check = nullptr;
     ET_TRY(pst);
     prof.begin(ET_PROF_PCG_VEC, s);
     int n_rz = n_rz_fused;
@@ -1092,7 +1072,7 @@ int MGSolver::pcg(MGHierarchy<T>& h, const double* b, double* x, double tol, int
       pcg_dot_kernel<T><<<kRedBlocks, 256, 0, s>>>(n_dof, r, z, partial);
       n_rz = kRedBlocks;
     }
-    pcg_update_p_kernel<T><<<kRedBlocks, 256, 0, s>>>(n_dof, sh.scal, it & 1, partial, n_rz, z, p_, x, 0);
+    pcg_update_p_kernel<T><<<n_pb, 256, 0, s>>>(n_dof, sh.scal, it & 1, partial, n_rz, z, p_, x, 0);
     prof.end(s);
     ET_CHECK_LAUNCH();
   }

@@ -6,6 +6,7 @@
 #include "common.hpp"
 #include "level1.hpp"
 #include "stiffness.hpp"
+#include "vcycle_2d.hpp"
 
 namespace et {
 
@@ -78,6 +79,10 @@ struct MGShared {
   bool want_dot = false;
   double* dot_part = nullptr;
   bool dot_done = false;
+  // When set (2-D legs on the fine grid), the V-cycle's first kernel makes the
+  // convergence test; check_ev is recorded behind it.
+  const PcgCheck* check = nullptr;
+  hipEvent_t check_ev = nullptr;
   template <typename T>
   const T* K0() const;
   template <typename T>

@@ -13,6 +13,9 @@
 // that every stage is one round.  A is the element operator on level 0 (any K0, constrained rows
 // identity) and the half-stored block stencil below (layout in solver.hip).  Sums run in the order
 // of the single kernels, so results are theirs to rounding.
+// The convergence test of the PCG iteration is part of the first leg down: every workgroup sums r.r
+// (up to 1024 partials) while its operands are on their way, instead of a launch of 4 us between the
+// update of r and the cycle (512 x 256 mixed 10.7 -> 8.9 ms).
 // Whole solves, six launches per level -> two: 512 x 256 mixed 13.3 -> 10.6 ms, 120 x 40 FP64
 // 3.47 -> 2.76 ms.  The legs also read each vector once where the single kernels read it up to
 // three times, so they stay ahead on large grids: a PCG iteration takes 143 us at 1024 x 512, mixed,
@@ -21,6 +24,7 @@
 #include "common.hpp"
 #include "mg_weights.hpp"
 #include "op_tiled.hpp"
+#include "pcg_check.hpp"
 #include "stiffness.hpp"
 #include "vcycle_2d.hpp"
 
@@ -119,7 +123,8 @@ __global__ __launch_bounds__(kThreads) void down2_kernel(const Grid g, const Gri
                                                          const T* __restrict__ E, const uint8_t* __restrict__ cons,
                                                          const T* __restrict__ b, const T* __restrict__ Dinv,
                                                          const double* __restrict__ omega, double wscale,
-                                                         T* __restrict__ x1, T* __restrict__ r, T* __restrict__ bc) {
+                                                         T* __restrict__ x1, T* __restrict__ r, T* __restrict__ bc,
+                                                         const PcgCheck ck) {
   constexpr int P0 = kW + 5, P1 = kW + 3, P2 = kW + 1, PE = kW + 4;
   __shared__ Field<T, P0> fb, fd, u0;
   __shared__ Field<T, P1> u1, v1;  // x1 with constrained DOFs zeroed, and as it is (level 0)
@@ -129,23 +134,49 @@ __global__ __launch_bounds__(kThreads) void down2_kernel(const Grid g, const Gri
   const int nx = g.nx(), ny = g.ny(), N = nx * ny;
   const int ntx = (nx + kW - 1) / kW;
   const int x0 = blockIdx.x % ntx * kW, y0 = blockIdx.x / ntx * kW;
-  const T w = (T)(*omega * wscale);
   const int tid = threadIdx.x;
 
+  // operands of the first stage (clamped: every lane loads)
+  const int t0 = min(tid, P0 * P0 - 1), i0 = x0 - 3 + t0 % P0, j0 = y0 - 3 + t0 / P0;
+  const bool in0 = i0 >= 0 && i0 < nx && j0 >= 0 && j0 < ny;
+  const int d0 = 2 * (min(max(j0, 0), ny - 1) * nx + min(max(i0, 0), nx - 1));
+  T b0[2], dv0[2];
+  bool f0[2];
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    b0[c] = b[d0 + c];
+    dv0[c] = Dinv[d0 + c];
+    f0[c] = L0 && cons[d0 + c] != 0;
+  }
   if (L0) stage_elements<T, PE>(g, E, x0 - 3, y0 - 3, sE);
+  T w;
+  if (L0 && ck.sc != nullptr) {
+    // every workgroup sums r.r in the same order and takes omega from it; the first one records the
+    // test.  Once the loop has stopped, omega does not matter: nothing of this cycle is used.
+    __shared__ double srr[kThreads / 64];
+    const PcgState st = pcg_state(ck.sc);
+    double rr = 0.0;
+    for (int t = tid; t < ck.n_rr; t += kThreads) rr += ck.rr_part[t];
+    rr = wave_sum(rr);
+    if ((tid & 63) == 0) srr[tid >> 6] = rr;
+    __syncthreads();
+    rr = 0.0;
+#pragma unroll
+    for (int k = 0; k < kThreads / 64; ++k) rr += srr[k];
+    w = (T)(pcg_omega(sqrt(rr) / sqrt(st.bb), ck.tol, ck.wmin, ck.dw) * wscale);
+    // by the last wavefront, which has no part in the next stages
+    if (blockIdx.x == 0 && tid == kThreads - 1) pcg_check(ck, st, rr);
+  } else {
+    w = (T)(*omega * wscale);
+  }
   if (tid < P0 * P0) {
-    const int i = x0 - 3 + tid % P0, j = y0 - 3 + tid / P0;
-    const bool in = i >= 0 && i < nx && j >= 0 && j < ny;
-    const int d = 2 * (min(max(j, 0), ny - 1) * nx + min(max(i, 0), nx - 1));
     int m = 0;
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
-      const T bv = b[d + c], dv = Dinv[d + c];
-      const bool f = L0 && cons[d + c] != 0;
-      m |= f ? 1 << c : 0;
-      fb.v[c][tid] = in ? bv : T(0);
-      fd.v[c][tid] = in ? dv : T(0);
-      u0.v[c][tid] = in && !f ? w * dv * bv : T(0);
+      m |= f0[c] ? 1 << c : 0;
+      fb.v[c][tid] = in0 ? b0[c] : T(0);
+      fd.v[c][tid] = in0 ? dv0[c] : T(0);
+      u0.v[c][tid] = in0 && !f0[c] ? w * dv0[c] * b0[c] : T(0);
     }
     if (L0) fx[tid] = (uint8_t)m;
   }
@@ -198,6 +229,7 @@ __global__ __launch_bounds__(kThreads) void down2_kernel(const Grid g, const Gri
     for (int c = 0; c < 2; ++c) fr.v[c][tid] = v[c];
   }
   __syncthreads();
+  if (L0 && ck.sc != nullptr && blockIdx.x == 0 && tid == kThreads - 1) __threadfence_system();
   // restriction to the coarse nodes whose fine node lies in the tile (r is zero outside the grid)
   constexpr int HC = kW / 2;
   if (tid < HC * HC) {
@@ -351,12 +383,13 @@ int vcycle2_tiles(const Grid& g) { return ((g.nx() + kW - 1) / kW) * ((g.ny() + 
 
 template <typename T>
 int vcycle2_down(const Grid& g, bool level0, const T* op, const T* E, const uint8_t* cons, const T* b, const T* Dinv,
-                 const double* omega, double wscale, T* x1, T* r, T* bc, hipStream_t s) {
+                 const double* omega, double wscale, T* x1, T* r, T* bc, const PcgCheck* ck, hipStream_t s) {
   const int n = vcycle2_tiles(g);
+  const PcgCheck c = ck != nullptr ? *ck : PcgCheck{};
   if (level0)
-    down2_kernel<T, true><<<n, kThreads, 0, s>>>(g, g.coarse(), op, E, cons, b, Dinv, omega, wscale, x1, r, bc);
+    down2_kernel<T, true><<<n, kThreads, 0, s>>>(g, g.coarse(), op, E, cons, b, Dinv, omega, wscale, x1, r, bc, c);
   else
-    down2_kernel<T, false><<<n, kThreads, 0, s>>>(g, g.coarse(), op, E, cons, b, Dinv, omega, wscale, x1, r, bc);
+    down2_kernel<T, false><<<n, kThreads, 0, s>>>(g, g.coarse(), op, E, cons, b, Dinv, omega, wscale, x1, r, bc, c);
   ET_CHECK_LAUNCH();
   return ET_OK;
 }
@@ -379,7 +412,7 @@ int vcycle2_up(const Grid& g, bool level0, const T* op, const T* E, const uint8_
 
 #define ET_V2(T)                                                                                                    \
   template int vcycle2_down<T>(const Grid&, bool, const T*, const T*, const uint8_t*, const T*, const T*,           \
-                               const double*, double, T*, T*, T*, hipStream_t);                                     \
+                               const double*, double, T*, T*, T*, const PcgCheck*, hipStream_t);                    \
   template int vcycle2_up<T>(const Grid&, bool, const T*, const T*, const uint8_t*, const T*, const T*, const T*,   \
                              const T*, const double*, double, T*, const T*, double*, hipStream_t);
 ET_V2(double)
