@@ -92,6 +92,13 @@ __host__ __device__ constexpr int qx(int a) { return (a == 1 || a == 2) ? 1 : 0;
 __host__ __device__ constexpr int qy(int a) { return (a == 2 || a == 3) ? 1 : 0; }
 
 // Wavefront (64-lane) sum via DPP-backed shuffles.
+// v rounded to T here: what follows is not contracted with the product that v comes from
+template <typename T>
+__device__ __forceinline__ T rounded(T v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+
 template <typename T>
 __device__ inline T wave_sum(T v) {
 #pragma unroll

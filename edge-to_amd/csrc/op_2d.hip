@@ -3,7 +3,7 @@
 //   TM_Y y = A x; TM_RES y = b - A x; TM_JAC y = x + w D^-1 (b - A x); TM_JAC_ADD the same + xadd;
 //   TM_YDOT y = A x and per-workgroup sums of x.y; TM_JAC0 the first two Jacobi sweeps from the
 //   zero guess (x = w D^-1 b formed while staging); TM_JAC_ADD_DOT TM_JAC_ADD and per-workgroup
-//   sums of bdot.y.
+//   sums of bdot.y (bdot in FP64 also beside FP32 sweeps: r.z loses nothing to r's FP32 copy).
 //
 // A_hat = M K(E) M + I_c with any symmetric or unsymmetric 8 x 8 K0 (core/_templated_cuda.cu:782-834
 // for Q4 elements).  One thread owns one node of a 32 x 8 tile and sums its four elements in the
@@ -33,7 +33,7 @@ __global__ __launch_bounds__(256) void op2d_kernel(const Grid g, const T* __rest
                                                    const T* __restrict__ b, const T* __restrict__ Dinv,
                                                    const double* __restrict__ omega, double wscale,
                                                    const T* __restrict__ xadd, T* __restrict__ y,
-                                                   const T* __restrict__ bdot, double* __restrict__ part) {
+                                                   const double* __restrict__ bdot, double* __restrict__ part) {
   constexpr int PX = kTX + 2, PY = kTY + 2, EX = kTX + 1, EY = kTY + 1;
   constexpr bool kJac = MODE == TM_JAC || MODE == TM_JAC_ADD || MODE == TM_JAC0 || MODE == TM_JAC_ADD_DOT;
   constexpr bool kAdd = MODE == TM_JAC_ADD || MODE == TM_JAC_ADD_DOT;
@@ -46,7 +46,8 @@ __global__ __launch_bounds__(256) void op2d_kernel(const Grid g, const T* __rest
 
   // the own node's operands (clamped to the grid: every lane loads)
   const int i = x0 + tx, j = y0 + ty;
-  T ob[2], od[2], oa[2], ot[2], ox[2];
+  T ob[2], od[2], oa[2], ox[2];
+  double ot[2];
   bool fixed[2];
   {
     const int d = 2 * (min(j, ny - 1) * nx + min(i, nx - 1));
@@ -109,7 +110,7 @@ __global__ __launch_bounds__(256) void op2d_kernel(const Grid g, const T* __rest
     const int d = 2 * (j * nx + i);
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
-      const T xv = MODE == TM_JAC0 ? w * od[c] * ob[c] : ox[c];
+      const T xv = MODE == TM_JAC0 ? rounded(w * od[c] * ob[c]) : ox[c];
       const T ax = fixed[c] ? xv : acc[c];
       T v;
       if (MODE == TM_Y || MODE == TM_YDOT)
@@ -121,7 +122,7 @@ __global__ __launch_bounds__(256) void op2d_kernel(const Grid g, const T* __rest
       if (kAdd) v += oa[c];
       y[d + c] = v;
       if (MODE == TM_YDOT) dot += (double)xv * (double)v;
-      if (MODE == TM_JAC_ADD_DOT) dot += (double)ot[c] * (double)v;
+      if (MODE == TM_JAC_ADD_DOT) dot += ot[c] * (double)v;
     }
   }
   if (MODE == TM_YDOT || MODE == TM_JAC_ADD_DOT) {
@@ -138,7 +139,7 @@ int op2d_partials(const Grid& g) {
 
 template <typename T>
 int op2d(int mode, const Grid& g, const T* K0, const T* E, const uint8_t* cons, const T* x, const T* b, const T* Dinv,
-         const double* omega, double wscale, const T* xadd, T* y, const T* bdot, double* part, hipStream_t s) {
+         const double* omega, double wscale, const T* xadd, T* y, const double* bdot, double* part, hipStream_t s) {
   const unsigned grid = op2d_partials(g);
 #define ET_OP2(M) \
   op2d_kernel<T, M><<<grid, 256, 0, s>>>(g, K0, E, cons, x, b, Dinv, omega, wscale, xadd, y, bdot, part)
@@ -160,7 +161,7 @@ template int op2d<double>(int, const Grid&, const double*, const double*, const 
                           const double*, const double*, double, const double*, double*, const double*, double*,
                           hipStream_t);
 template int op2d<float>(int, const Grid&, const float*, const float*, const uint8_t*, const float*, const float*,
-                         const float*, const double*, double, const float*, float*, const float*, double*,
+                         const float*, const double*, double, const float*, float*, const double*, double*,
                          hipStream_t);
 
 }  // namespace et

@@ -507,8 +507,8 @@ int MGHierarchy<T>::vcycle(int l, MGShared& sh, hipStream_t s, bool x0_ready) {
     ET_TRY(vcycle(l + 1, sh, s));
     const bool dot = l == 0 && sh.want_dot;
     sh.prof->begin(l == 0 ? ET_PROF_L0_JACADD : ET_PROF_COARSE_OPS, s);
-    ET_TRY(vcycle2_up<T>(L.g, l == 0, op, sh.E<T>(), sh.cons, C.x, L.r, L.x, L.Dinv, om, ws, L.t, L.b,
-                         dot ? sh.dot_part : nullptr, s));
+    ET_TRY(vcycle2_up<T>(L.g, l == 0, op, sh.E<T>(), sh.cons, C.x, L.r, L.x, L.Dinv, om, ws, L.t,
+                         sh.dot_r, dot ? sh.dot_part : nullptr, s));
     sh.prof->end(s);
     if (dot) sh.dot_done = true;
     std::swap(L.x, L.t);
@@ -565,7 +565,7 @@ int MGHierarchy<T>::vcycle(int l, MGShared& sh, hipStream_t s, bool x0_ready) {
         const int st =
             L.g.dim == 2
                 ? op2d<T>(TM_JAC_ADD_DOT, L.g, sh.K0<T>(), sh.E<T>(), sh.cons, L.e, L.r, L.Dinv, om, ws, L.x, L.t,
-                          L.b, sh.dot_part, s)
+                          sh.dot_r, sh.dot_part, s)
             : sh.tiled && tile3_faster(L.g, sizeof(T))
                 ? op_tile3<T>(TM_JAC_ADD_DOT, L.g, sh.K0<T>(), &sh.wht, sh.E<T>(), sh.cons, L.e,
                               L.r, L.Dinv, om, ws, L.x, L.t, L.b, sh.dot_part, s)
@@ -1059,6 +1059,7 @@ int MGSolver::pcg(MGHierarchy<T>& h, const double* b, double* x, double tol, int
     // r.z partials from the V-cycle's last fine sweep where it can produce them
     sh.want_dot = fused_rz;
     sh.dot_part = partial;
+    sh.dot_r = r;
     sh.dot_done = false;
     sh.check = legs2 ? &ck : nullptr;
     sh.check_ev = ring_ev[it & 1];

@@ -78,6 +78,7 @@ struct MGShared {
   // V-cycle's precision, z its output) to dot_part and sets dot_done.
   bool want_dot = false;
   double* dot_part = nullptr;
+  const double* dot_r = nullptr;  // 2-D: r itself, FP64
   bool dot_done = false;
   // When set (2-D legs on the fine grid), the V-cycle's first kernel makes the
   // convergence test; check_ev is recorded behind it.

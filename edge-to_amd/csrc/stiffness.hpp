@@ -119,7 +119,7 @@ int tile3_partials(const Grid& g, size_t elem_bytes);
 // product, which write op2d_partials(g) per-workgroup sums to part.
 template <typename T>
 int op2d(int mode, const Grid& g, const T* K0, const T* E, const uint8_t* cons, const T* x, const T* b, const T* Dinv,
-         const double* omega, double wscale, const T* xadd, T* y, const T* bdot, double* part, hipStream_t s);
+         const double* omega, double wscale, const T* xadd, T* y, const double* bdot, double* part, hipStream_t s);
 int op2d_partials(const Grid& g);
 // whether op0_fine supports the fused zero-guess Jacobi mode (5) on this grid
 bool fine_jac0_supported(const Grid& g, size_t elem_bytes);

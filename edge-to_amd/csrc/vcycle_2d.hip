@@ -206,7 +206,7 @@ __global__ __launch_bounds__(kThreads) void down2_kernel(const Grid g, const Gri
         st1.template apply<P0>(u0, lx + 1, ly + 1, ax);
 #pragma unroll
       for (int c = 0; c < 2; ++c) {
-        const T bv = fb.v[c][at], dv = fd.v[c][at], xv = w * dv * bv;
+        const T bv = fb.v[c][at], dv = fd.v[c][at], xv = rounded(w * dv * bv);
         if (L0 && ((fx[at] >> c) & 1)) ax[c] = xv;
         v[c] = xv + w * dv * (bv - ax[c]);
         if (lx >= 2 && lx < kW + 2 && ly >= 2 && ly < kW + 2) x1[2 * (j1 * nx + i1) + c] = v[c];
@@ -261,14 +261,15 @@ __global__ __launch_bounds__(kThreads) void down2_kernel(const Grid g, const Gri
   }
 }
 
-// DOT: also per-workgroup sums of bdot.x
+// DOT: also per-workgroup sums of bdot.x, bdot in FP64 (r.z with r's FP32 copy cost the mixed 2-D
+// solver a quarter more iterations at 512 x 256)
 template <typename T, bool L0, bool DOT>
 __global__ __launch_bounds__(kThreads) void up2_kernel(const Grid g, const Grid gc, const T* __restrict__ op,
                                                        const T* __restrict__ E, const uint8_t* __restrict__ cons,
                                                        const T* __restrict__ xc, const T* __restrict__ r,
                                                        const T* __restrict__ x1, const T* __restrict__ Dinv,
                                                        const double* __restrict__ omega, double wscale,
-                                                       T* __restrict__ x, const T* __restrict__ bdot,
+                                                       T* __restrict__ x, const double* __restrict__ bdot,
                                                        double* __restrict__ part) {
   constexpr int P0 = kW + 4, P1 = kW + 2, PE = kW + 3;
   __shared__ Field<T, P0> u0, v0;
@@ -289,13 +290,14 @@ __global__ __launch_bounds__(kThreads) void up2_kernel(const Grid g, const Grid 
   const int ic1 = min(max(i1, 0), nx - 1), jc1 = min(max(j1, 0), ny - 1), d1 = 2 * (jc1 * nx + ic1);
   Stencil<T> st1;
   if (!L0) st1.load(op, N, nx, ny, ic1, jc1);
-  T r1[2], dd1[2], xa[2], bt[2];
+  T r1[2], dd1[2], xa[2];
+  double bt[2];
 #pragma unroll
   for (int c = 0; c < 2; ++c) {
     r1[c] = r[d1 + c];
     dd1[c] = Dinv[d1 + c];
     xa[c] = x1[d1 + c];
-    bt[c] = DOT ? bdot[d1 + c] : T(0);
+    bt[c] = DOT ? bdot[d1 + c] : 0.0;
   }
   if (L0) stage_elements<T, PE>(g, E, x0 - 2, y0 - 2, sE);
   if (tid < P0 * P0) {
@@ -368,7 +370,7 @@ __global__ __launch_bounds__(kThreads) void up2_kernel(const Grid g, const Grid 
       T v = e + w * dd1[c] * (r1[c] - ax[c]);
       v += xa[c];
       x[d1 + c] = v;
-      if (DOT) dot += (double)bt[c] * (double)v;
+      if (DOT) dot += bt[c] * (double)v;
     }
   }
   if (DOT) {
@@ -403,7 +405,7 @@ int vcycle2_down(const Grid& g, bool level0, const T* op, const T* E, const uint
 
 template <typename T>
 int vcycle2_up(const Grid& g, bool level0, const T* op, const T* E, const uint8_t* cons, const T* xc, const T* r,
-               const T* x1, const T* Dinv, const double* omega, double wscale, T* x, const T* bdot, double* part,
+               const T* x1, const T* Dinv, const double* omega, double wscale, T* x, const double* bdot, double* part,
                hipStream_t s) {
   const int n = vcycle2_tiles(g);
   const Grid gc = g.coarse();
@@ -421,7 +423,7 @@ int vcycle2_up(const Grid& g, bool level0, const T* op, const T* E, const uint8_
   template int vcycle2_down<T>(const Grid&, bool, const T*, const T*, const uint8_t*, const T*, const T*,           \
                                const double*, double, T*, T*, T*, const PcgCheck*, hipStream_t);                    \
   template int vcycle2_up<T>(const Grid&, bool, const T*, const T*, const uint8_t*, const T*, const T*, const T*,   \
-                             const T*, const double*, double, T*, const T*, double*, hipStream_t);
+                             const T*, const double*, double, T*, const double*, double*, hipStream_t);
 ET_V2(double)
 ET_V2(float)
 #undef ET_V2

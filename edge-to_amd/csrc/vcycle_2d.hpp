@@ -27,7 +27,7 @@ int vcycle2_down(const Grid& g, bool level0, const T* op, const T* E, const uint
 // e = two Jacobi sweeps on A e = r from e0 = P xc, x = x1 + e; part (level 0 only, may be null): sums of bdot.x
 template <typename T>
 int vcycle2_up(const Grid& g, bool level0, const T* op, const T* E, const uint8_t* cons, const T* xc, const T* r,
-               const T* x1, const T* Dinv, const double* omega, double wscale, T* x, const T* bdot, double* part,
+               const T* x1, const T* Dinv, const double* omega, double wscale, T* x, const double* bdot, double* part,
                hipStream_t s);
 
 }  // namespace et
