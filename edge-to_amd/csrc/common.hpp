@@ -91,7 +91,6 @@ __host__ __device__ constexpr int hz(int a) { return a >= 4 ? 1 : 0; }
 __host__ __device__ constexpr int qx(int a) { return (a == 1 || a == 2) ? 1 : 0; }
 __host__ __device__ constexpr int qy(int a) { return (a == 2 || a == 3) ? 1 : 0; }
 
-// Wavefront (64-lane) sum via DPP-backed shuffles.
 // v rounded to T here: what follows is not contracted with the product that v comes from
 template <typename T>
 __device__ __forceinline__ T rounded(T v) {
@@ -99,6 +98,7 @@ __device__ __forceinline__ T rounded(T v) {
   return v;
 }
 
+// Wavefront (64-lane) sum via DPP-backed shuffles.
 template <typename T>
 __device__ inline T wave_sum(T v) {
 #pragma unroll

@@ -13,15 +13,14 @@
 // that every stage is one round.  A is the element operator on level 0 (any K0, constrained rows
 // identity) and the half-stored block stencil below (layout in solver.hip); a thread keeps one node
 // through the stages, so the stencil's 36 values are loaded once, ahead of the first stage (6.4 ->
-// 5.2 us for a leg down in FP32, 6.2 -> 5.2 in FP64).  Sums run in the order
-// of the single kernels, so results are theirs to rounding.
+// 5.2 us for a leg down in FP32, 6.2 -> 5.2 in FP64).  Sums run in the order of the single kernels.
 // The convergence test of the PCG iteration is part of the first leg down: every workgroup sums r.r
-// (up to 1024 partials) while its operands are on their way, instead of a launch of 4 us between the
-// update of r and the cycle (512 x 256 mixed 10.7 -> 8.9 ms).
-// Whole solves, six launches per level -> two: 512 x 256 mixed 13.3 -> 10.6 ms, 120 x 40 FP64
-// 3.47 -> 2.76 ms.  The legs also read each vector once where the single kernels read it up to
-// three times, so they stay ahead on large grids: a PCG iteration takes 143 us at 1024 x 512, mixed,
-// and 855 us at 2048 x 2048, FP64, where six launches of per-node gathers took 270 and 1730.
+// (up to 1024 partials) while its operands are on their way (512 x 256: the leg takes 9.2 us with it,
+// 7.2 without), instead of a launch of 4 us between the update of r and the cycle.
+// Six launches per level -> two: 120 x 40 FP64 solve 3.47 -> 2.76 ms.  The legs also read each vector
+// once where the single kernels read it up to three times, so they stay ahead on large grids: a PCG
+// iteration takes 143 us at 1024 x 512, mixed, and 855 us at 2048 x 2048, FP64, where six launches
+// of per-node gathers took 270 and 1730.
 #include "blas.hpp"
 #include "common.hpp"
 #include "mg_weights.hpp"

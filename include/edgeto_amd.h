@@ -76,10 +76,10 @@ const char* et_version(void);
  * ET_TUNE_LEVEL1_MF: 1 (default) = the first coarse level of 3-D hierarchies with even
  *   element counts is applied matrix-free from the element densities; 0 = stored stencil.
  *   Read by et_mg_create.
- * ET_TUNE_FUSED_RZ: 1 (default) = in PCG with the transformed-basis operator, the
+ * ET_TUNE_FUSED_RZ: 1 (default) = in PCG with the transformed-basis or a 2-D operator, the
  *   last fine-grid sweep of each V-cycle also sums r.z per workgroup, r taken in the
- *   V-cycle's precision (FP32 V-cycles: their FP32 copy of r); no separate pass over r
- *   and z.  0 = separate reduction with r in FP64.  Read by each solve.
+ *   V-cycle's precision (FP32 V-cycles: their FP32 copy of r; 2-D: always the FP64 r); no
+ *   separate pass over r and z.  0 = separate reduction with r in FP64.  Read by each solve.
  * ET_TUNE_FILTER_ROWS: y rows of the 3-D filter stencils' tiles (64 elements along z each):
  *   8 (default, 512 threads) or 4 (256 threads).
  * ET_TUNE_TILE3_NODES: 3-D fine grids with at most this many nodes (and at most 64 elements

@@ -403,6 +403,33 @@ def test_fused_2d_cycle(nel, n_level, precision):
     assert err < (1e-11 if precision == "fp64" else 2e-3)
 
 
+def test_mixed_2d_iterations():
+    """An ill-conditioned 2-D solve (moduli over two decades, more than 100 PCG iterations): the FP32
+    V-cycle costs no iterations while r.z is summed with r in FP64 (with r's FP32 copy: a quarter
+    more).  A tenth is left for the cycle's own rounding."""
+    ET = _edgeto()
+    nel = (352, 96)
+    mesh = ET.CuStructuredMesh2D(*nel, *nel, stiffness=lambda x0: ET.auto_stiffness(x0, 1.0, 0.3))
+    kernel = ET.CuStructuredStiffnessKernel(mesh)
+    rng = np.random.default_rng(7)
+    X, Y = np.meshgrid(np.linspace(0, 1, nel[0]), np.linspace(0, 1, nel[1]), indexing="ij")
+    f = sum(np.sin(2 * np.pi * (rng.uniform(-3, 3) * X + rng.uniform(-6, 6) * Y + rng.uniform())) for _ in range(8))
+    kernel.set_rho(torch.tensor((0.5 + 0.35 * np.tanh(f)).ravel() ** 3, device="cuda"))
+    tp = ET.CuTopOpt(mesh, ET.SingleMaterial(void=1e-9, penalty=3.0, volume_fraction=0.3), kernel,
+                     None, ET.CuStructuredFilter2D(mesh, 1.5), verbose=False)
+    tp.add_BC_nodal(np.arange(nel[1] + 1) * (nel[0] + 1), np.array([[1, 0]]))
+    tp.add_BC_nodal(np.array([nel[0]]), np.array([[0, 1]]))
+    tp.add_F_nodal(np.array([nel[1] * (nel[0] + 1)]), np.array([[0.0, -1.0]]))
+    iters = {}
+    for precision in ("fp64", "mixed"):
+        solver = ET.CuMultiGrid(mesh, kernel, tol=1e-8, n_smooth=2, n_level=4, precision=precision)
+        _, res = solver.solve(tp.f, use_last=False)
+        assert res < 1e-8
+        iters[precision] = solver.last_iterations
+    print(iters)
+    assert iters["mixed"] <= 1.1 * iters["fp64"], iters
+
+
 @pytest.mark.parametrize("nel", [(16, 8), (8, 4, 4), (12, 6, 6)])
 @pytest.mark.parametrize("method", ["cg", "gmres"])
 def test_krylov_solvers(nel, method):
