@@ -403,6 +403,35 @@ def test_fused_2d_cycle(nel, n_level, precision):
     assert err < (1e-11 if precision == "fp64" else 2e-3)
 
 
+@pytest.mark.parametrize("w_level", [0, 1, [0, 1]])
+def test_fused_2d_cycle_beside_w_levels(w_level):
+    """2-D W-cycles: levels visited twice take one kernel per operation, the others the fused legs.
+    The iterate after five PCG iterations against the oracle's (bound as in test_fused_2d_cycle)."""
+    ET = _edgeto()
+    nel = (48, 32)
+    mesh = ET.CuStructuredMesh2D(*nel, *nel, stiffness=lambda x0: ET.auto_stiffness(x0, 1.0, 0.3))
+    kernel = ET.CuStructuredStiffnessKernel(mesh)
+    rng = np.random.default_rng(43)
+    E = rng.uniform(0.3, 1.0, mesh.n_el)
+    kernel.set_rho(torch.tensor(E, device="cuda"))
+    tp = ET.CuTopOpt(mesh, ET.SingleMaterial(void=1e-9, penalty=3.0, volume_fraction=0.3), kernel,
+                     None, ET.CuStructuredFilter2D(mesh, 1.5), verbose=False)
+    clamp, load = np.arange(nel[1] + 1) * (nel[0] + 1), (nel[0] + 1) * (nel[1] + 1) - 1
+    tp.add_BC_nodal(clamp, np.array([[1, 1]]))
+    tp.add_F_nodal(np.array([load]), np.array([[1.0, 0.0]]))
+    args = dict(tol=1e-30, maxiter=5, n_smooth=2, n_level=3, cycle="w", w_level=w_level)
+    solver = ET.CuMultiGrid(mesh, kernel, strict=False, **args)
+    x, _ = solver.solve(tp.f, use_last=False)
+    prob = otop.Problem(nel, nu=0.3, r_min=1.5)
+    prob.cons[clamp * 2] = prob.cons[clamp * 2 + 1] = True
+    prob.f[2 * load] = 1.0
+    A = oops.assemble(prob.K0, prob.elements, E, prob.cons, prob.n_dof)
+    om = OMultiGrid(nel, 2, mode="gpu", **{**args, "w_level": np.atleast_1d(w_level).tolist()})
+    xo, _ = om.solve(A, prob.f, use_last=False)
+    assert om.last_iters == solver.last_iterations == 5
+    assert np.linalg.norm(x.cpu().numpy() - xo) / np.linalg.norm(xo) < 1e-11
+
+
 def test_mixed_2d_iterations():
     """An ill-conditioned 2-D solve (moduli over two decades, more than 100 PCG iterations): the FP32
     V-cycle costs no iterations while r.z is summed with r in FP64 (with r's FP32 copy: a quarter
