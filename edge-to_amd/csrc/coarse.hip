@@ -435,6 +435,10 @@ __global__ __launch_bounds__(256) void mirror_upper_kernel(double* A, int ld, in
 static int g_coarse_lib = 2;
 void set_coarse_lib(int mode) { g_coarse_lib = mode >= 0 && mode <= 2 ? mode : 2; }
 int get_coarse_lib() { return g_coarse_lib; }
+bool coarse_supported(int64_t n) {
+  const int64_t ld = (n + NB - 1) / NB * NB;
+  return ld < INT32_MAX && (g_coarse_lib == 0 || ld * ld <= INT32_MAX);
+}
 
 __global__ void f64_to_f32_kernel(int64_t n, const double* __restrict__ a, float* __restrict__ b) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;

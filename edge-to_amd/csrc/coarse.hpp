@@ -38,5 +38,8 @@ struct CoarseSolver {
 // potrf + potri, 0 = in-house dense Cholesky and inverse.
 void set_coarse_lib(int mode);
 int get_coarse_lib();
+// Whether those solvers take n unknowns: the library routines index the n x n matrix in 32 bits, the
+// in-house one in 64.
+bool coarse_supported(int64_t n);
 
 }  // namespace et

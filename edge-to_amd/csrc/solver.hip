@@ -710,6 +710,9 @@ int MGSolver::create(const et_mg_params& p, const double* K0_host, hipStream_t s
                  "n_level too deep for this mesh (a level would have fewer than one element)");
       g = g.coarse();
     }
+    // (a 2048 x 1024 grid halved three times leaves 66 306)
+    ET_REQUIRE(coarse_supported(g.n_nodes() * dof),
+               "coarsest grid too large for its direct solve (more than 46336 unknowns): use more levels");
   }
   n_dof = g0.n_nodes() * dof;
   n_elem = g0.n_elem();

@@ -441,7 +441,7 @@ typedef struct et_mg et_mg;
 typedef struct et_mg_params {
   int dim;
   int nel[3];
-  int n_level;       /* number of coarsenings (grids = n_level + 1) */
+  int n_level;       /* number of coarsenings (grids = n_level + 1); the coarsest grid has at most 46336 DOFs */
   int n_smooth;      /* damped-Jacobi sweeps before and after the coarse correction */
   double omega;      /* reference `omega` (max omega) */
   double min_omega;  /* reference `min_omega`; min = max(omega/2, min_omega) */

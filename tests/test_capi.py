@@ -54,6 +54,23 @@ def test_mg_create_rejects_bad_params():
     assert b"n_level" in lib.et_last_error()
 
 
+@pytest.mark.parametrize("nel,n_level", [((2048, 1024), 3), ((192, 192, 192), 3)])
+def test_mg_create_rejects_a_coarsest_grid_beyond_32_bit_indices(nel, n_level):
+    """The coarsest grid's dense factor has at most 2^31 entries (the library routines index it in
+    32 bits): 66 306 and 46 875 unknowns are refused before any device work."""
+    from edgeto_amd import _lib
+    lib = _lib.load(require_gpu=False)
+    p = _lib.MGParams()
+    p.dim, p.n_level, p.n_smooth, p.precision = len(nel), n_level, 2, 0
+    for i, v in enumerate(nel):
+        p.nel[i] = v
+    K0 = np.zeros(576)
+    h = ctypes.c_void_p()
+    st = lib.et_mg_create(ctypes.byref(h), ctypes.byref(p), K0.ctypes.data_as(ctypes.POINTER(ctypes.c_double)), None)
+    assert st == _lib.ET_EINVAL and not h.value
+    assert b"coarsest grid" in lib.et_last_error()
+
+
 def test_product_filter_offsets_match_oracle():
     from edgeto_amd.geom import _offsets_weights
     from oracle import filters
