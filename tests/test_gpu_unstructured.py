@@ -356,3 +356,35 @@ def test_csr_cg_steps(n, per_row):
     st = L.lib().et_csr_cg_f64(n, L.i32(rp), L.i32(cols), L.f64(vals), L.f64(bt), L.f64(x), 1e-9, 5,
                                L.f64(work), less - 256, ctypes.byref(it), ctypes.byref(res), L.stream())
     assert st == L.ET_EINVAL
+
+
+@pytest.mark.parametrize("form", ["structured", "matrix_free", "assembled"])
+def test_cg_enqueues_little_past_the_stop(form):
+    """The host reads the state once per chunk of iterations.  A matrix-free operator's product runs
+    whether the iterations have stopped or not, so at most 7 more than the solve needs are enqueued;
+    assembled, on a system that converges at an even rate, at most 15 row passes more."""
+    import edgeto_amd as ET
+    from torch.profiler import ProfilerActivity, profile
+    if form == "structured":
+        mesh = ET.CuStructuredMesh3D(16, 8, 8, 16.0, 8.0, 8.0, stiffness=lambda x0: ET.auto_stiffness(x0, 1.0, 0.3))
+        kernel = ET.CuStructuredStiffnessKernel(mesh)
+    else:
+        mesh = ET.CuGeneralMesh(*cases.tet_mesh((6, 5, 4)), stiffness=ET.AutoStiffness(1.0, 0.3))
+        kernel = ET.CuGeneralStiffnessKernel(mesh)
+    n = kernel.shape[0]
+    kernel.add_constraints(np.arange(0, n, 5))  # every fifth DOF held: well conditioned
+    kernel.set_rho(torch.ones(mesh.n_el, dtype=torch.float64, device="cuda"))
+    f = torch.tensor(np.random.default_rng(3).standard_normal(n), device="cuda")
+    f[::5] = 0.0
+    kw = {} if form == "structured" else {"matrix_free": form == "matrix_free"}
+    for tol in (1e-1, 1e-2, 1e-4):
+        solver = ET.CuCG(kernel, maxiter=1000, tol=tol, **kw)
+        solver.solve(f, use_last=False)
+        torch.cuda.synchronize()
+        with profile(activities=[ProfilerActivity.CUDA]) as prof:
+            solver.solve(f, use_last=False)
+            torch.cuda.synchronize()
+        name = "cg_csr_kernel" if form == "assembled" else "cg_pq_kernel"
+        steps = sum(e.count for e in prof.key_averages() if name in e.key)
+        assert steps >= solver.last_iterations > 0, (tol, steps)
+        assert steps - solver.last_iterations <= (15 if form == "assembled" else 7), (tol, steps, solver.last_iterations)
