@@ -7,8 +7,8 @@
 // workgroups per compute unit busy).  Each step stages one element plane of the tile with its
 // y/z halo into one of two LDS planes and adds it to the 2R + 1 outputs of its column that it
 // reaches, which wait in registers: an LDS value is read once per thread and not once per tap.
-// At 256 x 128 x 128, radius 1, that took the forward from 51 to 25 us (67 MB, 2.7 TB/s) and the
-// transpose from 51 to 27 us (100 MB, 3.7 TB/s) against one LDS read per tap and weight; what is
+// At 256 x 128 x 128, radius 1, that took the forward from 51 to 23 us (67 MB, 2.9 TB/s) and the
+// transpose from 51 to 26 us (100 MB, 3.9 TB/s) against one LDS read per tap and weight; what is
 // left is load and barrier latency at 4 wavefronts per SIMD (128 VGPRs at radius 2).
 // 2-D: one workgroup stages one 4 x 64 tile with its halo and sums it; a small grid is bound by
 // launch and load latency (120 x 40: 9 us with the plane march, 4.4 us with one tile).
@@ -34,9 +34,10 @@
 // structure (k0_structure); any other K0 takes the full product.
 //
 // The march needs a radius of at most kMaxR per axis and a table in ascending (dx, dy, dz) order
-// with weights even in each of them (every table the meshes build up to rmin 3); the 2-D tile a
-// radius of at most kR2.  Each workgroup checks that on the device, where the table is; any
-// other table is gathered from memory tap by tap (the adjoint then recomputes the neighbour's
+// with weights even in each of them (every table the meshes build up to rmin 3); any other table
+// of that radius is summed tap by tap from a ring of LDS planes.  The 2-D tile takes any table with a
+// radius of at most kR2.  Each workgroup checks that on the device, where the table is; wider
+// tables are gathered from memory tap by tap (the adjoint then recomputes the neighbour's
 // sensitivity per tap).
 #include "common.hpp"
 #include "op_tiled.hpp"
@@ -366,8 +367,8 @@ __device__ __forceinline__ void add_plane(const double* me, const ClassWeights<R
   }
 }
 
-// Taps beyond the march (radius above kMaxR, or a table in another order or without the mirror
-// symmetry): gathers from memory, the adjoint recomputing each tap's value.
+// Taps beyond the LDS planes (radius above kMaxR): gathers from memory, the adjoint recomputing each
+// tap's value.
 template <int MODE, int DIM, int EN>
 __device__ __forceinline__ void wide_taps(const Grid& g, const SGrid& sg, int x0, int x1, int oy, int oz, int n_off,
                                           const int32_t* __restrict__ off, const TapTable& T,
@@ -392,23 +393,65 @@ __device__ __forceinline__ void wide_taps(const Grid& g, const SGrid& sg, int x0
   }
 }
 
+// Any other table of radius R <= kMaxR (another order, duplicates, uneven weights), summed in the
+// table's order: the planes an output reaches and the next one wait in a ring of kRing LDS planes, and
+// a tap is one LDS read at an offset tabulated for each position of the ring (phase: the slot of the
+// newest plane, the output's plus R).  128 x 64 x 64, 81 taps shuffled: forward 33 us, transpose 23,
+// adjoint 37, against 75, 105 and 1480 gathered from memory, and 27, 17 and 33 for the ascending table.
+constexpr int kRing = 2 * kMaxR + 2;
+
+template <int R, int PZ, int PL, int NT>
+__device__ __forceinline__ void load_phases(unsigned short (*phase)[kMaxTaps], const TapTable& T, int n_off) {
+  for (int t = threadIdx.x; t < n_off; t += NT) {
+    const int d = T.d[t];
+    const int dx = (d >> 10) - 8, dy = ((d >> 5) & 31) - 8, dz = (d & 31) - 8;
+    for (int p = 0; p < kRing; ++p) {
+      const int slot = p - R + dx;  // >= p - 2R
+      phase[p][t] = (unsigned short)((slot < 0 ? slot + kRing : slot) * PL + (dy + R) * PZ + dz + R);
+    }
+  }
+  __syncthreads();
+}
+__device__ __forceinline__ double sum_taps(const double* me, const unsigned short* off, const double* w, int n_off) {
+  double sv = 0.0;
+  int t = 0;
+#pragma unroll 1
+  for (; t + 4 <= n_off; t += 4) {
+    double wv[4], v[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      wv[k] = w[t + k];
+      v[k] = me[off[t + k]];
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) sv = fma(wv[k], v[k], sv);
+  }
+  for (; t < n_off; ++t) sv = fma(w[t], me[off[t]], sv);
+  return sv;
+}
+
 // ------------------------------------------------- 3-D forward, transpose ---
 
 // Marches planes x0 - R .. x1 - 1 + R through two LDS planes.  A plane's loads are issued PD steps
 // before it is stored, unconditionally (slots outside the grid read a clamped element and are
 // zeroed at the store), so no wait but the store's own touches them.  Returns whether all of the
-// thread's outputs are finite.
-template <int MODE, int R, int TY>
-__device__ __forceinline__ bool march(const SGrid& sg, int x0, int x1, int y0, int z0, const TapTable& T,
-                                      double* planes, const double* __restrict__ x,
-                                      const double* __restrict__ norm, double* __restrict__ y) {
+// thread's outputs are finite.  ODD: a table that add_plane does not take (always true: only the table's
+// own taps are summed).
+template <int MODE, int R, int TY, bool ODD>
+__device__ __forceinline__ bool march(const SGrid& sg, int x0, int x1, int y0, int z0, int n_off, const TapTable& T,
+                                      unsigned short (*phase)[kMaxTaps], double* planes,
+                                      const double* __restrict__ x, const double* __restrict__ norm,
+                                      double* __restrict__ y) {
   constexpr int NT = 64 * TY, PY = TY + 2 * R, PZ = 64 + 2 * R, PL = PY * PZ;
   constexpr int KP = (PL + NT - 1) / NT, PD = 4;
   const int tid = threadIdx.x, ty = tid >> 6, tz = tid & 63;
   const int oy = y0 + ty, oz = z0 + tz;
   const bool mine = oy < sg.Y && oz < sg.Z;
   ClassWeights<R> cw;
-  cw.load(T);
+  if (ODD)
+    load_phases<R, PZ, PL, NT>(phase, T, n_off);
+  else
+    cw.load(T);
   int qe[KP];  // element of the slot within a plane, -1 outside the grid
 #pragma unroll
   for (int q = 0; q < KP; ++q) {
@@ -427,8 +470,9 @@ __device__ __forceinline__ bool march(const SGrid& sg, int x0, int x1, int y0, i
       if (MODE == 2) rn[q] = norm[e];
     }
   };
+  int ph = 0;  // ODD: ring slot of plane xs
   auto put = [&](const double (&r)[KP], const double (&rn)[KP], int xs) {
-    double* pl = planes + (xs & 1) * PL;
+    double* pl = planes + (ODD ? ph : xs & 1) * PL;
     const bool xin = xs >= 0 && xs < sg.X;
 #pragma unroll
     for (int q = 0; q < KP; ++q) {
@@ -443,10 +487,10 @@ __device__ __forceinline__ bool march(const SGrid& sg, int x0, int x1, int y0, i
   const int cyz = MODE == 1 && mine ? axis_class(oy, sg.Y, R) * ncz + axis_class(oz, sg.Z, R) : 0;
   bool fine = true;
   auto step = [&](int xs) {
-    add_plane<R, PZ>(planes + (xs & 1) * PL + (ty + R) * PZ + tz + R, cw, a);
+    if (!ODD) add_plane<R, PZ>(planes + (xs & 1) * PL + (ty + R) * PZ + tz + R, cw, a);
     const int xo = xs - R;
     if (xo >= x0 && mine) {
-      double out = a[0];
+      double out = ODD ? sum_taps(planes + ty * PZ + tz, phase[ph], T.w, n_off) : a[0];
       if (MODE == 1) {
         const double sw = T.bw[axis_class(xo, sg.X, R) * (ncy * ncz) + cyz];
         out = sw > 0.0 ? out / sw : 0.0;
@@ -460,7 +504,10 @@ __device__ __forceinline__ bool march(const SGrid& sg, int x0, int x1, int y0, i
   };
   const int xe = x1 + R;  // one past the last plane
 #pragma unroll
-  for (int k = 0; k < PD; ++k) fetch(pre[k], prn[MODE == 2 ? k : 0], x0 - R + k);
+  for (int k = 0; k < PD; ++k) {
+    fetch(pre[k], prn[MODE == 2 ? k : 0], x0 - R + k);
+    asm volatile("" ::: "memory");  // in plane order: the first store waits for its own plane's loads only
+  }
   // groups of PD steps whose loads and stores have no conditions: every path issues the same ones
   for (int xb = x0 - R; xb < xe; xb += PD) {
 #pragma unroll
@@ -469,9 +516,31 @@ __device__ __forceinline__ bool march(const SGrid& sg, int x0, int x1, int y0, i
       __syncthreads();
       fetch(pre[k], prn[MODE == 2 ? k : 0], xb + k + PD);
       if (xb + k < xe) step(xb + k);
+      ph = ph + 1 < kRing ? ph + 1 : 0;
     }
   }
-  return fine;
+  return ODD || fine;
+}
+
+// bw of every boundary class: the sum of the in-grid taps in table order, as the reference's loop adds
+// them.  Visible behind the next barrier.
+template <int NT>
+__device__ __forceinline__ void class_sums(TapTable& T, const SGrid& sg, int rc, int n_off) {
+  const int tid = threadIdx.x;
+  const int nx = min(sg.X, 2 * rc + 1), ny = min(sg.Y, 2 * rc + 1), nz = min(sg.Z, 2 * rc + 1);
+  for (int c = tid; c < nx * ny * nz; c += NT) {
+    int lx, hx, ly, hy, lz, hz;
+    class_reach(c / (ny * nz), sg.X, rc, lx, hx);
+    class_reach((c / nz) % ny, sg.Y, rc, ly, hy);
+    class_reach(c % nz, sg.Z, rc, lz, hz);
+    double ws = 0.0;
+    for (int t = 0; t < n_off; ++t) {
+      const int d = T.d[t];
+      const int dx = (d >> 10) - 8, dy = ((d >> 5) & 31) - 8, dz = (d & 31) - 8;
+      ws += (dx >= -lx && dx <= hx && dy >= -ly && dy <= hy && dz >= -lz && dz <= hz) ? T.w[t] : 0.0;
+    }
+    T.bw[c] = ws;
+  }
 }
 
 // MODE 1: forward, 2: transpose (values v / N).  Tile: TY x 64 outputs per plane, one per thread.
@@ -481,33 +550,23 @@ __global__ __launch_bounds__(64 * TY) __attribute__((amdgpu_waves_per_eu(4))) vo
     const double* __restrict__ x, const double* __restrict__ norm, double* __restrict__ y) {
   constexpr int NT = 64 * TY;
   __shared__ TapTable T;
-  __shared__ double planes[2 * (TY + 2 * kMaxR) * (64 + 2 * kMaxR)];
+  __shared__ unsigned short phase[kRing][kMaxTaps];
+  __shared__ double planes[kRing * (TY + 2 * kMaxR) * (64 + 2 * kMaxR)];  // two in use but for odd tables
   const int tid = threadIdx.x;
   load_taps<3, NT>(T, n_off, off, w);
   const int rm = max(T.r[0], max(T.r[1], T.r[2])), rc = max(rm, 1);
   const int y0 = blockIdx.x * TY, z0 = blockIdx.y * 64;
   const int x0 = blockIdx.z * cx, x1 = min(x0 + cx, sg.X);
   bool fine = false;
+#define ET_MARCH(R, ODD) march<MODE, R, TY, ODD>(sg, x0, x1, y0, z0, n_off, T, phase, planes, x, norm, y)
   if (rm <= kMaxR && !T.odd) {
-    if (MODE == 1) {
-      const int nx = min(sg.X, 2 * rc + 1), ny = min(sg.Y, 2 * rc + 1), nz = min(sg.Z, 2 * rc + 1);
-      for (int c = tid; c < nx * ny * nz; c += NT) {
-        int lx, hx, ly, hy, lz, hz;
-        class_reach(c / (ny * nz), sg.X, rc, lx, hx);
-        class_reach((c / nz) % ny, sg.Y, rc, ly, hy);
-        class_reach(c % nz, sg.Z, rc, lz, hz);
-        double ws = 0.0;
-        for (int t = 0; t < n_off; ++t) {
-          const int d = T.d[t];
-          const int dx = (d >> 10) - 8, dy = ((d >> 5) & 31) - 8, dz = (d & 31) - 8;
-          ws += (dx >= -lx && dx <= hx && dy >= -ly && dy <= hy && dz >= -lz && dz <= hz) ? T.w[t] : 0.0;
-        }
-        T.bw[c] = ws;  // made visible by the march's first barrier
-      }
-    }
-    fine = rc == 1 ? march<MODE, 1, TY>(sg, x0, x1, y0, z0, T, planes, x, norm, y)
-                   : march<MODE, 2, TY>(sg, x0, x1, y0, z0, T, planes, x, norm, y);
+    if (MODE == 1) class_sums<NT>(T, sg, rc, n_off);
+    fine = rc == 1 ? ET_MARCH(1, false) : ET_MARCH(2, false);
+  } else if (rm <= kMaxR) {
+    if (MODE == 1) class_sums<NT>(T, sg, rc, n_off);
+    fine = rc == 1 ? ET_MARCH(1, true) : ET_MARCH(2, true);
   }
+#undef ET_MARCH
   const int oy = y0 + (tid >> 6), oz = z0 + (tid & 63);
   if (!fine && oy < sg.Y && oz < sg.Z) {
     AdjArgs adj{};
@@ -580,10 +639,11 @@ __device__ __forceinline__ double face_energy(const Face& lo, const Face& hi, co
 // at 128 x 64 x 64 against 24 gathered displacements and 45 couplings per value).  In the transformed basis (EN & 3 == 1) a thread
 // keeps its element column's x + 1 face for the next plane, so each node column is read once per
 // plane; any other K0 takes the full product.
-template <int EN, int R, int TY>
+template <int EN, int R, int TY, bool ODD, int NT>
 __device__ __forceinline__ bool march_adjoint(const Grid& g, const SGrid& sg, int x0, int x1, int y0, int z0,
-                                              const TapTable& T, double* planes, const AdjArgs& adj,
-                                              const double* sK, const double* sC, double* __restrict__ y) {
+                                              int n_off, const TapTable& T, unsigned short (*phase)[kMaxTaps],
+                                              double* planes, const AdjArgs& adj, const double* sK, const double* sC,
+                                              double* __restrict__ y) {
   constexpr int PY = TY + 2 * R, PZ = 64 + 2 * R, PL = PY * PZ;
   constexpr bool WHT = (EN & 3) == 1;
   const int tid = threadIdx.x, ty = tid >> 6, tz = tid & 63;
@@ -595,7 +655,10 @@ __device__ __forceinline__ bool march_adjoint(const Grid& g, const SGrid& sg, in
   const int YZ = sg.Y * sg.Z, nz = g.nz(), sy = g.nx() * nz;
   const int q = cy * sg.Z + cz, m = cy * sy + cz;  // this slot's element in plane 0 and its first node
   ClassWeights<R> cw;
-  cw.load(T);
+  if (ODD)
+    load_phases<R, PZ, PL, NT>(phase, T, n_off);
+  else
+    cw.load(T);
   Face lo, hi;
   double xv = 0.0, nv = 1.0;
   // operands of plane xs: the face at xs + 1, the density and N (clamped to the grid)
@@ -614,6 +677,7 @@ __device__ __forceinline__ bool march_adjoint(const Grid& g, const SGrid& sg, in
   }
   fetch(x0 - R);
   bool fine = true;
+  int ph = 0;  // ODD: ring slot of plane xs
   for (int xs = x0 - R; xs < x1 + R; ++xs) {
     const bool xin = xs >= 0 && xs < sg.X;
     double v = 0.0;
@@ -628,10 +692,14 @@ __device__ __forceinline__ bool march_adjoint(const Grid& g, const SGrid& sg, in
     }
     const double xe = fmin(fmax(xv, adj.vmin), 1.0);
     v = simp_factor<(EN & 4) != 0>(xe, adj.penal) * v / nv;
-    if (slot) planes[(xs & 1) * PL + tid] = xin && in ? v : 0.0;
+    if (slot) planes[(ODD ? ph : xs & 1) * PL + tid] = xin && in ? v : 0.0;
     fetch(xs + 1);
     __syncthreads();
-    if (mine) {
+    if (ODD) {
+      if (mine && xs - R >= x0)
+        y[(xs - R) * YZ + oy * sg.Z + oz] = sum_taps(planes + ty * PZ + tz, phase[ph], T.w, n_off);
+      ph = ph + 1 < kRing ? ph + 1 : 0;
+    } else if (mine) {
       add_plane<R, PZ, (R > 1)>(planes + (xs & 1) * PL + (ty + R) * PZ + tz + R, cw, a);
       if (xs - R >= x0) {
         y[(xs - R) * YZ + oy * sg.Z + oz] = a[0];
@@ -642,7 +710,7 @@ __device__ __forceinline__ bool march_adjoint(const Grid& g, const SGrid& sg, in
       a[2 * R] = 0.0;
     }
   }
-  return fine;
+  return ODD || fine;
 }
 
 // threads of the adjoint's workgroup: one staged slot each at the largest radius, whole wavefronts
@@ -658,7 +726,8 @@ __global__ __launch_bounds__(adjoint_threads(TY)) void adjoint_kernel(
     const AdjArgs adj, double* __restrict__ y) {
   constexpr int NT = adjoint_threads(TY);
   __shared__ TapTable T;
-  __shared__ double planes[2 * (TY + 2 * kMaxR) * (64 + 2 * kMaxR)];
+  __shared__ unsigned short phase[kRing][kMaxTaps];
+  __shared__ double planes[kRing * (TY + 2 * kMaxR) * (64 + 2 * kMaxR)];  // two in use but for odd tables
   __shared__ double sK[576];
   __shared__ double sC[kEnCoef];
   __shared__ double sG[63];
@@ -691,9 +760,12 @@ __global__ __launch_bounds__(adjoint_threads(TY)) void adjoint_kernel(
   const int y0 = blockIdx.x * TY, z0 = blockIdx.y * 64;
   const int x0 = blockIdx.z * cx, x1 = min(x0 + cx, sg.X);
   bool fine = false;
-  if (rm <= kMaxR && !T.odd)
-    fine = rm <= 1 ? march_adjoint<EN, 1, TY>(g, sg, x0, x1, y0, z0, T, planes, adj, sK, sC, y)
-                   : march_adjoint<EN, 2, TY>(g, sg, x0, x1, y0, z0, T, planes, adj, sK, sC, y);
+#define ET_MARCH(R, ODD) march_adjoint<EN, R, TY, ODD, NT>(g, sg, x0, x1, y0, z0, n_off, T, phase, planes, adj, sK, sC, y)
+  if (rm <= kMaxR && T.odd)
+    fine = rm <= 1 ? ET_MARCH(1, true) : ET_MARCH(2, true);
+  else if (rm <= kMaxR)
+    fine = rm <= 1 ? ET_MARCH(1, false) : ET_MARCH(2, false);
+#undef ET_MARCH
   const int oy = y0 + (tid >> 6), oz = z0 + (tid & 63);
   if (!fine && tid < 64 * TY && oy < sg.Y && oz < sg.Z)
     wide_taps<3, 3, EN>(g, sg, x0, x1, oy, oz, n_off, off, T, nullptr, adj, sK, sG, y);
