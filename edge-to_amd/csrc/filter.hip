@@ -10,8 +10,9 @@
 // At 256 x 128 x 128, radius 1, that took the forward from 51 to 23 us (67 MB, 2.9 TB/s) and the
 // transpose from 51 to 26 us (100 MB, 3.9 TB/s) against one LDS read per tap and weight; what is
 // left is load and barrier latency at 4 wavefronts per SIMD (128 VGPRs at radius 2).
-// 2-D: one workgroup stages one 4 x 64 tile with its halo and sums it; a small grid is bound by
-// launch and load latency (120 x 40: 9 us with the plane march, 4.4 us with one tile).
+// 2-D: one workgroup stages one tile with its halo and sums it, 4 x 64 outputs on small grids, which
+// are bound by launch and load latency (120 x 40: 9 us with a plane march, 4.4 us with one tile), and
+// 32 x 64 on large ones.
 // Every output is written once, with no atomics, and sums follow the offset table's order, so
 // results are deterministic; the forward pass is bitwise the reference's (out-of-grid taps add
 // an exact 0.0).  The forward's denominator depends only on the output's distances to the six
@@ -774,53 +775,109 @@ __global__ __launch_bounds__(adjoint_threads(TY)) void adjoint_kernel(
 // -------------------------------------------------------------------- 2-D ---
 
 constexpr int kR2 = 4;                  // halo radius of the 2-D tile (rmin <= 5)
-constexpr int kTX2 = 4, kTZ2 = 64;      // outputs per workgroup, one per thread
+constexpr int kTZ2 = 64;                // outputs of a tile along z
 
-// MODE 1: forward, 2: transpose, 3: SIMP adjoint, on one staged tile with its halo.  At most
-// 2^19 outputs in use and all of them in cache: launch and load latency bound, so one
-// workgroup does one tile and meets two barriers.
-template <int MODE, int EN>
-__global__ __launch_bounds__(256) void filter2_kernel(const Grid g, const SGrid sg, int n_off,
+// MODE 1: forward, 2: transpose, 3: SIMP adjoint, on one staged tile of TX x 64 outputs with its
+// halo, NO outputs of a column per thread (launch_filter2 says which).
+template <int MODE, int EN, int TX, int NO>
+__global__ __launch_bounds__(64 * TX / NO) void filter2_kernel(const Grid g, const SGrid sg, int n_off,
                                                       const int32_t* __restrict__ off,
                                                       const double* __restrict__ w, const double* __restrict__ x,
                                                       const AdjArgs adj, double* __restrict__ y) {
-  constexpr int PZ = kTZ2 + 2 * kR2;
+  constexpr int PZ = kTZ2 + 2 * kR2, NT = 64 * TX / NO;
   __shared__ TapTable T;
-  __shared__ double tile[(kTX2 + 2 * kR2) * PZ];
+  __shared__ double tile[(TX + 2 * kR2) * PZ];
   __shared__ double sK[MODE == 3 ? 64 : 1];
   const int tid = threadIdx.x;
   if (MODE == 3 && tid < 64) sK[tid] = adj.K0[tid];
-  load_taps<2, 256>(T, n_off, off, w);
+  load_taps<2, NT>(T, n_off, off, w);
   const int rx = T.r[0], rz = T.r[2];
-  const int x0 = blockIdx.y * kTX2, z0 = blockIdx.x * kTZ2;
-  const int ox = x0 + (tid >> 6), oz = z0 + (tid & 63);
-  const bool mine = ox < sg.X && oz < sg.Z;
+  const int ntz = (sg.Z + kTZ2 - 1) / kTZ2, bx = blockIdx.x / ntz;
+  const int x0 = bx * TX, z0 = (blockIdx.x - bx * ntz) * kTZ2;
+  const int ox = x0 + (tid >> 6) * NO, oz = z0 + (tid & 63);
   if (rx > kR2 || rz > kR2) {
-    if (mine) wide_taps<MODE, 2, EN>(g, sg, ox, ox + 1, 0, oz, n_off, off, T, x, adj, sK, nullptr, y);
+    if (oz < sg.Z)
+      wide_taps<MODE, 2, EN>(g, sg, ox, min(ox + NO, sg.X), 0, oz, n_off, off, T, x, adj, sK, nullptr, y);
     return;
   }
-  const int pz = kTZ2 + 2 * rz, pn = (kTX2 + 2 * rx) * pz;
-  for (int t = tid; t < pn; t += 256) {
-    const int lx = t / pz, lz = t - lx * pz;
-    const int gx = x0 - rx + lx, gz = z0 - rz + lz;
-    double v = 0.0;
-    if (gx >= 0 && gx < sg.X && gz >= 0 && gz < sg.Z)
-      v = stencil_value<MODE, 2, EN>(g, sg, gx, 0, gz, x, adj, sK, nullptr);
-    tile[lx * PZ + lz] = v;
+  const int pz = kTZ2 + 2 * rz, pn = (TX + 2 * rx) * pz;
+  if constexpr (MODE == 3 || TX == 4) {
+    for (int t = tid; t < pn; t += NT) {
+      const int lx = t / pz, lz = t - lx * pz;
+      const int gx = x0 - rx + lx, gz = z0 - rz + lz;
+      double v = 0.0;
+      if (gx >= 0 && gx < sg.X && gz >= 0 && gz < sg.Z)
+        v = stencil_value<MODE, 2, EN>(g, sg, gx, 0, gz, x, adj, sK, nullptr);
+      tile[lx * PZ + lz] = v;
+    }
+  } else {
+    // four slots of a thread at a time, loads unconditional (clamped to the grid): all in flight together
+    const int dl = NT / pz, dr = NT - dl * pz;  // NT slots further on
+    int lx = tid / pz, lz = tid - lx * pz;
+#pragma unroll 1
+    for (int t0 = tid; t0 < pn; t0 += NT * 4) {
+      double v[4], nv[4];
+      int at[4];
+      bool in[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int gx = x0 - rx + lx, gz = z0 - rz + lz;
+        in[k] = gx >= 0 && gx < sg.X && gz >= 0 && gz < sg.Z;
+        at[k] = t0 + NT * k < pn ? lx * PZ + lz : -1;
+        const int64_t e = (int64_t)min(max(gx, 0), sg.X - 1) * sg.Z + min(max(gz, 0), sg.Z - 1);
+        v[k] = x[e];
+        nv[k] = MODE == 2 ? adj.norm[e] : 1.0;
+        lx += dl;
+        lz += dr;
+        if (lz >= pz) {
+          lz -= pz;
+          ++lx;
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        if (MODE == 2) v[k] /= nv[k];
+        if (at[k] >= 0) tile[at[k]] = in[k] ? v[k] : 0.0;
+      }
+    }
   }
   __syncthreads();
-  if (!mine) return;
-  const double* me = tile + ((tid >> 6) + rx) * PZ + (tid & 63) + rz;
-  double sv = 0.0, sw = 0.0;
+  if (oz >= sg.Z) return;
+  const double* me = tile + ((tid >> 6) * NO + rx) * PZ + (tid & 63) + rz;
+  double sv[NO], sw[NO];
+#pragma unroll
+  for (int r = 0; r < NO; ++r) sv[r] = sw[r] = 0.0;
+  if (MODE != 1 || (x0 >= rx && x0 + TX + rx <= sg.X && z0 >= rz && z0 + kTZ2 + rz <= sg.Z)) {
+    // every tap of every output lies in the grid: one sum of weights
 #pragma unroll 4
-  for (int t = 0; t < n_off; ++t) {
-    const int d = T.d[t];
-    const int dx = (d >> 10) - 8, dz = (d & 31) - 8;
-    const double wk = T.w[t];
-    sv = fma(wk, me[dx * PZ + dz], sv);
-    if (MODE == 1) sw += ox + dx >= 0 && ox + dx < sg.X && oz + dz >= 0 && oz + dz < sg.Z ? wk : 0.0;
+    for (int t = 0; t < n_off; ++t) {
+      const int d = T.d[t];
+      const double wk = T.w[t];
+      const double* p = me + ((d >> 10) - 8) * PZ + (d & 31) - 8;
+#pragma unroll
+      for (int r = 0; r < NO; ++r) sv[r] = fma(wk, p[r * PZ], sv[r]);
+      if (MODE == 1) sw[0] += wk;
+    }
+#pragma unroll
+    for (int r = 1; r < NO; ++r) sw[r] = sw[0];
+  } else {
+#pragma unroll(TX == 4 ? 4 : 1)
+    for (int t = 0; t < n_off; ++t) {
+      const int d = T.d[t];
+      const int dx = (d >> 10) - 8, dz = (d & 31) - 8;
+      const double wk = T.w[t];
+      const bool in = oz + dz >= 0 && oz + dz < sg.Z;
+#pragma unroll
+      for (int r = 0; r < NO; ++r) {
+        sv[r] = fma(wk, me[(dx + r) * PZ + dz], sv[r]);
+        sw[r] += in && ox + r + dx >= 0 && ox + r + dx < sg.X ? wk : 0.0;
+      }
+    }
   }
-  y[(int64_t)ox * sg.Z + oz] = MODE == 1 ? (sw > 0.0 ? sv / sw : 0.0) : sv;
+#pragma unroll
+  for (int r = 0; r < NO; ++r)
+    if (ox + r < sg.X)
+      y[(int64_t)(ox + r) * sg.Z + oz] = MODE == 1 ? (sw[r] > 0.0 ? sv[r] / sw[r] : 0.0) : sv[r];
 }
 
 // ------------------------------------------------------------------- host ---
@@ -854,6 +911,31 @@ static dim3 march_grid(const SGrid& sg, int ty, int cx) {
   return dim3((sg.Y + ty - 1) / ty, (sg.Z + 63) / 64, (sg.X + cx - 1) / cx);
 }
 
+// 2-D tiles.  A small grid is bound by launch and load latency: 4 x 64 outputs, one per thread.  A large
+// one pays for the halo (2.1 staged values per output at radius 2; 1.2 with 32 x 64) and for the
+// table, which every workgroup reads and every tap decodes: 32 x 64 outputs, 4 of a column per thread.
+// The adjoint, whose energies take 168 registers and more, gains more from fewer threads: 8.
+// Strips of a few rows fill too little of a tall tile (us, 4 / 32 rows, 16 x 200 000: forward 30 / 33,
+// transpose 29 / 23, adjoint 81 / 53; 3 x 1 M: 34 / 128, 28 / 81, 79 / 125).
+// us, 4 / 32 rows (and a march of 256-wide rows), radius 1: forward 7.6 / 7.6 (10) at 1024 x 512, 12.1 /
+// 9.5 (14) at 1024 x 1024, 72 / 42 (41) at 4096 x 2048 (134 MB, 3.2 TB/s); transpose 6.5 / 6.0 (9.6), 10.4 /
+// 7.6 (14), 62 / 43 (44); adjoint 14 / 12 (23), 28 / 17 (37), 215 / 120 (237); radius 2: forward 12 / 12
+// (17), 20 / 15 (24), 125 / 73 (74).
+constexpr int64_t kTall2 = (int64_t)1 << 20;
+
+template <int MODE, int EN>
+static void launch_filter2(const Grid& g, const SGrid& sg, int n_off, const int32_t* off, const double* w,
+                           const double* x, const AdjArgs& adj, double* y, hipStream_t s) {
+  constexpr int TX = 32, NO = MODE == 3 ? 8 : 4;
+  const bool tall = (int64_t)sg.X * sg.Z >= kTall2 && sg.X >= (MODE == 3 ? 8 : 24);
+  const int tx = tall ? TX : 4;
+  const unsigned grid = (unsigned)((sg.Z + kTZ2 - 1) / kTZ2) * (unsigned)((sg.X + tx - 1) / tx);
+  if (tall)
+    filter2_kernel<MODE, EN, TX, NO><<<grid, 64 * TX / NO, 0, s>>>(g, sg, n_off, off, w, x, adj, y);
+  else
+    filter2_kernel<MODE, EN, 4, 1><<<grid, 256, 0, s>>>(g, sg, n_off, off, w, x, adj, y);
+}
+
 template <int MODE>
 static int launch_filter(const Grid& g, int n_off, const int32_t* off, const double* w, const double* norm,
                          const double* x, double* y, hipStream_t s) {
@@ -862,8 +944,7 @@ static int launch_filter(const Grid& g, int n_off, const int32_t* off, const dou
   adj.norm = norm;
   const int ty = g_stencil_ty, cx = chunk_planes(sg, ty);
   if (g.dim == 2)
-    filter2_kernel<MODE, 0><<<dim3((sg.Z + kTZ2 - 1) / kTZ2, (sg.X + kTX2 - 1) / kTX2), 256, 0, s>>>(
-        g, sg, n_off, off, w, x, adj, y);
+    launch_filter2<MODE, 0>(g, sg, n_off, off, w, x, adj, y, s);
   else if (ty == 4)
     march_kernel<MODE, 4><<<march_grid(sg, ty, cx), 256, 0, s>>>(g, sg, cx, n_off, off, w, x, norm, y);
   else
@@ -878,8 +959,7 @@ static int launch_adjoint(const Grid& g, int n_off, const int32_t* off, const do
   const SGrid sg = sgrid(g);
   const int ty = g_stencil_ty, cx = chunk_planes(sg, ty);
   if (g.dim == 2)
-    filter2_kernel<3, EN><<<dim3((sg.Z + kTZ2 - 1) / kTZ2, (sg.X + kTX2 - 1) / kTX2), 256, 0, s>>>(
-        g, sg, n_off, off, w, nullptr, adj, y);
+    launch_filter2<3, EN>(g, sg, n_off, off, w, nullptr, adj, y, s);
   else if (ty == 4)
     adjoint_kernel<EN, 4><<<march_grid(sg, ty, cx), adjoint_threads(4), 0, s>>>(g, sg, cx, n_off, off, w, adj, y);
   else

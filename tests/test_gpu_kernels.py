@@ -161,6 +161,38 @@ FILTER_CASES = [((12, 8), 1.5, (1, 1)), ((20, 7), 2.6, (1, 1)), ((300, 270), 3.0
                 ((10, 6, 4), 2.2, (1.0, 0.5, 2.0)), ((40, 9, 70), 2.0, (1, 1, 1)),
                 ((12, 10, 9), 4.5, (1, 1, 1)), ((33, 20), 5.2, (1, 1))]
 
+# 2-D grids of 2^20 elements and more take tiles of 32 rows: edges of the tiles, radius 1 to 4, and
+# beyond; a grid of fewer rows than a tile keeps the small one
+LARGE_2D = [((1100, 961), 1.5), ((2051, 515), 2.6), ((1024, 1024), 3.5), ((33, 31777), 4.5), ((65537, 17), 4.2),
+            ((1031, 1025), 5.2), ((9, 120001), 2.0)]
+
+
+@pytest.mark.parametrize("nel,rmin", LARGE_2D)
+def test_filter_large_2d(nel, rmin):
+    """Forward, transpose and SIMP adjoint on the tall 2-D tiles against the oracle; values of one sign
+    and at most 89 taps: a few ulps of the result."""
+    L = _lib()
+    offs, w = ofilt.offsets_weights(rmin, (1, 1))
+    norm = ofilt.normalizer(nel, offs, w)
+    n = int(np.prod(nel))
+    rng = np.random.default_rng(17)
+    x, y = rng.uniform(0.1, 1, n), torch.empty(n, dtype=torch.float64, device="cuda")
+    tab = (len(w), L.ptr(dev(offs.astype(np.int32))), L.ptr(dev(w)))
+    xt, nt = dev(x), dev(norm)
+    L.call("et_filter_fwd_f64", 2, L.nel_arg(nel), *tab, L.ptr(xt), L.ptr(y), L.stream())
+    assert rel(y.cpu().numpy(), ofilt.forward(x, nel, offs, w)) < 1e-14
+    L.call("et_filter_adj_f64", 2, L.nel_arg(nel), *tab, L.ptr(nt), L.ptr(xt), L.ptr(y), L.stream())
+    assert rel(y.cpu().numpy(), ofilt.transpose(x, nel, offs, w, norm)) < 1e-14
+    K0 = _problem((2, 2))["K0"]
+    u = rng.standard_normal(2 * (nel[0] + 1) * (nel[1] + 1))
+    energy = oops.process_dk(K0, omesh.elements_2d(*nel), u)
+    for penal in (3.0, 2.5):
+        mat = otop.SingleMaterial(void=1e-9, penalty=penal)
+        ref = ofilt.transpose(mat.grad(x) * energy, nel, offs, w, norm)
+        L.call("et_simp_adjoint_f64", 2, L.nel_arg(nel), L.ptr(dev(K0)), L.ptr(dev(u)), L.ptr(xt), penal, 1e-9, *tab,
+               L.ptr(nt), 0, L.ptr(y), L.stream())
+        assert rel(y.cpu().numpy(), ref) < 1e-12
+
 
 @pytest.mark.parametrize("nel,rmin,spacing", FILTER_CASES)
 def test_filter(nel, rmin, spacing):
@@ -222,6 +254,31 @@ def test_filter_tap_orders_and_tiles(nel, rmin, spacing):
     for order in ("asc", "perm"):
         assert torch.equal(outs[(4, order)][0], outs[(8, order)][0])
         assert torch.equal(outs[(4, order)][1], outs[(8, order)][1])
+
+
+def test_filter_2d_longest_axis():
+    """More x tiles than a grid's second axis takes (65 535): forward, transpose and SIMP adjoint of a
+    300 000 x 3 grid against the oracle."""
+    L = _lib()
+    nel = (300000, 3)
+    offs, w = ofilt.offsets_weights(1.5, (1, 1))
+    norm = ofilt.normalizer(nel, offs, w)
+    n = int(np.prod(nel))
+    rng = np.random.default_rng(16)
+    x, y = rng.uniform(0.1, 1, n), torch.empty(n, dtype=torch.float64, device="cuda")
+    tab = (len(w), L.ptr(dev(offs.astype(np.int32))), L.ptr(dev(w)))
+    L.call("et_filter_fwd_f64", 2, L.nel_arg(nel), *tab, L.ptr(dev(x)), L.ptr(y), L.stream())
+    assert rel(y.cpu().numpy(), ofilt.forward(x, nel, offs, w)) < 1e-12
+    L.call("et_filter_adj_f64", 2, L.nel_arg(nel), *tab, L.ptr(dev(norm)), L.ptr(dev(x)), L.ptr(y), L.stream())
+    assert rel(y.cpu().numpy(), ofilt.transpose(x, nel, offs, w, norm)) < 1e-12
+    el = omesh.elements_2d(*nel)
+    K0 = _problem((2, 2))["K0"]
+    u = rng.standard_normal(2 * (nel[0] + 1) * (nel[1] + 1))
+    mat = otop.SingleMaterial(void=1e-9, penalty=3.0)
+    ref = ofilt.transpose(mat.grad(x) * oops.process_dk(K0, el, u), nel, offs, w, norm)
+    L.call("et_simp_adjoint_f64", 2, L.nel_arg(nel), L.ptr(dev(K0)), L.ptr(dev(u)), L.ptr(dev(x)), 3.0, 1e-9, *tab,
+           L.ptr(dev(norm)), 0, L.ptr(y), L.stream())
+    assert rel(y.cpu().numpy(), ref) < 1e-12
 
 
 @pytest.mark.parametrize("rmin", [1.5, 2.5])
