@@ -16,7 +16,7 @@
 // The host picks CX and CY for the grid: the fewest element columns on the busiest compute unit.
 // It is bound by VALU issue (CX CY / ((CX - 1)(CY - 1)) times the grid's elements) and the load
 // latencies of the two ends (half of the time at 120 x 56 x 48).  FP64 y = A x, 97 x 45 x 51, any K0:
-// 26 us a call; the marching kernel takes 26 us after the read-back of K0 that its structure check
+// 24 us a call; the marching kernel takes 26 us after the read-back of K0 that its structure check
 // needs (78 us a call).
 #include <algorithm>
 
@@ -97,6 +97,32 @@ __global__ __launch_bounds__(kT3Threads) void op_tile3_kernel(const T3Table<T> G
   const uint8_t cbyte = cons != nullptr ? (uint8_t)0xff : (uint8_t)0;
   const T w = kJac ? (T)((omega != nullptr ? *omega : 1.0) * wscale) : T(0);
 
+  // FULL: whether K0 takes a rigid translation to zero but for the rounding of its entries (each
+  // row's sum per component within 32 units of rounding of the row's largest entry).  Then only
+  // differences of displacements are multiplied: the entries' rounding, times displacements that are
+  // large beside their differences, was most of the error (97 x 45 x 51 smooth FP64 field: 6.2e-16 of
+  // the result without, 3.5e-16 with; the transformed basis has no translations either).  The loads
+  // also bring K0 near before the element rounds read it through the scalar cache: 33.6 -> 24.2 us
+  // a call on new operands at that size.
+  __shared__ int s_loose[2];
+  if (FULL && wave < 2) {
+    const int q = min(tid, 71), row = q / 3, d = q - 3 * row;
+    T sum = T(0), big = T(0);
+#pragma unroll
+    for (int t = 0; t < 24; ++t) {
+      const T v = K0[row * 24 + t];
+      big = max(big, abs(v));
+      sum += t % 3 == d ? v : T(0);
+    }
+    constexpr T kRound = T(32) * (sizeof(T) == 8 ? T(2.220446049250313e-16) : T(1.1920929e-7f));
+    const bool loose = !(abs(sum) <= kRound * big);
+    if (__builtin_amdgcn_ballot_w64(loose) != 0) {
+      if (lane == 0) s_loose[wave] = 1;
+    } else if (lane == 0) {
+      s_loose[wave] = 0;
+    }
+  }
+
   // Stage, a node or element column per wavefront (lane = z, so the column's indices are scalar).
   // Loads are unconditional (clamped to the grid) and masks are applied at the store, so the loads
   // of kSC columns are in flight together.
@@ -136,6 +162,7 @@ __global__ __launch_bounds__(kT3Threads) void op_tile3_kernel(const T3Table<T> G
   }
   for (int t = tid; t < 3 * ospan; t += kT3Threads) sa[t] = T(0);
   __syncthreads();
+  const bool loose = FULL && (s_loose[0] | s_loose[1]) != 0;
 
   // nz lanes per column: the last one holds no element and only takes the results moved to node nelz
   const int lcol = lane / nz, lez = lane - lcol * nz;
@@ -161,9 +188,11 @@ __global__ __launch_bounds__(kT3Threads) void op_tile3_kernel(const T3Table<T> G
       };
       if constexpr (FULL) {
 #pragma unroll
-        for (int c = 0; c < 3; ++c)
+        for (int c = 0; c < 3; ++c) {
+          const T base = loose ? T(0) : T(0.5) * (u[c][0] + u[c][7]);  // about the element's middle
 #pragma unroll
-          for (int h = 0; h < 8; ++h) u[c][h] *= e;
+          for (int h = 0; h < 8; ++h) u[c][h] = (u[c][h] - base) * e;
+        }
         // scalar loads that the compiler may not hoist out of the column loop
         const __attribute__((address_space(4))) T* k = (const __attribute__((address_space(4))) T*)(const void*)K0;
         asm volatile("" : "+s"(k));
@@ -300,7 +329,7 @@ __global__ __launch_bounds__(kT3Threads) void op_tile3_kernel(const T3Table<T> G
   }
 }
 
-constexpr size_t kT3MaxLds = 160 * 1024;
+constexpr size_t kT3MaxLds = 160 * 1024 - 64;  // 64: the kernel's own
 
 size_t t3_lds_bytes(const Grid& g, int cx, int cy, size_t elem_bytes) {
   return elem_bytes * ((size_t)3 * g.nz() * ((cx + 1) * (cy + 1) + (cx - 1) * (cy - 1)) + (size_t)cx * cy * g.ez);

@@ -835,3 +835,29 @@ def test_op_tile3(nel, dt, k0):
         assert rel(y.cpu().numpy(), b - ax) < tol
         L.call("et_jacobi_" + s, *args, L.ptr(bt), L.ptr(dev(Dinv, dt)), 0.6, L.ptr(y), L.stream())
         assert rel(y.cpu().numpy(), p["u"] + 0.6 * Dinv * (b - ax)) < tol
+
+
+@pytest.mark.parametrize("nel", [(7, 6, 31), (12, 11, 20), (40, 3, 48)])
+@pytest.mark.parametrize("dt", [torch.float64, torch.float32])
+def test_op_tile3_translation(nel, dt):
+    """A rigid translation costs no digits: the product of v + t, t about 1e6 (FP32: 1e3) in every node
+    and v + t free of rounding, is that of v (the entries of K0, rounded, take t to t times their
+    rounding: 6e-11 and 2e-5 of the largest value without the differences).  A K0
+    whose rows do not sum to zero is multiplied as it is."""
+    L = _lib()
+    p = _problem(nel, seed=43)
+    big, bits = (2.0 ** 20, 20) if dt == torch.float64 else (2.0 ** 10, 10)
+    tol = 1e-13 if dt == torch.float64 else 5e-6
+    s = "f64" if dt == torch.float64 else "f32"
+    v = np.round(p["u"] * 2.0 ** bits) / 2.0 ** bits
+    t = np.tile(big * np.array([1.0, -0.5, 0.25]), p["n_dof"] // 3)
+    y = torch.empty(p["n_dof"], dtype=dt, device="cuda")
+    K0, E = dev(p["K0"], dt), dev(p["E"], dt)
+    L.call("et_matvec_" + s, 3, L.nel_arg(nel), L.ptr(K0), L.ptr(E), None, L.ptr(dev(v + t, dt)), L.ptr(y), L.stream())
+    assert rel(y.cpu().numpy(), oops.matvec(p["K0"], p["el"], p["E"], v, None)) < tol
+    loose = p["K0"].copy()
+    loose[4, 7] += 0.01 if dt == torch.float32 else 1e-9
+    L.call("et_matvec_" + s, 3, L.nel_arg(nel), L.ptr(dev(loose, dt)), L.ptr(E), None, L.ptr(dev(t / big, dt)),
+           L.ptr(y), L.stream())
+    ref = oops.matvec(loose - p["K0"], p["el"], p["E"], t / big, None)
+    assert np.abs(y.cpu().numpy() - ref).max() < (1e-14 if dt == torch.float64 else 2e-6)
