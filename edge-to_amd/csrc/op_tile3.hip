@@ -365,12 +365,10 @@ template <typename T, int MODE, bool FULL>
 void t3_launch(const T3Args& A, const T3Table<T>& Gk, const T* K0, const T* E, const uint8_t* cons, const T* x,
                const T* b, const T* Dinv, const double* omega, double wscale, const T* xadd, T* y, double* part,
                const T* dotv, hipStream_t s) {
-  static bool attr_set = false;
-  if (!attr_set) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&op_tile3_kernel<T, MODE, FULL>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)kT3MaxLds);
-    attr_set = true;
-  }
+  // once; the batched engine launches from several host threads
+  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&op_tile3_kernel<T, MODE, FULL>),
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)kT3MaxLds);
+  (void)attr;
   const size_t lds = std::max(t3_lds_bytes(A.g, A.cx, A.cy, sizeof(T)), (size_t)(kT3Threads / 64) * sizeof(double));
   op_tile3_kernel<T, MODE, FULL><<<t3_tiles(A), kT3Threads, lds, s>>>(Gk, A, K0, E, cons, x, b, Dinv, omega, wscale,
                                                                      xadd, y, part, dotv);
