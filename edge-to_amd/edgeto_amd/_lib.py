@@ -172,12 +172,16 @@ def call(name, *args):
 # around a 4.4 us kernel), so the current stream is taken as a raw handle, pointers are passed as
 # integers, and a valid tensor is accepted by one chain of attribute tests.  Any other tensor goes
 # through ptr(), which says what is wrong with it.
-_raw_stream = torch._C._cuda_getCurrentRawStream
-_device_index = torch._C._cuda_getDevice
+# A torch without a GPU backend lacks both functions: the package still imports, and the first call
+# says what is missing.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_device_index = getattr(torch._C, "_cuda_getDevice", None)
 
 
 def stream():
     """Handle of torch's current stream on the current device."""
+    if _raw_stream is None or _device_index is None:
+        return torch.cuda.current_stream().cuda_stream
     return _raw_stream(_device_index())
 
 

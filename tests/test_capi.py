@@ -5,6 +5,8 @@ import ctypes
 import glob
 import os
 import re
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -69,6 +71,20 @@ def test_mg_create_rejects_a_coarsest_grid_beyond_32_bit_indices(nel, n_level):
     st = lib.et_mg_create(ctypes.byref(h), ctypes.byref(p), K0.ctypes.data_as(ctypes.POINTER(ctypes.c_double)), None)
     assert st == _lib.ET_EINVAL and not h.value
     assert b"coarsest grid" in lib.et_last_error()
+
+
+def test_import_on_a_torch_without_gpu_backend():
+    """The package imports on a torch that lacks the raw-stream functions, and asking for a stream
+    raises torch's own error."""
+    code = ("import torch\n"
+            "for a in ('_cuda_getCurrentRawStream', '_cuda_getDevice'):\n"
+            "    if hasattr(torch._C, a): delattr(torch._C, a)\n"
+            "torch.cuda.current_stream = lambda *a: (_ for _ in ()).throw(RuntimeError('no GPU backend'))\n"
+            "from edgeto_amd import _lib\n"
+            "try:\n    _lib.stream()\nexcept RuntimeError as e:\n    print('raised:', e)\n")
+    out = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300,
+                         env={**os.environ, "PYTHONPATH": os.path.join(ROOT, "edge-to_amd")})
+    assert out.returncode == 0 and "raised: no GPU backend" in out.stdout, out.stderr[-2000:]
 
 
 def test_product_filter_offsets_match_oracle():
