@@ -160,22 +160,23 @@ __global__ __launch_bounds__(256) void cg_csr_kernel(int64_t n, CgState* __restr
                                                      double* __restrict__ q, double* __restrict__ part_pq) {
   constexpr int NP = 6;
   const int lane = threadIdx.x & 7;
-  // the first row's entries are on their way while the partials are summed
+  // the first row's entries are on their way while the partials are summed; entries count from the
+  // row's first (a matrix of nearly 2^31 entries leaves no room above them in an int)
   int64_t row = (int64_t)blockIdx.x * 32 + (threadIdx.x >> 3);
-  int a = 0, e = 0;
+  int a = 0, len = 0;
   double pv[NP];
   CgPair pg[NP], own{0.0, 0.0};
   auto fetch = [&]() {
     const int64_t rc = row < n ? row : n - 1;
     a = row_ptr[rc];
-    e = row < n ? row_ptr[rc + 1] : a;
+    len = row < n ? row_ptr[rc + 1] - a : 0;
     own = rp[rc];
 #pragma unroll
     for (int u = 0; u < NP; ++u) {
-      const int t = a + lane + 8 * u;
-      const bool in = t < e;
-      pv[u] = in ? vals[t] : 0.0;
-      pg[u] = in ? rp[cols[t]] : CgPair{0.0, 0.0};
+      const int t = lane + 8 * u;
+      const bool in = t < len;
+      pv[u] = in ? vals[a + t] : 0.0;
+      pg[u] = in ? rp[cols[a + t]] : CgPair{0.0, 0.0};
     }
   };
   fetch();
@@ -186,10 +187,10 @@ __global__ __launch_bounds__(256) void cg_csr_kernel(int64_t n, CgState* __restr
     double s = 0.0;
 #pragma unroll
     for (int u = 0; u < NP; ++u)
-      if (a + lane + 8 * u < e) s += pv[u] * (k == 0 ? pg[u].r : pg[u].r + beta * pg[u].p);
-    for (int t = a + lane + 8 * NP; t < e; t += 8) {
-      const CgPair v = rp[cols[t]];
-      s += vals[t] * (k == 0 ? v.r : v.r + beta * v.p);
+      if (lane + 8 * u < len) s += pv[u] * (k == 0 ? pg[u].r : pg[u].r + beta * pg[u].p);
+    for (int t = lane + 8 * NP; t < len; t += 8) {
+      const CgPair v = rp[cols[a + t]];
+      s += vals[a + t] * (k == 0 ? v.r : v.r + beta * v.p);
     }
     s += __shfl_xor(s, 4, 8);
     s += __shfl_xor(s, 2, 8);

@@ -343,8 +343,9 @@ __global__ __launch_bounds__(256) void csr_spmv_kernel(int64_t n_rows, const int
   const int q = (int)(t & 7);
   double s = 0.0;
   if (row < n_rows) {
-    const int a = row_ptr[row], e = row_ptr[row + 1];
-    for (int p = a + q; p < e; p += 8) s += vals[p] * x[cols[p]];
+    // entries count from the row's first: the last of 2^31 - 1 leave no room above them in an int
+    const int a = row_ptr[row], len = row_ptr[row + 1] - a;
+    for (int p = q; p < len; p += 8) s += vals[a + p] * x[cols[a + p]];
   }
   s += __shfl_xor(s, 4, 8);
   s += __shfl_xor(s, 2, 8);

@@ -358,6 +358,34 @@ def test_csr_cg_steps(n, per_row):
     assert st == L.ET_EINVAL
 
 
+def test_csr_entries_at_the_end_of_the_int_range():
+    """Rows whose entries are numbered up to 2^31 - 1 (row_ptr starts there, and the arrays' addresses
+    are shifted so that exactly these entries are theirs): product and CG as with row_ptr from 0."""
+    _, L = _et()
+    n = 40
+    rng = np.random.default_rng(5)
+    Q = rng.standard_normal((n, n))
+    A = Q @ Q.T + n * np.eye(n)
+    counts = np.full(n, n)
+    ptr = np.concatenate([[0], np.cumsum(counts)])
+    cols = torch.tensor(np.tile(np.arange(n), n).astype(np.int32), device="cuda")
+    vals = torch.tensor(A.reshape(-1), device="cuda")
+    first = 2 ** 31 - 1 - int(ptr[-1])
+    rp = torch.tensor((ptr + first).astype(np.int32), device="cuda")
+    assert int(rp[-1]) == 2 ** 31 - 1
+    pc, pv = cols.data_ptr() - 4 * first, vals.data_ptr() - 8 * first  # entry `first` is the arrays' first
+    b = rng.standard_normal(n)
+    bt, y = torch.tensor(b, device="cuda"), torch.empty(n, dtype=torch.float64, device="cuda")
+    L.call("et_csr_spmv_f64", n, L.i32(rp), pc, pv, L.f64(bt), L.f64(y), L.stream())
+    assert rel(y.cpu().numpy(), A @ b) < 1e-13
+    size = int(L.lib().et_krylov_work_size(n, 0))
+    work, x = torch.empty(size // 8 + 1, dtype=torch.float64, device="cuda"), torch.zeros(n, dtype=torch.float64, device="cuda")
+    it, res = ctypes.c_int(0), ctypes.c_double(0.0)
+    L.call("et_csr_cg_f64", n, L.i32(rp), pc, pv, L.f64(bt), L.f64(x), 1e-12, 200, L.f64(work), size,
+           ctypes.byref(it), ctypes.byref(res), L.stream())
+    assert rel(x.cpu().numpy(), np.linalg.solve(A, b)) < 1e-10
+
+
 @pytest.mark.parametrize("form", ["structured", "matrix_free", "assembled"])
 def test_cg_enqueues_little_past_the_stop(form):
     """The host reads the state once per chunk of iterations.  A matrix-free operator's product runs
