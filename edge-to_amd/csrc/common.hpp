@@ -98,6 +98,33 @@ __device__ __forceinline__ T rounded(T v) {
   return v;
 }
 
+// lane j takes lane j - 1's value (lane 0 takes 0)
+__device__ __forceinline__ unsigned lane_shr(unsigned v) {
+  return __builtin_amdgcn_update_dpp(0u, v, 0x138, 0xf, 0xf, false);
+}
+__device__ __forceinline__ float lane_shr(float v) {
+  return __builtin_bit_cast(float, lane_shr(__builtin_bit_cast(unsigned, v)));
+}
+__device__ __forceinline__ double lane_shr(double v) {
+  const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+  const unsigned lo = lane_shr((unsigned)u), hi = lane_shr((unsigned)(u >> 32));
+  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+
+// 8-point Walsh-Hadamard transform in place, natural order (index bits x, y, z of a corner)
+template <typename T>
+__device__ __forceinline__ void wht8(T (&v)[8]) {
+#pragma unroll
+  for (int h = 1; h < 8; h <<= 1)
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (!(i & h)) {
+        const T a = v[i], b = v[i | h];
+        v[i] = a + b;
+        v[i | h] = a - b;
+      }
+}
+
 // Wavefront (64-lane) sum via DPP-backed shuffles.
 template <typename T>
 __device__ inline T wave_sum(T v) {

@@ -133,16 +133,6 @@ struct AdjArgs {
 // corner-bit order beta = bx + 2 by + 4 bz of the H8 corners
 __device__ __forceinline__ int fcorner(int beta) { return h8_corner(beta & 1, (beta >> 1) & 1, beta >> 2); }
 
-// kept couplings of G[M][c][d] (M = 1..7), as in the transformed-basis operator
-__host__ __device__ constexpr bool fk_kept(int M, int c, int d) {
-  if (M == 0) return false;
-  if (c == d) return true;
-  if (M == 7) return false;
-  const int pair = (1 << c) | (1 << d);
-  const int bits = __builtin_popcount(M);
-  return bits == 1 ? (pair & M) != 0 : pair != M;
-}
-
 // -u_e^T K0 u_e of element (x, y, z) of a 3-D grid: transformed basis or full product
 template <bool WHT>
 __device__ __forceinline__ double elem_energy3(const Grid& g, int ex, int ey, int ez, const double* __restrict__ U,
@@ -183,7 +173,7 @@ __device__ __forceinline__ double elem_energy3(const Grid& g, int ex, int ey, in
       for (int c = 0; c < 3; ++c)
 #pragma unroll
         for (int d = 0; d < 3; ++d)
-          if (fk_kept(M, c, d)) e = fma(uh[c][M] * sG[(M - 1) * 9 + c * 3 + d], uh[d][M ^ (1 << c) ^ (1 << d)], e);
+          if (wht_nz(M, c, d)) e = fma(uh[c][M] * sG[(M - 1) * 9 + c * 3 + d], uh[d][M ^ (1 << c) ^ (1 << d)], e);
     }
   } else {
     // full product in the element's own DOF order
@@ -746,7 +736,7 @@ __global__ __launch_bounds__(adjoint_threads(TY)) void adjoint_kernel(
           const double k = sK[(3 * fcorner(bb) + c) * 24 + 3 * fcorner(bp) + d];
           sum += ((__builtin_popcount(M & bb) ^ __builtin_popcount(Mp & bp)) & 1) ? -k : k;
         }
-      sG[tid] = fk_kept(M, c, d) ? sum / 64.0 : 0.0;
+      sG[tid] = wht_nz(M, c, d) ? sum / 64.0 : 0.0;
     }
     __syncthreads();
     if (tid < kEnDiag) sC[tid] = sG[tid / 3 * 9 + tid % 3 * 4];
@@ -958,9 +948,9 @@ static int launch_adjoint(const Grid& g, int n_off, const int32_t* off, const do
                           double* y, hipStream_t s) {
   const SGrid sg = sgrid(g);
   const int ty = g_stencil_ty, cx = chunk_planes(sg, ty);
-  if (g.dim == 2)
-    launch_filter2<3, EN>(g, sg, n_off, off, w, nullptr, adj, y, s);
-  else if (ty == 4)
+  if (g.dim == 2) {
+    if constexpr ((EN & 3) == 2) launch_filter2<3, EN>(g, sg, n_off, off, w, nullptr, adj, y, s);  // no basis in 2-D
+  } else if (ty == 4)
     adjoint_kernel<EN, 4><<<march_grid(sg, ty, cx), adjoint_threads(4), 0, s>>>(g, sg, cx, n_off, off, w, adj, y);
   else
     adjoint_kernel<EN, 8><<<march_grid(sg, ty, cx), adjoint_threads(8), 0, s>>>(g, sg, cx, n_off, off, w, adj, y);

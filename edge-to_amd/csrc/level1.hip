@@ -66,20 +66,6 @@ __device__ __forceinline__ T l1_inv_tw_t(const Grid& g, int i, int j, int k) {
   return t;
 }
 
-// in-place 8-point Walsh-Hadamard transform, natural order
-template <typename T>
-__device__ __forceinline__ void l1_wht8(T (&v)[8]) {
-#pragma unroll
-  for (int bit = 1; bit < 8; bit <<= 1)
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-      if (!(i & bit)) {
-        const T a = v[i], b = v[i | bit];
-        v[i] = a + b;
-        v[i | bit] = a - b;
-      }
-}
-
 // ------------------------------------------------------------ setup ----
 
 template <typename T>
@@ -97,7 +83,7 @@ __global__ void l1_eh_kernel(const Grid g0, const Grid g1, const double* __restr
     v[t] = E[e];
     sp |= eflag[e];
   }
-  l1_wht8(v);
+  wht8(v);
 #pragma unroll
   for (int m = 0; m < 8; ++m) Eh[(int64_t)C * 8 + m] = (T)v[m];
   special[C] = sp ? 1 : 0;
@@ -141,17 +127,6 @@ __global__ void l1_rows_kernel(const Grid g1, const double* __restrict__ S1, con
 }
 
 // ------------------------------------------------------------ apply ----
-
-// lane j takes lane j-1's value (lane 0 takes 0)
-__device__ __forceinline__ float l1_shr(float v) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0u, __builtin_bit_cast(unsigned, v), 0x138, 0xf, 0xf, false));
-}
-__device__ __forceinline__ double l1_shr(double v) {
-  const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
-  const unsigned lo = __builtin_amdgcn_update_dpp(0u, (unsigned)u, 0x138, 0xf, 0xf, false);
-  const unsigned hi = __builtin_amdgcn_update_dpp(0u, (unsigned)(u >> 32), 0x138, 0xf, 0xf, false);
-  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
-}
 
 constexpr int kL1FixNodes = 2;  // corrected nodes per 32 lanes
 // FP32 grids below this take one output component per wavefront: 12.4 against 13.5 us at 44 225 nodes,
@@ -293,15 +268,15 @@ __global__ __launch_bounds__(SPLIT ? 768 : 1024) void l1_tile_kernel(
       for (int c = 0; c < 3; ++c)
         xh[c][beta] = uc[(((beta & 1) + ((beta >> 1) & 1) * (CX + 1)) * zs + (beta >> 2)) * 3 + c];
 #pragma unroll
-    for (int c = 0; c < 3; ++c) l1_wht8(xh[c]);
+    for (int c = 0; c < 3; ++c) wht8(xh[c]);
     // node sums at the bottom face corners f = bx + 2 by, and the unmoved top results
     constexpr int NC = SPLIT ? 1 : 3;
     T sum[4][NC], top[4][NC];
     auto faces = [&](T (&v)[8], int s) {
-      l1_wht8(v);
+      wht8(v);
 #pragma unroll
       for (int f = 0; f < 4; ++f) {
-        const T moved = l1_shr(v[f + 4]);
+        const T moved = lane_shr(v[f + 4]);
         sum[f][s] = v[f] + (lez > 0 ? moved : T(0));
         top[f][s] = v[f + 4];
       }

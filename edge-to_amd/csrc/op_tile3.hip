@@ -42,30 +42,6 @@ struct T3Table {
   T g[48];
 };
 
-__device__ __forceinline__ unsigned t3_shr32(unsigned v) { return __builtin_amdgcn_update_dpp(0u, v, 0x138, 0xf, 0xf, false); }
-__device__ __forceinline__ float t3_shr(float v) {
-  return __builtin_bit_cast(float, t3_shr32(__builtin_bit_cast(unsigned, v)));
-}
-__device__ __forceinline__ double t3_shr(double v) {
-  const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
-  const unsigned lo = t3_shr32((unsigned)u), hi = t3_shr32((unsigned)(u >> 32));
-  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
-}
-
-// 8-point Walsh-Hadamard transform in place, index bits x, y, z
-template <typename T>
-__device__ __forceinline__ void t3_wht(T (&a)[8]) {
-#pragma unroll
-  for (int h = 1; h < 8; h <<= 1)
-#pragma unroll
-    for (int b = 0; b < 8; ++b)
-      if (!(b & h)) {
-        const T p = a[b], q = a[b | h];
-        a[b] = p + q;
-        a[b | h] = p - q;
-      }
-}
-
 // MODE as in op_tiled.hpp.  FULL: K0 (24 x 24, row-major) in place of the table.
 template <typename T, int MODE, bool FULL>
 __global__ __launch_bounds__(kT3Threads) void op_tile3_kernel(const T3Table<T> Gk, const T3Args A,
@@ -183,7 +159,7 @@ __global__ __launch_bounds__(kT3Threads) void op_tile3_kernel(const T3Table<T> G
       T sum[4][3];
       // component c of the results at face corner f (lo: hz = 0, up: hz = 1)
       auto add = [&](int f, int c, T lo, T up) {
-        const T moved = t3_shr(up);
+        const T moved = lane_shr(up);
         sum[f][c] = (lez < ez_n ? lo : T(0)) + (lez > 0 ? moved : T(0));
       };
       if constexpr (FULL) {
@@ -214,7 +190,7 @@ __global__ __launch_bounds__(kT3Threads) void op_tile3_kernel(const T3Table<T> G
       } else {
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
-          t3_wht(u[c]);
+          wht8(u[c]);
 #pragma unroll
           for (int h = 0; h < 8; ++h) u[c][h] *= e;
         }
@@ -234,7 +210,7 @@ __global__ __launch_bounds__(kT3Threads) void op_tile3_kernel(const T3Table<T> G
               if (wht_nz(M, c, d)) s = fma(gq[gi++], u[d][M ^ (1 << c) ^ (1 << d)], s);
             yc[M] = s;
           }
-          t3_wht(yc);
+          wht8(yc);
 #pragma unroll
           for (int f = 0; f < 4; ++f) add(f, c, yc[f], yc[f + 4]);
         }
@@ -401,24 +377,33 @@ int op_tile3(int mode, const Grid& g, const T* K0, const WhtTable* tab, const T*
              double* part, hipStream_t s) {
   const T3Args A = t3_args(g, sizeof(T));
   ET_REQUIRE(A.cx > 0 && g.nz() <= 64, "tile operator: grid not supported");
+#define ET_T3(M, FULL)                                                                                            \
+  case M:                                                                                                         \
+    t3_launch<T, M, FULL>(A, Gk, K0, E, cons, x, b, Dinv, omega, wscale, xadd, y, part, dotv, s);                 \
+    break;
   T3Table<T> Gk{};
-  if (tab != nullptr)
+  if (tab == nullptr) {
+    // single calls
+    switch (mode) {
+      ET_T3(TM_Y, true)
+      ET_T3(TM_RES, true)
+      ET_T3(TM_JAC, true)
+      default: ET_REQUIRE(false, "tile operator: this mode takes the transformed basis");
+    }
+  } else if constexpr (sizeof(T) == 8) {
     for (int i = 0; i < 48; ++i) Gk.g[i] = (T)tab->g[i];
-#define ET_T3(M)                                                                                                  \
-  do {                                                                                                            \
-    if (tab != nullptr)                                                                                           \
-      t3_launch<T, M, false>(A, Gk, K0, E, cons, x, b, Dinv, omega, wscale, xadd, y, part, dotv, s);              \
-    else                                                                                                          \
-      t3_launch<T, M, true>(A, Gk, K0, E, cons, x, b, Dinv, omega, wscale, xadd, y, part, dotv, s);               \
-  } while (0)
-  switch (mode) {
-    case TM_Y: ET_T3(TM_Y); break;
-    case TM_RES: ET_T3(TM_RES); break;
-    case TM_JAC: ET_T3(TM_JAC); break;
-    case TM_YDOT: ET_T3(TM_YDOT); break;
-    case TM_JAC0: ET_T3(TM_JAC0); break;
-    case TM_JAC_ADD_DOT: ET_T3(TM_JAC_ADD_DOT); break;
-    default: ET_T3(TM_JAC_ADD); break;
+    switch (mode) {
+      ET_T3(TM_Y, false)
+      ET_T3(TM_RES, false)
+      ET_T3(TM_JAC, false)
+      ET_T3(TM_JAC_ADD, false)
+      ET_T3(TM_YDOT, false)
+      ET_T3(TM_JAC0, false)
+      ET_T3(TM_JAC_ADD_DOT, false)
+      default: ET_REQUIRE(false, "tile operator: unknown mode");
+    }
+  } else {
+    ET_REQUIRE(false, "tile operator: the transformed basis runs in FP64");  // see tile3_faster
   }
 #undef ET_T3
   ET_CHECK_LAUNCH();

@@ -114,17 +114,6 @@ void wht_table(const double* K0, WhtTable* t) {
   }
 }
 
-// lane j takes lane j-1 of the wavefront, lane 0 takes 0
-__device__ inline unsigned wht_shr32(unsigned v) { return __builtin_amdgcn_update_dpp(0u, v, 0x138, 0xf, 0xf, false); }
-__device__ inline float wht_shr(float v) {
-  return __builtin_bit_cast(float, wht_shr32(__builtin_bit_cast(unsigned, v)));
-}
-__device__ inline double wht_shr(double v) {
-  const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
-  const unsigned lo = wht_shr32((unsigned)u), hi = wht_shr32((unsigned)(u >> 32));
-  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
-}
-
 // 4-point transform over (hx, hz): F[px + 2 pz] = sum (-1)^(px hx + pz hz) u[hx][hz]
 template <typename T>
 __device__ inline void wht_face(const T u00, const T u10, const T u01, const T u11, T* F) {
@@ -427,7 +416,7 @@ void op0_wht_kernel(const WhtK<T> Gk, const MxArgs A,
 #pragma unroll
           for (int hx = 0; hx < 2; ++hx) {
             const T up = o[hx + 2];
-            const T zv = o[hx] + wht_shr(up);
+            const T zv = o[hx] + lane_shr(up);
             if (out && k <= nelz) sw[((c * 2 + hx) * tc + cl) * nz + k] = zv;
             if (out && lane == 63) ss[((c * 2 + hx) * tc + cl) * 2 + (ez >> 6)] = up;
           }

@@ -26,8 +26,8 @@ namespace et {
 
 // ------------------------------------------------------------ kernels ----
 
-// OP_JAC0: first Jacobi sweep from the zero guess fused with it (fine grid,
-// transformed-basis operator only); x is not read
+// OP_JAC0: first Jacobi sweep from the zero guess fused with it (fine grid: the
+// transformed-basis operators, and any K0 in 2-D); x is not read
 enum OpMode { OP_Y = 0, OP_RES = 1, OP_JAC = 2, OP_JAC_ADD = 3, OP_JAC0 = 5 };
 
 template <typename T, int DIM, int MODE>
@@ -51,7 +51,7 @@ __device__ __forceinline__ void op_epilogue(int64_t n, const T (&ax)[DIM],
 }
 
 // Level-0 operator, matrix free: 3-D grids with a general K0.  omega is read from device memory.
-template <typename T, int DIM, int MODE>
+template <typename T, int MODE>
 __global__ __launch_bounds__(256) void op0_kernel(const Grid g, const T* __restrict__ K0,
                                                   const T* __restrict__ E,
                                                   const uint8_t* __restrict__ cons,
@@ -60,52 +60,38 @@ __global__ __launch_bounds__(256) void op0_kernel(const Grid g, const T* __restr
                                                   const double* __restrict__ omega, double wscale,
                                                   const T* __restrict__ xadd,
                                                   T* __restrict__ y) {
-  constexpr int NE = DIM == 3 ? 8 : 4;
-  constexpr int ND = NE * DIM;
   const int64_t n = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (n >= g.n_nodes()) return;
   const int nz = g.nz(), nx = g.nx();
-  const int k = DIM == 3 ? (int)(n % nz) : 0;
-  const int64_t t = DIM == 3 ? n / nz : n;
+  const int k = (int)(n % nz);
+  const int64_t t = n / nz;
   const int i = (int)(t % nx), j = (int)(t / nx);
-  T acc[DIM];
+  T acc[3] = {T(0), T(0), T(0)};
 #pragma unroll
-  for (int r = 0; r < DIM; ++r) acc[r] = T(0);
+  for (int a = 0; a < 8; ++a) {
+    const int ex = i - hx(a), ey = j - hy(a), ez = k - hz(a);
+    if (!(ex >= 0 && ex < g.ex && ey >= 0 && ey < g.ey && ez >= 0 && ez < g.ez)) continue;
+    const T Ee = E[((int64_t)ex * g.ey + ey) * g.ez + ez];
+    T s[3] = {T(0), T(0), T(0)};
 #pragma unroll
-  for (int a = 0; a < NE; ++a) {
-    const int ex = i - (DIM == 3 ? hx(a) : qx(a));
-    const int ey = j - (DIM == 3 ? hy(a) : qy(a));
-    const int ez = k - (DIM == 3 ? hz(a) : 0);
-    bool valid = ex >= 0 && ex < g.ex && ey >= 0 && ey < g.ey;
-    if (DIM == 3) valid = valid && ez >= 0 && ez < g.ez;
-    if (!valid) continue;
-    const int64_t e = DIM == 3 ? ((int64_t)ex * g.ey + ey) * g.ez + ez : (int64_t)ex * g.ey + ey;
-    const T Ee = E[e];
-    T s[DIM];
+    for (int b2 = 0; b2 < 8; ++b2) {
+      const int64_t m = ((int64_t)(ey + hy(b2)) * nx + ex + hx(b2)) * nz + ez + hz(b2);
+      T um[3];
 #pragma unroll
-    for (int r = 0; r < DIM; ++r) s[r] = T(0);
+      for (int c = 0; c < 3; ++c) um[c] = (cons != nullptr && cons[m * 3 + c]) ? T(0) : x[m * 3 + c];
 #pragma unroll
-    for (int b2 = 0; b2 < NE; ++b2) {
-      const int bx = ex + (DIM == 3 ? hx(b2) : qx(b2));
-      const int by = ey + (DIM == 3 ? hy(b2) : qy(b2));
-      const int bz = ez + (DIM == 3 ? hz(b2) : 0);
-      const int64_t m = DIM == 3 ? ((int64_t)by * nx + bx) * nz + bz : (int64_t)by * nx + bx;
-      T um[DIM];
+      for (int r = 0; r < 3; ++r)
 #pragma unroll
-      for (int c = 0; c < DIM; ++c) um[c] = (cons != nullptr && cons[m * DIM + c]) ? T(0) : x[m * DIM + c];
-#pragma unroll
-      for (int r = 0; r < DIM; ++r)
-#pragma unroll
-        for (int c = 0; c < DIM; ++c) s[r] += K0[(DIM * a + r) * ND + DIM * b2 + c] * um[c];
+        for (int c = 0; c < 3; ++c) s[r] += K0[(3 * a + r) * 24 + 3 * b2 + c] * um[c];
     }
 #pragma unroll
-    for (int r = 0; r < DIM; ++r) acc[r] += Ee * s[r];
+    for (int r = 0; r < 3; ++r) acc[r] += Ee * s[r];
   }
 #pragma unroll
-  for (int r = 0; r < DIM; ++r)
-    if (cons != nullptr && cons[n * DIM + r]) acc[r] = x[n * DIM + r];
+  for (int r = 0; r < 3; ++r)
+    if (cons != nullptr && cons[n * 3 + r]) acc[r] = x[n * 3 + r];
   const T w = MODE >= OP_JAC ? (T)((omega != nullptr ? *omega : 1.0) * wscale) : T(0);
-  op_epilogue<T, DIM, MODE>(n, acc, x, b, Dinv, w, xadd, y);
+  op_epilogue<T, 3, MODE>(n, acc, x, b, Dinv, w, xadd, y);
 }
 
 // Coarse level operator: symmetric block stencil stored by halves.  S holds
@@ -440,9 +426,9 @@ static int op_launch(const MGLevel<T>& L, const MGShared& sh, int mode, const T*
     return st;
   }
   const unsigned grid = grid_for(g.n_nodes());
-#define ET_OP0(DIM, MODE)                                                                   \
-  op0_kernel<T, DIM, MODE><<<grid, kBlock, 0, s>>>(g, sh.K0<T>(), sh.E<T>(), sh.cons, x, b, \
-                                                   L.Dinv, omega, wscale, xadd, y)
+#define ET_OP0(MODE)                                                                                     \
+  op0_kernel<T, MODE><<<grid, kBlock, 0, s>>>(g, sh.K0<T>(), sh.E<T>(), sh.cons, x, b, L.Dinv, omega, wscale, \
+                                              xadd, y)
 #define ET_OPS(DIM, MODE)                                                                            \
   do {                                                                                               \
     if (g.n_nodes() <= g_row_stencil_max_nodes && g.n_nodes() * 126 * (int64_t)sizeof(T) < ((int64_t)1 << 32)) \
@@ -454,7 +440,7 @@ static int op_launch(const MGLevel<T>& L, const MGShared& sh, int mode, const T*
 #define ET_DISPATCH(M)                \
   do {                                \
     if (L.level == 0) {               \
-      ET_OP0(3, M);                   \
+      ET_OP0(M);                      \
     } else {                          \
       if (g.dim == 3)                 \
         ET_OPS(3, M);                 \
@@ -633,7 +619,7 @@ int level0_op(int mode, const Grid& g, const T* K0, const T* E, const uint8_t* c
     return op2d<T>(mode, g, K0, E, cons, x, b, Dinv, omega, wscale, xadd, y, nullptr, nullptr, s);
   const unsigned grid = grid_for(g.n_nodes());
 #define ET_L0(MODE) \
-  op0_kernel<T, 3, MODE><<<grid, kBlock, 0, s>>>(g, K0, E, cons, x, b, Dinv, omega, wscale, xadd, y)
+  op0_kernel<T, MODE><<<grid, kBlock, 0, s>>>(g, K0, E, cons, x, b, Dinv, omega, wscale, xadd, y)
   switch (mode) {
     case OP_Y: ET_L0(OP_Y); break;
     case OP_RES: ET_L0(OP_RES); break;
@@ -901,9 +887,9 @@ int MGSolver::apply_A64(const double* x, double* y, int mode, const double* b) {
     return st;
   }
   if (mode == OP_Y)
-    op0_kernel<double, 3, OP_Y><<<grid, kBlock, 0, s>>>(g0, sh.K0d, sh.Ed, sh.cons, x, b, nullptr, sh.scal, 1.0, nullptr, y);
+    op0_kernel<double, OP_Y><<<grid, kBlock, 0, s>>>(g0, sh.K0d, sh.Ed, sh.cons, x, b, nullptr, sh.scal, 1.0, nullptr, y);
   else
-    op0_kernel<double, 3, OP_RES><<<grid, kBlock, 0, s>>>(g0, sh.K0d, sh.Ed, sh.cons, x, b, nullptr, sh.scal, 1.0, nullptr, y);
+    op0_kernel<double, OP_RES><<<grid, kBlock, 0, s>>>(g0, sh.K0d, sh.Ed, sh.cons, x, b, nullptr, sh.scal, 1.0, nullptr, y);
   prof.end(s);
   ET_CHECK_LAUNCH();
   return ET_OK;

@@ -48,53 +48,8 @@ __global__ void gen_elements_3d(int nelx, int nely, int nelz, int32_t* __restric
 
 // ---------------------------------------------------------------- matvec ---
 
-// Accumulate (M K(E) M u) at node (i, j[, k]) into out[0..dim).  cons may be null.
-template <typename T, int DIM>
-__device__ __forceinline__ void node_Ku(const Grid g, int i, int j, int k, const T* __restrict__ K0,
-                                        const T* __restrict__ E, const uint8_t* __restrict__ cons,
-                                        const T* __restrict__ u, T (&out)[DIM]) {
-  constexpr int NE = DIM == 3 ? 8 : 4;
-  constexpr int ND = NE * DIM;
-  const int nx = g.nx(), nz = g.nz();
-#pragma unroll
-  for (int r = 0; r < DIM; ++r) out[r] = T(0);
-#pragma unroll
-  for (int a = 0; a < NE; ++a) {
-    const int ox = DIM == 3 ? hx(a) : qx(a);
-    const int oy = DIM == 3 ? hy(a) : qy(a);
-    const int oz = DIM == 3 ? hz(a) : 0;
-    const int ex = i - ox, ey = j - oy, ez = k - oz;
-    bool valid = ex >= 0 && ex < g.ex && ey >= 0 && ey < g.ey;
-    if (DIM == 3) valid = valid && ez >= 0 && ez < g.ez;
-    if (!valid) continue;
-    const int64_t e = DIM == 3 ? ((int64_t)ex * g.ey + ey) * g.ez + ez : (int64_t)ex * g.ey + ey;
-    const T Ee = E[e];
-    T s[DIM];
-#pragma unroll
-    for (int r = 0; r < DIM; ++r) s[r] = T(0);
-#pragma unroll
-    for (int b = 0; b < NE; ++b) {
-      const int bx = ex + (DIM == 3 ? hx(b) : qx(b));
-      const int by = ey + (DIM == 3 ? hy(b) : qy(b));
-      const int bz = ez + (DIM == 3 ? hz(b) : 0);
-      const int64_t m = DIM == 3 ? ((int64_t)by * nx + bx) * nz + bz : (int64_t)by * nx + bx;
-      T um[DIM];
-#pragma unroll
-      for (int c = 0; c < DIM; ++c) {
-        um[c] = u[m * DIM + c];
-        if (cons != nullptr && cons[m * DIM + c]) um[c] = T(0);
-      }
-#pragma unroll
-      for (int r = 0; r < DIM; ++r)
-#pragma unroll
-        for (int c = 0; c < DIM; ++c) s[r] += K0[(DIM * a + r) * ND + DIM * b + c] * um[c];
-    }
-#pragma unroll
-    for (int r = 0; r < DIM; ++r) out[r] += Ee * s[r];
-  }
-}
-
-template <typename T, int DIM>
+// 3-D grids that no fine operator takes: y = (M K(E) M + I_c) u at one node per thread.  cons may be null.
+template <typename T>
 __global__ __launch_bounds__(256) void matvec_kernel(const Grid g, const T* __restrict__ K0,
                                                      const T* __restrict__ E,
                                                      const uint8_t* __restrict__ cons,
@@ -102,14 +57,36 @@ __global__ __launch_bounds__(256) void matvec_kernel(const Grid g, const T* __re
   const int64_t n = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (n >= g.n_nodes()) return;
   const int nz = g.nz(), nx = g.nx();
-  const int k = DIM == 3 ? (int)(n % nz) : 0;
-  const int64_t t = DIM == 3 ? n / nz : n;
+  const int k = (int)(n % nz);
+  const int64_t t = n / nz;
   const int i = (int)(t % nx), j = (int)(t / nx);
-  T acc[DIM];
-  node_Ku<T, DIM>(g, i, j, k, K0, E, cons, u, acc);
+  T acc[3] = {T(0), T(0), T(0)};
 #pragma unroll
-  for (int r = 0; r < DIM; ++r) {
-    const int64_t d = n * DIM + r;
+  for (int a = 0; a < 8; ++a) {
+    const int ex = i - hx(a), ey = j - hy(a), ez = k - hz(a);
+    if (!(ex >= 0 && ex < g.ex && ey >= 0 && ey < g.ey && ez >= 0 && ez < g.ez)) continue;
+    const T Ee = E[((int64_t)ex * g.ey + ey) * g.ez + ez];
+    T s[3] = {T(0), T(0), T(0)};
+#pragma unroll
+    for (int b = 0; b < 8; ++b) {
+      const int64_t m = ((int64_t)(ey + hy(b)) * nx + ex + hx(b)) * nz + ez + hz(b);
+      T um[3];
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        um[c] = u[m * 3 + c];
+        if (cons != nullptr && cons[m * 3 + c]) um[c] = T(0);
+      }
+#pragma unroll
+      for (int r = 0; r < 3; ++r)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) s[r] += K0[(3 * a + r) * 24 + 3 * b + c] * um[c];
+    }
+#pragma unroll
+    for (int r = 0; r < 3; ++r) acc[r] += Ee * s[r];
+  }
+#pragma unroll
+  for (int r = 0; r < 3; ++r) {
+    const int64_t d = n * 3 + r;
     y[d] = (cons != nullptr && cons[d]) ? u[d] : acc[r];
   }
 }
@@ -117,16 +94,14 @@ __global__ __launch_bounds__(256) void matvec_kernel(const Grid g, const T* __re
 template <typename T>
 int matvec(const Grid& g, const T* K0, const T* E, const uint8_t* cons, const T* u, T* y,
            hipStream_t s, const WhtTable* fine) {
-  const unsigned grid = grid_for(g.n_nodes());
   if (fine == nullptr ? tile3_active(g, sizeof(T)) : tile3_faster(g, sizeof(T)))
     return op_tile3<T>(TM_Y, g, K0, fine, E, cons, u, nullptr, nullptr, nullptr, 1.0, nullptr, y, nullptr, nullptr, s);
   if (g.dim == 3 && fine != nullptr && fine_supported(g, sizeof(T)))
     return op0_fine<T>(0, g, (int64_t)g.ey * g.ez, g.ez, K0, *fine, E, cons, u, nullptr, nullptr, nullptr,
                         1.0, nullptr, y, s);
-  if (g.dim == 3)
-    matvec_kernel<T, 3><<<grid, kBlock, 0, s>>>(g, K0, E, cons, u, y);
-  else
+  if (g.dim == 2)
     return op2d<T>(TM_Y, g, K0, E, cons, u, nullptr, nullptr, nullptr, 1.0, nullptr, y, nullptr, nullptr, s);
+  matvec_kernel<T><<<grid_for(g.n_nodes()), kBlock, 0, s>>>(g, K0, E, cons, u, y);
   ET_CHECK_LAUNCH();
   return ET_OK;
 }
