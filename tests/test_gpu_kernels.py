@@ -568,11 +568,12 @@ WHT_MESHES = MX_MESHES + [(7, 4, 64), (5, 3, 65), (30, 4, 100), (4, 2, 1)]
 
 # fine-operator variants by knob values
 # (ET_TUNE_WHT, ET_TUNE_MX_F32, ET_TUNE_MX_F64, ET_TUNE_WHT_THREADS_F32, ET_TUNE_WHT_THREADS_F64,
-#  ET_TUNE_WHT_SLICES_F32, ET_TUNE_WHT_SLICES_F64)
-_KN = (7, 3, 4, 10, 11, 15, 16)
-_FINE = {"tiled": (0, 0, 0, 1024, 512, 16, 8), "matrix": (0, 1, 1, 1024, 512, 16, 8),
-         "wht": (1, 0, 0, 1024, 512, 16, 8), "wht_alt": (1, 0, 0, 512, 1024, 16, 16),
-         "wht_half": (1, 0, 0, 512, 256, 8, 8)}
+#  ET_TUNE_WHT_SLICES_F32, ET_TUNE_WHT_SLICES_F64, ET_TUNE_TILE3_NODES); the last is 0: a single call
+# on a small grid would take the one-shot tile operator, which knows none of these shapes
+_KN = (7, 3, 4, 10, 11, 15, 16, 18)
+_FINE = {"tiled": (0, 0, 0, 1024, 512, 16, 8, 0), "matrix": (0, 1, 1, 1024, 512, 16, 8, 0),
+         "wht": (1, 0, 0, 1024, 512, 16, 8, 0), "wht_alt": (1, 0, 0, 512, 1024, 16, 16, 0),
+         "wht_half": (1, 0, 0, 512, 256, 8, 8, 0)}
 
 
 def _matvec_variant(L, nel, prec, variant, seed):
@@ -789,7 +790,8 @@ def test_simp_adjoint_fused(nel, rmin, spacing, k0):
 
 @pytest.fixture
 def no_tile3():
-    """Single operator calls on small grids through the marching and node-gather kernels."""
+    """Single operator calls on small grids through the marching kernels (the node-gather kernels where
+    K0 has no transformed basis)."""
     L = _lib()
     old = L.lib().et_tune_get(18)
     L.call("et_tune_set", 18, 0)

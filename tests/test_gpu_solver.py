@@ -317,6 +317,46 @@ def test_pcg_maxiter_status():
     assert iters == 7 and res > 1e-10
 
 
+@pytest.mark.parametrize("nel", [(96, 48, 12), (72, 48, 16), (48, 36, 28), (36, 32, 40), (28, 28, 60)])
+def test_tile_operator_with_the_transformed_basis(nel):
+    """The one-shot tile operator as the FP64 solver uses it from 50 000 nodes, one to four element
+    columns per wavefront: the fine-grid product against the oracle (rows of 192 products), and three
+    PCG iterations against the marching operator's for one to three sweeps, with r.z summed in the
+    last sweep and apart from it (every mode of the V-cycle; other summation orders)."""
+    ET = _edgeto()
+    from edgeto_amd import _lib as L
+    rng = np.random.default_rng(61)
+    E = rng.uniform(0.05, 1.0, int(np.prod(nel)))
+    mesh, kernel, filt, clamp, load = _cantilever_3d(ET, nel)
+    kernel.set_rho(torch.tensor(E, device="cuda"))
+    tp = ET.CuTopOpt(mesh, ET.SingleMaterial(void=1e-9, penalty=3.0, volume_fraction=0.3), kernel, None, filt,
+                     verbose=False)
+    tp.add_BC_nodal(clamp, np.array([[1, 1, 1]]))
+    tp.add_F_nodal(load, np.array([[0.0, -1.0 / len(load), 0.0]]))
+    assert mesh.n_nodes >= 50000  # below, the solver keeps the marching operator
+    xs, old = {}, (L.lib().et_tune_get(18), L.lib().et_tune_get(14))
+    try:
+        for n_smooth in (1, 2, 3):
+            for rz in (1, 0):
+                for nodes in (old[0], 0):
+                    L.call("et_tune_set", 18, nodes)
+                    L.call("et_tune_set", 14, rz)
+                    solver = ET.CuMultiGrid(mesh, kernel, tol=1e-30, maxiter=3, n_smooth=n_smooth, n_level=2)
+                    xs[nodes] = solver.solve(tp.f, use_last=False)[0]
+                    if nodes and n_smooth == 2 and rz:
+                        x = torch.tensor(rng.standard_normal(kernel.shape[0]), device="cuda")
+                        y = torch.empty_like(x)
+                        L.call("et_mg_apply_level", solver._handle, 0, L.ptr(x), L.ptr(y))
+                        prob = _oracle_problem(nel, 0.3, 2.0, clamp, load, -1.0 / len(load))
+                        ref = oops.matvec(prob.K0, prob.elements, E, x.cpu().numpy(), prob.cons)
+                        assert np.abs(y.cpu().numpy() - ref).max() < 1e-13 * np.abs(ref).max()
+                err = ((xs[old[0]] - xs[0]).norm() / xs[0].norm()).item()
+                assert 0 < err < 1e-12, (n_smooth, rz, err)  # 0: the same operator twice
+    finally:
+        L.call("et_tune_set", 18, old[0])
+        L.call("et_tune_set", 14, old[1])
+
+
 # (ET_TUNE_WHT_THREADS_F32, ET_TUNE_WHT_THREADS_F64, ET_TUNE_WHT_SLICES_F32, ET_TUNE_WHT_SLICES_F64)
 _TILES = {"default": (1024, 512, 16, 8), "f32_half": (512, 512, 8, 8), "f64_full": (1024, 512, 16, 16),
           "f64_256": (1024, 256, 16, 8)}

@@ -121,10 +121,22 @@ def _mesh(ET, nel, case):
     return mesh, (lx, ly, lz)
 
 
+@pytest.fixture(params=["tile", "march_or_gather"])
+def small_grid_form(request):
+    """Single operator calls on small grids through the one-shot tile operator, and without it through
+    the marching kernels (K0 with the reflection structure) or the node-gather kernels (any other)."""
+    from edgeto_amd import _lib as L
+    old = L.lib().et_tune_get(18)
+    if request.param != "tile":
+        L.call("et_tune_set", 18, 0)
+    yield
+    L.call("et_tune_set", 18, old)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("case", list(CASES))
 @pytest.mark.parametrize("nel", [(6, 4, 5), (16, 8, 8)])
-def test_operators_general_k0(case, nel):
+def test_operators_general_k0(small_grid_form, case, nel):
     """kernel.dot, et_residual_f64/f32 and et_jacobi_f64 with the case's K0 against the oracle
     gather on the same K0 (1e-12 FP64, 1e-5 FP32), constrained face x = 0."""
     import edgeto_amd as ET
