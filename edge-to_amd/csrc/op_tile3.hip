@@ -5,7 +5,7 @@
 // The marching operator gives each of 256 persistent workgroups a range of node planes, with one
 // extra element layer per range and a serial chain of planes; below about half a million nodes a
 // range is one or two planes, so half of the work is the extra layer and the rest is latency.
-// Here a workgroup owns a tile of CX x CY element columns (all of z, at most 64 elements) once:
+// Here a workgroup owns a tile of CX x CY element columns (all of z, at most 63 elements: 64 nodes) once:
 //   stage    the nodes of (CX + 1) x (CY + 1) columns (constrained DOFs zeroed) and the tile's E in LDS;
 //   elements a lane computes one element (as many whole columns per wavefront as fit in 64 lanes),
 //            the hz = 1 results move one lane up, and the 12 node sums are added to the LDS

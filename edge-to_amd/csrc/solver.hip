@@ -971,7 +971,8 @@ int MGSolver::pcg(MGHierarchy<T>& h, const double* b, double* x, double tol, int
   pcg_update_p_kernel<T><<<n_pb, 256, 0, s>>>(n_dof, sh.scal, 0, partial, kRedBlocks, z, p_, x, 1);
   prof.end(s);
   ET_CHECK_LAUNCH();
-  // the fused q = A p, p.q path exists for the 2-D and the transformed-basis operator
+  // the fused q = A p, p.q path exists for the 2-D and the transformed-basis operator, up to the
+  // kRedBlocks sums that the buffer of partials holds; beyond, the sums are passes of their own
   const bool fused2 = g0.dim == 2 && op2d_partials(g0) <= kRedBlocks;
   const bool legs2 = h.vcycle2_level(0);
   const bool tile3 = sh.tiled && tile3_faster(g0, sizeof(double));

@@ -104,7 +104,7 @@ template <typename T>
 int op0_fine(int mode, const Grid& g, int64_t e_sx, int64_t e_sy, const T* K0, const WhtTable& tab, const T* E,
              const uint8_t* cons, const T* x, const T* b, const T* Dinv, const double* omega,
              double wscale, const T* xadd, T* y, hipStream_t s);
-// Small 3-D grids (at most 64 elements in z), every mode; tab: the transformed basis, null: any K0
+// Small 3-D grids (at most 63 elements in z, 64 nodes), every mode; tab: the transformed basis, null: any K0
 // (op_tile3.hip).  dotv and part: the modes with a dot product, which write tile3_partials sums.
 template <typename T>
 int op_tile3(int mode, const Grid& g, const T* K0, const WhtTable* tab, const T* E, const uint8_t* cons, const T* x,

@@ -82,8 +82,8 @@ const char* et_version(void);
  *   separate pass over r and z.  0 = separate reduction with r in FP64.  Read by each solve.
  * ET_TUNE_FILTER_ROWS: y rows of the 3-D filter stencils' tiles (64 elements along z each):
  *   8 (default, 512 threads) or 4 (256 threads).
- * ET_TUNE_TILE3_NODES: 3-D fine grids with at most this many nodes (and at most 64 elements
- *   in z) apply their operator on one-shot tiles instead of marching, while ET_TUNE_WHT is on;
+ * ET_TUNE_TILE3_NODES: 3-D fine grids with at most this many nodes (and at most 63 elements
+ *   in z, 64 nodes) apply their operator on one-shot tiles instead of marching, while ET_TUNE_WHT is on;
  *   0 = never. */
 enum {
   ET_TUNE_TILED_JC = 0,
