@@ -281,6 +281,42 @@ def test_filter_2d_longest_axis():
     assert rel(y.cpu().numpy(), ref) < 1e-12
 
 
+@pytest.mark.parametrize("nel", [(1, 1, 1), (5, 9, 65), (37, 17, 4)])
+@pytest.mark.parametrize("table", ["one", "single_off_centre", "one_sided", "duplicates"])
+def test_filter_odd_tables(nel, table):
+    """3-D tables that no mesh builds, within the LDS planes: one tap, one tap beside the centre, the
+    upper half of a ball, and 512 taps of 93 positions.  Weights of one sign: a few ulps per 512 taps."""
+    L = _lib()
+    rng = np.random.default_rng(18)
+    offs, w = ofilt.offsets_weights(2.9, (1, 1, 1))
+    if table == "one":
+        offs, w = np.zeros((1, 3), int), np.array([0.7])
+    elif table == "single_off_centre":
+        offs, w = np.array([[-2, 1, 2]]), np.array([0.7])
+    elif table == "one_sided":
+        offs, w = offs[offs[:, 0] >= 0], w[offs[:, 0] >= 0]
+    else:
+        i = rng.integers(0, len(w), 512)
+        offs, w = offs[i], w[i]
+    n = int(np.prod(nel))
+    x, norm = rng.uniform(0.1, 1, n), rng.uniform(1, 2, n)
+    y = torch.empty(n, dtype=torch.float64, device="cuda")
+    tab = (len(w), L.ptr(dev(np.ascontiguousarray(offs).astype(np.int32))), L.ptr(dev(np.ascontiguousarray(w))))
+    L.call("et_filter_fwd_f64", 3, L.nel_arg(nel), *tab, L.ptr(dev(x)), L.ptr(y), L.stream())
+    with np.errstate(invalid="ignore"):
+        ref = np.nan_to_num(_plain_filter(x, nel, offs, w, None))  # an output with no tap in the grid is 0
+    assert rel(y.cpu().numpy(), ref) < 1e-13
+    L.call("et_filter_adj_f64", 3, L.nel_arg(nel), *tab, L.ptr(dev(norm)), L.ptr(dev(x)), L.ptr(y), L.stream())
+    assert rel(y.cpu().numpy(), _plain_filter(x / norm, nel, offs, w, norm)) < 1e-13
+    p = _problem(nel, seed=19)
+    mat = otop.SingleMaterial(void=1e-9, penalty=3.0)
+    s = mat.grad(x) * oops.process_dk(p["K0"], p["el"], p["u"])
+    for flags in (7, 0):
+        L.call("et_simp_adjoint_f64", 3, L.nel_arg(nel), L.ptr(dev(p["K0"])), L.ptr(dev(p["u"])), L.ptr(dev(x)), 3.0,
+               1e-9, *tab, L.ptr(dev(norm)), flags, L.ptr(y), L.stream())
+        assert rel(y.cpu().numpy(), _plain_filter(s / norm, nel, offs, w, norm)) < 1e-12
+
+
 @pytest.mark.parametrize("rmin", [1.5, 2.5])
 @pytest.mark.parametrize("table", ["shuffled", "uneven"])
 def test_filter_tables_in_any_order_are_staged_once(rmin, table):
